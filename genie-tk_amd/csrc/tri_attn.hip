@@ -13,9 +13,9 @@
 //        fp32 path and the raw op:
 //          q, k  [B][Np r][H][Np j][32]     v^T [B][Np r][H][32][Np j]
 //          gate  [B][Np r][Np j][c_h]       bias [B][H][Np q][Np k]
-//        bf16 module path (channel-major, written as 32-byte runs):
-//          q, k, v^T  [B][Np r][H][32][Np j]    gate [B][Np r][c_h][Np j]
-//          bias       [B][H][Np q][Np k]
+//        bf16 module path: q, k, v^T and gate in tiles of 32 channels x 32
+//        positions, [B][Np r][H][Np/32][32][32]; bias in the flash kernel's
+//        fragment order (bias_frag_off)
 //  2. flash core: one wave = one head x 32 queries of one row; keys in tiles
 //     of 32.  S^T = K Q^T is accumulated on top of the bias tile, so lane l
 //     owns one query and 16 of its keys; the row max needs one lane^32
@@ -78,12 +78,10 @@ static TriAttnPacked<T> carve_triattn(Carve& cv, int cin, int /*ch*/, int H) {
 
 template <typename T> struct AttnWs {
   T *q, *k, *vt, *gate, *bias;
-  // (row, head) flash path (bf16 module forward with Np <= kFlashRhMaxNp),
-  // else null: the gated attention output (B x rows x Np x c_h, fragment
-  // order: see the flash kernel), and the
-  // triangle bias without its per-head constant in bf16, B x H x Np x Np in
-  // the flash kernel's fragment order (bias_frag_off; then bias is empty)
-  T* og;
+  // (row, head) flash path (bf16 module forward), else null: the triangle
+  // bias without its per-head constant in bf16, B x H x Np x Np in the flash
+  // kernel's fragment order (bias_frag_off; then bias is empty).  That path
+  // writes the gated attention output over the gate (og_tile_off).
   bf16* biasfr;
   // (row, head) flash path, else null: the key-mask bits of every attention
   // row (B x Np x Np/32 words: bit j of word t is key 32t + j, set for a
@@ -104,19 +102,13 @@ template <typename T> struct AttnWs {
 // Rows and positions are padded to a multiple of the flash kernel's query block.
 inline int64_t attn_pad(int64_t N) { return round_up(N, 128); }
 
-// Largest padded N of the (row, head) flash path: K^T and V^T of one row and
-// head (2 x 32 x Np bf16) stay in LDS.
-constexpr int64_t kFlashRhMaxNp = 1024;
-
-// Gated attention output og of the (row, head) path, in the output
-// projection's B-fragment order: tile (workspace row, query tile qt) is 8
-// chunks ks of [64 lanes][8 channels]; lane = 32 * (c >= c_h/2) + (q & 31)
-// holds channels c = (c_h/2) * (lane >= 32) + 8 ks .. +7 of query q.  The
-// projection kernel reads each chunk as 1 KiB contiguous.  Element offset of
-// (og tile = workspace row * Np/32 + qt, chunk ks, lane):
-__host__ __device__ __forceinline__ int64_t og_frag_off(int64_t tile, int ks, int lane) {
-  return ((tile * 8 + ks) * 64 + lane) * 8;
-}
+// Gated attention output og of the (row, head) path.  The wave that attends
+// (row, head, query tile) is the only reader of that 2 KiB tile of the gate,
+// so it writes its output tile there: 4 chunks of 8 channels, each [32
+// queries][8], which the output projection's B fragments read as 512-byte
+// runs (chunk ks & 3 of head 2 * (lane / 32) + ks / 4).  Element offset of
+// chunk k4, query q of a tile:
+__host__ __device__ __forceinline__ int og_tile_off(int k4, int q) { return (k4 * 32 + q) * 8; }
 
 // bf16 triangle bias of the (row, head) path, per batch element, in the
 // flash kernel's S^T fragment order: tile (query tile qt, key tile kt) of
@@ -142,8 +134,8 @@ __host__ __device__ __forceinline__ int vt_pos(int j) {
 
 // rows = 0: every row (Np); otherwise a chunk of that many rows.  ch: the
 // gate's channels (0: none, the raw op); fast: the bf16 module kernels
-// (c_in = 128, H = 4), whose (row, head) flash path at Np <= kFlashRhMaxNp
-// keeps the bias in fp32 fragment order and writes og.
+// (c_in = 128, H = 4), whose (row, head) flash path keeps the bias in bf16
+// fragment order.
 template <typename T>
 static AttnWs<T> carve_attn_ws(Carve& cv, int64_t B, int64_t Np, int H, int ch, int64_t rows = 0,
                                bool fast = true) {
@@ -155,9 +147,8 @@ static AttnWs<T> carve_attn_ws(Carve& cv, int64_t B, int64_t Np, int H, int ch, 
   w.k = cv.take<T>(qkv);
   w.vt = cv.take<T>(qkv);
   w.gate = cv.take<T>(ch > 0 ? B * w.rows * Np * ch : 0);
-  const bool rh = fast && ch > 0 && sizeof(T) == 2 && Np <= kFlashRhMaxNp;
+  const bool rh = fast && ch > 0 && sizeof(T) == 2;
   w.bias = rh ? nullptr : cv.take<T>(B * H * Np * Np);
-  w.og = rh ? cv.take<T>(B * w.rows * Np * ch) : nullptr;
   w.biasfr = rh ? cv.take<bf16>(B * H * Np * Np) : nullptr;
   w.mbits = rh ? cv.take<uint32_t>(B * Np * (Np / 32)) : nullptr;
   w.mflags = rh ? cv.take<int>(B * Np * (Np / 32)) : nullptr;
@@ -260,32 +251,27 @@ __global__ __launch_bounds__(256) void triattn_prologue_kernel(const T* __restri
 //     beside them; each wave then loops over 32-pair tiles.
 //     Lane i32 of a wave normalises pair 16*((i32>>2)&1) + 4*(i32>>3) + (i32&3)
 //     of the tile and the pairs are the MFMA A operand, so every accumulator
-//     lane holds 16 consecutive positions of one output channel.  All outputs
-//     of this path are channel-major over positions (below): each lane writes
-//     32 contiguous bytes, or, in the (row, head) path's tiles, its pieces
-//     after a register swap so that each store writes 1 KiB whole.  Workspace
-//     layouts of the bf16 path (Np = N rounded up to 128):
-//        q, k  [B][Np r][H][32 d][Np j]    v^T [B][Np r][H][32 d][Np j] (vt_pos order)
-//        gate  [B][Np r][c_h][Np j]        bias [B][H][Np q][Np k]
-//     Padding values are those of triattn_prologue_kernel.
-//     The (row, head) tiles leave as device-scope (sc1) buffer stores of
+//     lane holds 16 consecutive positions of one output channel.  q, k, v^T
+//     (positions in vt_pos order) and the gate leave as tiles of 32 channels
+//     x 32 positions, after a register swap so that each store writes 1 KiB
+//     whole.  q, k and v are zero outside the N x N pair grid.
+//     The tiles leave as device-scope (sc1) buffer stores of
 //     1 KiB runs (N = 256: 22.4 -> 20.0 us; no change at N = 512), and MODE
-//     15 unrolls its 16 projection steps so that the wait for the next
+//     3 unrolls its 16 projection steps so that the wait for the next
 //     tile's prefetched rows counts the stores behind them (73.5 -> 71.6 us
 //     at N = 512).
 // ---------------------------------------------------------------------------
-// MODE bit 0: q, k, v^T and gate; bit 1: the triangle bias; bit 2: the bias
-// in the flash kernel's fragment order without its per-head constant
-// (ws.biasfr) instead of row-major (ws.bias); bit 3: q, k, v^T and gate in
-// the tiled layout of the (row, head) flash kernel (each (row, head) block of
-// 32 channels x Np positions as Np/32 tiles [32 channels][32 positions],
-// 2 KiB contiguous) instead of channel-major rows.  The tiles cover rows r0
-// .. r0 + nrows - 1 of every batch element: [B][nrows][Np / 32].
+// MODE bit 0: q, k, v^T and gate, each (row, head) block of 32 channels x Np
+// positions as Np/32 tiles [32 channels][32 positions], 2 KiB contiguous; bit
+// 1: the triangle bias in the flash kernel's fragment order without its
+// per-head constant (ws.biasfr), and the key-mask words.  The tiles cover
+// position tiles 0 .. vtiles - 1 of rows r0 .. r0 + nrows - 1 of every batch
+// element; rows and positions of a workspace row past them are never read.
 template <int CIN, int H, int MODE>
 __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
     const bf16* __restrict__ x, const float* __restrict__ mask, TriAttnPacked<bf16> w, AttnWs<bf16> ws,
-    int N, int Np, int starting, float eps, int64_t ntiles, int r0, int nrows) {
-  static_assert((MODE & 3) != 0 && MODE <= 15, "q/k/v/gate, bias, or both");
+    int N, int Np, int starting, float eps, int64_t ntiles, int r0, int nrows, int vtiles) {
+  static_assert(MODE >= 1 && MODE <= 3, "q/k/v/gate, bias, or both");
   constexpr int CH = H * HD;
   constexpr int KCH = CIN / 16;
   constexpr int PE = (CH / 32) * KCH * 512;  // one packed c_in -> c_h projection
@@ -312,8 +298,7 @@ __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
   const int half = lane >> 5;
   const int i32 = lane & 31;
   const int prow = 16 * ((i32 >> 2) & 1) + 4 * (i32 >> 3) + (i32 & 3);
-  const int vtiles = Np / 32;
-  // Tiles [B][Np rows r][vtiles], walked without divisions.  The input rows of
+  // Tiles [B][nrows][vtiles], walked without divisions.  The input rows of
   // the next tile are loaded at the start of each tile, ahead of its stores:
   // loads complete in issue order, so waiting for rows loaded after a store
   // would wait for that store too.  A lane outside the pair grid reads pair 0
@@ -328,11 +313,12 @@ __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
   TileWalk tw;
   tw.init(tile, tstride, nrows, vtiles);  // row r0 + tw.r
   // (exists = false: a tile past the end, also read as pair 0).  With the
-  // bias (mode bit 1) on the (row, head) path, also the mask value of key
+  // bias (mode bit 1) also the mask value of key
   // position t.c * 32 + i32 of attention row r (pair (r, k) for the starting
   // node, (k, r) for the ending node; 1 outside the grid).
-  constexpr bool kMaskBits = (MODE & 2) != 0;
-  const bool mbits_on = kMaskBits && ws.mbits != nullptr;
+  // (mbits is never null here; tested at compile time only, the kernel needs
+  // two registers more than it has.)
+  const bool mbits_on = (MODE & 2) != 0 && ws.mbits != nullptr;
   auto load_rows = [&](Frag<bf16>* raw, float& mv, const TileWalk& t, bool exists) {
     const int jo = t.c * 32 + prow;
     const int tr = r0 + t.r;
@@ -399,8 +385,7 @@ __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
 #pragma unroll
         for (int m = 0; m < 16; m += 2)
           pk[m / 2] = pack_bf16x2(gate_from_u(acc[m] + bc), gate_from_u(acc[m + 1] + bc));
-        dst = ws.gate + (rowbase * CH + h * HD + i32) * (int64_t)Np + j0;
-        if constexpr ((MODE & 8) != 0) dst = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np + vt * 1024;
+        dst = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np + vt * 1024;
       } else {
         // q, k, v: zero outside the N x N pair grid; v^T in vt_pos order, which
         // swaps bits 2 and 3 of the position inside its group of 16: packed
@@ -418,11 +403,9 @@ __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
           pk[5] = w3;
         }
         bf16* base = kind == 0 ? ws.q : kind == 1 ? ws.k : ws.vt;
-        dst = base + ((rowbase * H + h) * HD + i32) * (int64_t)Np + j0;
-        if constexpr ((MODE & 8) != 0) dst = base + (rowbase * H + h) * HD * (int64_t)Np + vt * 1024;
+        dst = base + (rowbase * H + h) * HD * (int64_t)Np + vt * 1024;
       }
-      uint4* o = reinterpret_cast<uint4*>(dst);
-      if constexpr ((MODE & 8) != 0) {
+      {
         // tile (2 KiB, 16-byte piece 4c + j for channel c, positions 8j ..
         // 8j+7): after v_permlane16_swap register set s holds channels 16s ..
         // 16s+15 (lane l: channel 16s + l%16, piece j = 2*(l/32) + (l/16)%2),
@@ -440,16 +423,13 @@ __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
         const auto trs = buf_rsrc(dst, 2048);
         buf_store16_sc1(trs, (uint32_t)sl * 16, make_uint4(lo[0], lo[1], lo[2], lo[3]));
         buf_store16_sc1(trs, (uint32_t)(64 + sl) * 16, make_uint4(hi[0], hi[1], hi[2], hi[3]));
-      } else {
-        o[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-        o[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
       }
     };
-    // MODE 15 unrolls the steps (a constant trip count, 128 VGPRs): the
+    // MODE 3 unrolls the steps (a constant trip count, 128 VGPRs): the
     // compiler then counts the stores issued after the prefetched rows, so
     // the next tile's wait for them does not wait for this tile's stores.
     // The other modes would spill unrolled.
-    if constexpr (MODE == 15) {
+    if constexpr (MODE == 3) {
 #pragma unroll
       for (int step = 0; step < 4 * H; ++step) step_body(step);
     } else {
@@ -483,34 +463,21 @@ __global__ __launch_bounds__(1024) void triattn_prologue_bf16_kernel(
         load_wfrag_lds(fb, wb, 0, ks, KCH);
         mma(ab, xf[ks], fb);
       }
-      // lanes i32 >= H store nothing (out-of-range offset, no branch)
-      const float bb = bl[4 * CH + (i32 & (H - 1))];
-      if constexpr ((MODE & 4) != 0) {
-        // bf16 in the flash kernel's S^T fragment order (bias_frag_off),
-        // without the head's constant bb: a logit offset shared by every
-        // query and key of the head, which the softmax cancels.  bb carries
-        // the LayerNorm beta (folded in at packing), so what remains,
-        // LN(x) . (gamma * w), is the part that varies between pairs.
-        (void)bb;
-        const auto brs = buf_rsrc(ws.biasfr + (int64_t)b * H * Np * Np, (uint32_t)(H * Np * Np * 2));
+      // lanes i32 >= H store nothing (out-of-range offset, no branch).  bf16
+      // in the flash kernel's S^T fragment order (bias_frag_off), without the
+      // head's constant b_b: a logit offset shared by every query and key of
+      // the head, which the softmax cancels.  b_b carries the LayerNorm beta
+      // (folded in at packing), so what remains, LN(x) . (gamma * w), is the
+      // part that varies between pairs.
+      const auto brs = buf_rsrc(ws.biasfr + (int64_t)b * H * Np * Np, (uint32_t)(H * Np * Np * 2));
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          // positions j0 + 4a .. +3: key kk = 16*half + 4a + rr of key tile vt
-          const uint32_t off = i32 < H ? bias_frag_off(i32, r, vt, 16 * half + 4 * a, Np) * 2 : kBufSkip;
-          float bv[4];
+      for (int a = 0; a < 4; ++a) {
+        // positions j0 + 4a .. +3: key kk = 16*half + 4a + rr of key tile vt
+        const uint32_t off = i32 < H ? bias_frag_off(i32, r, vt, 16 * half + 4 * a, Np) * 2 : kBufSkip;
+        float bv[4];
 #pragma unroll
-          for (int rr = 0; rr < 4; ++rr) bv[rr] = 4 * a + rr < nvalid ? ab[4 * a + rr] : 0.f;
-          buf_store4(brs, off, bv[0], bv[1], bv[2], bv[3]);
-        }
-      } else {
-        uint32_t pk[8];
-#pragma unroll
-        for (int m = 0; m < 16; m += 2)
-          pk[m / 2] = pack_bf16x2(m < nvalid ? ab[m] + bb : 0.f, m + 1 < nvalid ? ab[m + 1] + bb : 0.f);
-        const auto brs = buf_rsrc(ws.bias + (int64_t)b * H * Np * Np, (uint32_t)(H * Np * Np * 2));
-        const uint32_t off = i32 < H ? (uint32_t)((((int64_t)i32 * Np + r) * Np + j0) * 2) : kBufSkip;
-        buf_store16(brs, off, make_uint4(pk[0], pk[1], pk[2], pk[3]));
-        buf_store16(brs, off + 16, make_uint4(pk[4], pk[5], pk[6], pk[7]));
+        for (int rr = 0; rr < 4; ++rr) bv[rr] = 4 * a + rr < nvalid ? ab[4 * a + rr] : 0.f;
+        buf_store4(brs, off, bv[0], bv[1], bv[2], bv[3]);
       }
     }
   };
@@ -700,22 +667,6 @@ __global__ __launch_bounds__(64 * H) void triattn_fused_kernel(const T* __restri
   }
 }
 
-// ---------------------------------------------------------------------------
-// 3c. bf16 module kernel: 1024 threads = H heads x 4 query tiles of 32, for a
-//     block of 128 queries of one row.
-//   * Key blocks of 64 keys (K rows and V^T columns of all heads, 32 KiB)
-//     stream into a 3-stage LDS ring with direct global->LDS loads
-//     (global_load_lds_dwordx4), issued two blocks ahead: no staging VGPRs,
-//     one barrier per block.  Tiles are XOR-swizzled in 16-byte chunks so the
-//     fragment reads are bank-conflict free.
-//   * The triangle bias enters on the matrix cores: S^T += I . Bias^T with a
-//     constant identity fragment, so the bias tile needs no VALU work; its
-//     16-byte bf16 fragments for the next block are fetched as soon as the
-//     current ones have been consumed.
-//   * Online softmax with lazy rescaling: the reference max only moves when a
-//     tile exceeds it by more than 8 (log2 units); exponentials stay <= 2^8
-//     and the result is exact after the final division by l.
-// ---------------------------------------------------------------------------
 // l in [2^-60, 2^64], tested on the bits: positive floats order as unsigned
 // integers; NaN, zero, negative values and infinity fall outside.  (The
 // softmax code is built without NaN semantics, so a float compare would not
@@ -734,377 +685,15 @@ __device__ __forceinline__ float lane_pair_sum(float v) {
 }
 
 
-template <int CIN, int H, int QT>
-__global__ __launch_bounds__(64 * H * QT) __attribute__((amdgpu_waves_per_eu(4))) void triattn_flash_kernel(
-    const bf16* __restrict__ x, const float* __restrict__ mask, bf16* __restrict__ out,
-    TriAttnPacked<bf16> w, AttnWs<bf16> ws, int N, int Np, int starting, int residual, int r0,
-    int nrows, float inf) {
-  constexpr int CH = H * HD;
-  constexpr int QB = 32 * QT;              // queries per block (QT query tiles per head)
-  constexpr int NW = H * QT;               // waves
-  constexpr int KB = 64;                   // keys per stage
-  constexpr int NS = QT == 4 ? 3 : 2;      // LDS ring stages
-  constexpr bool WO_LDS = QT == 4;         // W_o staged in LDS (else read from L2)
-  constexpr int OP = CH + 8;               // gated-o row pitch in LDS (elements)
-  constexpr int HEAD_BYTES = KB * HD * 2;  // K (or V^T) bytes of one head per stage: 4 KiB
-  constexpr int STAGE_BYTES = 2 * H * HEAD_BYTES;
-  constexpr int RPW = (STAGE_BYTES / 1024) / NW;  // 1 KiB copy regions per wave per stage
-  constexpr float kRescale = 8.0f;         // lazy-rescale threshold (log2 units)
-  static_assert(H == 4 && (QT == 4 || QT == 2), "4 heads; 64 or 128 queries per block");
-  static_assert(QB * OP * 2 <= NS * STAGE_BYTES, "o staging must fit in the ring");
-  __shared__ __attribute__((aligned(1024))) char ring[NS][STAGE_BYTES];
-  __shared__ __attribute__((aligned(1024))) bf16 wo_l[WO_LDS ? (CIN / 32) * (CH / 16) * 512 : 8];
-  // keys of this row, one bit per key: bit j of word t is key 32t + j
-  __shared__ unsigned kmask[MAXN / 32];  // mask != 1: takes the bias inf * (mask - 1)
-  __shared__ unsigned kfrac[MAXN / 32];  // ... with mask != 0 (bias from the value)
-  __shared__ unsigned kpad[MAXN / 32];   // key >= N: no weight
-  __shared__ int row_dirty;  // some key of the row is masked or padding
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar addressing
-  const int half = lane >> 5;
-  const int t32 = lane & 31;
-  const int h = wave / QT;
-  const int qt = wave % QT;
-  const int qblocks = (N + QB - 1) / QB;
-  // XCD-aware order: the query blocks of one row run back to back on one XCD
-  const int64_t lin = xcd_remap(blockIdx.x, gridDim.x);
-  // blocks cover rows r0 .. r0 + nrows - 1 of every batch element
-  const int qb = (int)(lin % qblocks);
-  const int r = r0 + (int)((lin / qblocks) % nrows);
-  const int b = (int)(lin / ((int64_t)qblocks * nrows));
-  const int q0 = qb * QB + qt * 32;
-  const int64_t rowbase = ws.row(b, r);  // q/k/v^T/gate row in the workspace
-
-  // mask of this row: key k is pair (r, k) (starting) or (k, r) (ending)
-  const float* mrow = mask ? mask + (int64_t)b * N * N + (starting ? (int64_t)r * N : r) : nullptr;
-  const int64_t mks = starting ? 1 : N;
-  if (tid == 0) row_dirty = 0;
-  __syncthreads();
-  {
-    bool dirty = false;
-    for (int k0 = wave * 64; k0 < Np; k0 += NW * 64) {
-      const int k = k0 + lane;
-      const bool inrow = k < N;
-      const float mval = inrow && mrow ? mrow[k * mks] : 1.f;
-      const bool masked = mval != 1.f;
-      dirty = dirty || masked || !inrow;
-      const unsigned long long mb = __ballot(masked);
-      const unsigned long long fb = __ballot(masked && mval != 0.f);
-      const unsigned long long pb = __ballot(!inrow);
-      if (lane == 0) {
-        kmask[k0 / 32] = (unsigned)mb;
-        kmask[k0 / 32 + 1] = (unsigned)(mb >> 32);
-        kfrac[k0 / 32] = (unsigned)fb;
-        kfrac[k0 / 32 + 1] = (unsigned)(fb >> 32);
-        kpad[k0 / 32] = (unsigned)pb;
-        kpad[k0 / 32 + 1] = (unsigned)(pb >> 32);
-      }
-    }
-    if (__ballot(dirty) != 0ull && lane == 0) row_dirty = 1;
-  }
-  __syncthreads();
-  // block-uniform flag, kept in a scalar register
-  const bool row_clean = __builtin_amdgcn_readfirstlane(row_dirty) == 0;
-  const float madd0 = -inf * kLog2e;  // the bias of a key with mask == 0 (log2 units)
-
-  // Async stage load.  A stage holds, for each head, the K^T and the V^T
-  // block of 64 keys ([32 d][64 keys] each, 4 KiB); each splits into two 2 KiB
-  // sub-blocks of 32 keys (sb), rows d of 64 bytes.  A stage is 32 regions of
-  // 1 KiB (64 lanes x 16 B): region r is kind r>>4 (K^T, V^T), head (r>>2)&3,
-  // sub-block (r>>1)&1, rows 16*(r&1) .. +15; lane l lands at row l/4,
-  // physical 16-byte chunk l%4.  K^T chunks are unswizzled: the transposing
-  // reads of a 16-lane group cover 4 consecutive rows x 32 bytes and the
-  // paired group the other halves, every bank once.  V^T chunk p of row d sits
-  // at physical chunk p ^ ((d>>2)&3), so the 16-byte reads of rows d, d+4,
-  // d+8, d+12 fall in distinct banks.  Wave w moves regions RPW*w ..
-  // RPW*w + RPW-1, all of one kind.
-  static_assert(2 * H * 4 == 32 && (16 % RPW) == 0, "32 regions per stage, one kind per wave");
-  const int rg0 = wave * RPW;
-  const bool k_region = rg0 < 16;  // the first half of the waves move K^T
-  const bf16* gbase = (k_region ? ws.k : ws.vt) + (rowbase * H) * (int64_t)HD * Np;
-  const uint32_t ring_lds = lds_addr(&ring[0][0]);
-  auto issue_stage = [&](int stage, int k0) {
-    // The per-lane offset is recomputed from the lane id here rather than
-    // kept across the tile loop: at the register cap it would be spilled, and
-    // a reload from scratch waits for every outstanding load.  It is the same
-    // for every region; the rest of each source address is uniform.
-    const uint32_t ln = (uint32_t)(lane + opaque_zero());
-    const uint32_t p = k_region ? (ln & 3) : ((ln & 3) ^ ((ln >> 4) & 3));
-    const uint32_t voff = ((ln >> 2) * (uint32_t)Np + 8 * p) * 2;
-#pragma unroll
-    for (int i = 0; i < RPW; ++i) {
-      const int r = rg0 + i;
-      const bf16* src = gbase + (int64_t)(((r >> 2) & 3) * HD + 16 * (r & 1)) * Np + 32 * ((r >> 1) & 1) + k0;
-      g2lds16_sv(src, voff, ring_lds + stage * STAGE_BYTES + r * 1024);
-    }
-  };
-
-  // W_o for the epilogue, fetched now so that it is not waited for at the end
-  if constexpr (WO_LDS) copy_to_lds_async(wo_l, w.w_o, (int)sizeof(wo_l));
-  // q and the gate are channel-major ([32 channels][Np positions] per row and
-  // head); this wave's [32 channels][32 queries] tile of either goes through
-  // LDS (a 2 KiB region per wave, 64-byte rows) and is read back transposed.
-  // Copy j (0, 1) moves channels 16j .. 16j+15: lane l takes channel
-  // 16j + l/4, queries 8*(l%4) .. +7.
-  const bf16* q_src = ws.q + ((rowbase * H + h) * HD) * (int64_t)Np + q0;
-  const bf16* g_src = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np + q0;
-  auto issue_cq = [&](const bf16* src, int stage) {
-    const uint32_t ln = (uint32_t)(lane + opaque_zero());
-    const uint32_t voff = ((ln >> 2) * (uint32_t)Np + (ln & 3) * 8) * 2;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      g2lds16_sv(src + (int64_t)j * 16 * Np, voff, ring_lds + stage * STAGE_BYTES + wave * 2048 + j * 1024);
-  };
-  // Channels c0 .. c0+3 of this lane's query t32 (ds_read_b64_tr_b16: lane
-  // (group G = lane/16, i = lane%16) reads channel c0 + i/4 at queries
-  // 16*(G&1) + 4*(i%4) .. +3; c0 carries the lane's half)
-  auto read_cq4 = [&](int stage, int c0) {
-    const int i = lane & 15;
-    return lds_read_tr16(ring[stage] + wave * 2048 + (c0 + (i >> 2)) * 64 +
-                         (16 * ((lane >> 4) & 1) + 4 * (i & 3)) * 2);
-  };
-  // query fragments (filled once the q tile is in LDS)
-  Frag<bf16> qf[2];
-  // K fragments come from the K^T tile with transposing reads: fetching lane
-  // (group G = lane/16, i = lane%16) reads d row (i/4) of a 4-row group at
-  // keys 16*(G&1) + 4*(i%4) .. +3 of the 32-key tile; the receiving lane
-  // (key t32, half) gets d .. d+3 of its key
-  const int trG = lane >> 4;
-  const int tr_m = (lane & 15) >> 2;
-  const int tr_q = lane & 3;
-  const int kt_lane = ((trG >> 1) * 8 + tr_m) * 64 + 32 * (trG & 1) + 8 * tr_q;
-  // V^T reads (P V): row t32, chunk half ^ ((t32>>2)&3) for c = 0; c = 1 flips
-  // bit 1 of the chunk, i.e. byte offset ^ 32
-  const int vt_lane = t32 * 64 + 16 * (half ^ ((t32 >> 2) & 3));
-  // identity fragments: row key (t32), slot half*8+e of chunk cb <-> key cb*16+half*8+e
-  Frag<bf16> idf[2];
-#pragma unroll
-  for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      idf[cb].v[e] = (bf16)(t32 == cb * 16 + half * 8 + e ? 1.0f : 0.0f);
-  const bf16* brow = ws.bias + ((int64_t)(b * H + h) * Np + q0 + t32) * Np + half * 8;
-  Frag<bf16> bfr[2];  // bias fragments of the next S tile to issue
-  auto load_bias = [&](int t) {
-    bfr[0].load(brow + t * 32);
-    bfr[1].load(brow + t * 32 + 16);
-  };
-  // S^T - m of 32-key tile t: the accumulation starts from negm = -m_use in
-  // every register, then adds I.Bias^T and K Q^T.
-  f32x16 negm = zero16();
-  auto s_tile = [&](int t) {
-    f32x16 s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(idf[0].v, bfr[0].v, negm, 0, 0, 0);
-    mma(s, idf[1], bfr[1]);
-    // sub-block t&1 of this head's K^T; row d = m*16 + (trG>>1)*8 + hh*4 +
-    // tr_m, keys 16*(trG&1) + 4*tr_q: one base plus constant offsets
-    const char* kt_base = ring[(t >> 1) % NS] + h * HEAD_BYTES + (t & 1) * 2048 + kt_lane;
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      s16x4 part[2];
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) part[hh] = lds_read_tr16(kt_base + (m * 16 + hh * 4) * 64);
-      typedef short s16x8 __attribute__((ext_vector_type(8)));
-      const s16x8 v8 = {part[0][0], part[0][1], part[0][2], part[0][3],
-                        part[1][0], part[1][1], part[1][2], part[1][3]};
-      Frag<bf16> kf;
-      kf.v = __builtin_bit_cast(bf16x8, v8);
-      mma(s, kf, qf[m]);
-    }
-    return s;
-  };
-
-  const int nkb = (N + KB - 1) / KB;
-  const int ntiles = 2 * nkb;
-  static_assert(NW * 2048 <= STAGE_BYTES && NS >= 2, "q / gate tiles fit in one ring stage");
-  issue_stage(0, 0);
-  issue_cq(q_src, 1);
-  load_bias(0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  typedef short s16x8 __attribute__((ext_vector_type(8)));
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const s16x4 lo = read_cq4(1, m * 16 + half * 8), hi = read_cq4(1, m * 16 + half * 8 + 4);
-    const s16x8 v8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    qf[m].v = __builtin_bit_cast(bf16x8, v8);
-  }
-  barrier_only();  // every wave has read its q tile: stage 1 is free
-  // stage 1, or (a single key block) the gate tile, into the free stage
-  if (nkb > 1) issue_stage(1, KB);
-  else issue_cq(g_src, 1);
-
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  const bf16x2_t ones2 = {(bf16)1.0f, (bf16)1.0f};
-  f32x16 o = zero16();
-  float m_ref = -INFINITY, l_run = 0.f;
-  float m_use = 0.f;  // the reference subtracted from the scores: m_ref, or 0 while m_ref = -inf
-  // The part of m_use subtracted inside S (negm = -m_in): m_use while
-  // |m_use| < kFar, else 0.  A reference set by masked keys only (about
-  // -inf log2 e) folded into the fp32 accumulation would round the logits of
-  // the valid keys that follow to multiples of its ulp; such a lane
-  // subtracts it on the VALU instead (a rare path: a row whose running
-  // maximum so far comes from masked keys).
-  constexpr float kFar = 4096.f;
-  float m_in = 0.f;
-  for (int t = 0; t < ntiles; ++t) {
-    const bool opens = t > 0 && (t & 1) == 0;  // tile t opens key block t/2
-    if (opens) {
-      __builtin_amdgcn_s_waitcnt(0);      // stage t/2 and the bias of tile t landed
-      __syncthreads();                    // ... for every wave; block t/2-2 fully consumed
-    }
-    f32x16 sc = s_tile(t);
-    if (t + 1 < ntiles) load_bias(t + 1);
-    // The next block's copy goes out after the bias of tile t+1: loads
-    // complete in issue order, so waiting for that bias does not wait for it.
-    if (opens && (t >> 1) + 1 < nkb) issue_stage(((t >> 1) + 1) % NS, ((t >> 1) + 1) * KB);
-    // the last block opens: the gate tile goes into the stage it leaves free
-    if (opens && (t >> 1) + 1 == nkb) issue_cq(g_src, nkb % NS);
-    const int cur = (t >> 1) % NS;
-    // padding keys of tile t take no weight, masked keys their mask bias
-    // (none at all in a clean row: no LDS read).  For a row whose keys are
-    // all masked the scores follow the reference's fp32 arithmetic: with
-    // inf = 1e9 they round to one value, and the row attends uniformly.
-    const unsigned kx = row_clean ? 0u : (kpad[t] | kmask[t]);
-    if (kx != 0u) {
-      const unsigned kp = kpad[t] >> (4 * half), km = kmask[t] >> (4 * half);
-      const unsigned kf = kfrac[t];
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          float add = ((km >> (8 * g + rr)) & 1u) ? madd0 : 0.f;
-          if (kf != 0u && ((kf >> (8 * g + 4 * half + rr)) & 1u))
-            add = (inf * (mrow[(int64_t)(32 * t + 8 * g + 4 * half + rr) * mks] - 1.f)) * kLog2e;
-          sc[4 * g + rr] = ((kp >> (8 * g + rr)) & 1u) ? -INFINITY : sc[4 * g + rr] + add;
-        }
-    }
-    // sc holds s - m_in; the reference max m_ref moves only when a score
-    // exceeds it by more than kRescale
-    float mt = fmaxf(fmaxf(sc[0], sc[1]), sc[2]);
-#pragma unroll
-    for (int e = 3; e < 15; e += 2) mt = fmaxf(fmaxf(mt, sc[e]), sc[e + 1]);
-    mt = fmaxf(mt, sc[15]);
-    mt = lane_pair_max(mt) + m_in;        // the tile max of s
-    if (__ballot(mt > m_ref + kRescale) != 0ull) {
-      const float m_new = fmaxf(m_ref, mt);
-      const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
-      l_run *= alpha;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[e] *= alpha;
-      m_ref = m_new;
-      m_use = (m_ref == -INFINITY) ? 0.f : m_ref;
-      const float m_in_new = fabsf(m_use) < kFar ? m_use : 0.f;
-      const float shift = m_in - m_use;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        sc[e] += shift;
-        negm[e] = -m_in_new;
-      }
-      m_in = m_in_new;
-    } else if (__ballot(m_in != m_use) != 0ull) {
-      // a lane whose reference stays beyond kFar: its scores are raw
-#pragma unroll
-      for (int e = 0; e < 16; ++e) sc[e] += m_in - m_use;
-    }
-    // sub-block t&1 of this head's V^T, row t32
-    const char* vt_base = ring[cur] + (H + h) * HEAD_BYTES + (t & 1) * 2048;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      Frag<bf16> pf, vf;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) pf.v[e] = (bf16)__builtin_amdgcn_exp2f(sc[8 * c + e]);
-      // row sum over the bf16 probabilities that enter P V
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const bf16x2_t pp = {pf.v[e], pf.v[e + 1]};
-        l_run = __builtin_amdgcn_fdot2_f32_bf16(pp, ones2, l_run, false);
-      }
-      // keys 16c + 8*half .. +8 of the sub-block: chunk (2c + half) ^ ((t32>>2)&3)
-      vf.load(reinterpret_cast<const bf16*>(vt_base + (c ? (vt_lane ^ 32) : vt_lane)));
-      mma(o, vf, pf);
-    }
-  }
-  const float inv = 1.0f / lane_pair_sum(l_run);
-  // Epilogue.  Every global load it needs (the W_o fragments and the
-  // residual rows of this wave's output tile, the gate) is issued here,
-  // before the first store: vmcnt counts stores too, so a load issued after
-  // a store is only waited for together with that store.
-  constexpr int NT = CIN / 32;
-  static_assert(QT * NT == H * QT, "one output tile per wave");
-  const int oq = wave / NT, nt = wave % NT;
-  Frag<bf16> wof[CH / 16];
-  if constexpr (!WO_LDS) {
-#pragma unroll
-    for (int ks = 0; ks < CH / 16; ++ks) load_wfrag<bf16>(wof[ks], w.w_o, nt, ks, CH / 16);
-  }
-  const int q_out = qb * QB + oq * 32 + t32;
-  const bool q_ok = q_out < N;
-  const int64_t pair_out =
-      ((int64_t)b * N + (starting ? r : (q_ok ? q_out : 0))) * N + (starting ? (q_ok ? q_out : 0) : r);
-  f32x4 bo[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) bo[g] = *reinterpret_cast<const f32x4*>(w.b_o + nt * 32 + 8 * g + 4 * half);
-  bf16x4 xres[4];
-  if (residual) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      xres[g] = *reinterpret_cast<const bf16x4*>(x + pair_out * CIN + nt * 32 + 8 * g + 4 * half);
-  }
-  // this lane's gate values (channel-major, like q)
-  bf16x4 gpre[4];
-  __builtin_amdgcn_s_waitcnt(0);  // this wave's gate tile has landed (wave-local region)
-#pragma unroll
-  for (int g = 0; g < 4; ++g) gpre[g] = __builtin_bit_cast(bf16x4, read_cq4(nkb % NS, 8 * g + 4 * half));
-
-  // o * gate for all heads, staged as [query][CH] over the ring
-  __syncthreads();
-  bf16* os = reinterpret_cast<bf16*>(&ring[0][0]);
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int d0 = 8 * g + 4 * half;
-    const bf16x4 gv = gpre[g];
-    store4(os + (qt * 32 + t32) * OP + h * HD + d0, o[4 * g] * inv * (float)gv[0],
-           o[4 * g + 1] * inv * (float)gv[1], o[4 * g + 2] * inv * (float)gv[2],
-           o[4 * g + 3] * inv * (float)gv[3]);
-  }
-  __syncthreads();
-  // output projection: wave -> (query tile oq, output tile nt)
-  {
-    Frag<bf16> of[CH / 16];
-#pragma unroll
-    for (int ks = 0; ks < CH / 16; ++ks) of[ks].load(os + (oq * 32 + t32) * OP + half * (CH / 2) + ks * 8);
-    f32x16 acc = zero16();
-#pragma unroll
-    for (int ks = 0; ks < CH / 16; ++ks) {
-      if constexpr (WO_LDS) load_wfrag_lds(wof[ks], wo_l, nt, ks, CH / 16);
-      mma(acc, wof[ks], of[ks]);
-    }
-    if (q_ok) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int c0 = nt * 32 + 8 * g + 4 * half;
-        float v[4];
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          v[rr] = acc[4 * g + rr] + bo[g][rr];
-          if (residual) v[rr] += (float)xres[g][rr];
-        }
-        store4(out + pair_out * CIN + c0, v[0], v[1], v[2], v[3]);
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// 3d. bf16 flash kernel, one block per (row, head), for Np <= NPM (1024).
+// 3c. bf16 flash kernel.  STREAM = false: one block per (row, head), for Np
+//     <= NPM (1024).
 //   * K^T and V^T of the row and head (2 x 32 x Np bf16, 64 KiB at Np = 512)
 //     are copied into LDS once, with direct global->LDS loads, and stay there
 //     for the whole block: after one barrier the key loop runs without any.
 //     Layout: [kind][key tile t][32 d rows][64 bytes]; K^T rows unswizzled,
-//     V^T chunk p of row d at physical chunk p ^ ((d>>2)&3) (the read
-//     patterns of the module kernel above).
+//     V^T chunk p of row d at physical chunk p ^ ((d>>2)&3), so that the
+//     16-byte reads of rows d, d+4, d+8, d+12 fall in distinct banks.
 //   * NW waves (8, or 16 at Np = 1024); wave w attends query tiles w,
 //     w+NW, ... in turn.  Each
 //     query tile: q copied into the wave's 2 KiB LDS region and read back
@@ -1112,7 +701,7 @@ __global__ __launch_bounds__(64 * H * QT) __attribute__((amdgpu_waves_per_eu(4))
 //     the key loop (bf16 bias tiles prefetched two tiles ahead and widened
 //     into the S^T accumulator, the next tile's K fragments read a tile
 //     ahead), then o / l * gate stored into og in the
-//     output projection's fragment order (og_frag_off).  The next tile's q
+//     output projection's fragment order (og_tile_off).  The next tile's q
 //     copy is issued before those stores.
 //   * The excluded-key bits of the row are kept in one VGPR (lane t: key
 //     tile t) and read with v_readlane per tile.  The prologue's bias pass
@@ -1120,6 +709,19 @@ __global__ __launch_bounds__(64 * H * QT) __attribute__((amdgpu_waves_per_eu(4))
 //     64 contiguous bytes instead of the row's mask values, which for the
 //     ending node are a column of the mask, one cache line per key, read by
 //     every wave of every head's block.
+//   * STREAM (Np > 1024, where the keys of a row and head no longer fit): a
+//     block takes up to NW query tiles of its (row, head), one a wave, and the
+//     keys pass through LDS in two alternating stages of 256: while a stage
+//     is attended each wave copies its 4 KiB of the next one, one copy in each
+//     of its first four tiles, and one barrier opens each stage.  The blocks
+//     of a row re-read its K^T / V^T from L2 (5 times at N = 1100).  Every
+//     wave of a block walks the same key tiles, so the running maximum stays
+//     out of the key loop here too: a wave that needs the exact pass makes the
+//     block stream its keys once more.  With two 80 KiB blocks a CU holds 16
+//     waves, as in the resident form.  At N = 1100
+//     the kernel takes 1.46 ms (467 TFLOP/s of Q K^T and P V); blocks of 64
+//     queries over all four heads, with a row-major bias through an identity
+//     product and a barrier per 64 keys, took 6.46 ms.
 //   * Blocks run head-major, so the blocks of one XCD read one or two heads'
 //     triangle bias.  That bias (1 MiB per head at Np = 512) is re-read by
 //     every row's block, while K^T, V^T, q and the gate are read once: their
@@ -1131,15 +733,18 @@ __global__ __launch_bounds__(64 * H * QT) __attribute__((amdgpu_waves_per_eu(4))
 // NW waves per block: 8 at Np <= 512 (two blocks per CU), 16 at Np = 1024,
 // where K^T and V^T take 128 KiB of LDS and one block fills the CU (16 x 2 KiB
 // of staging beside them: 160 KiB), so the CU still holds 16 waves.
-template <int NPM, int NW>
+template <int NPM, int NW, bool STREAM>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void triattn_flash_rh_kernel(
     const float* __restrict__ mask, AttnWs<bf16> ws, int N, int Np, int starting, int r0, int nrows,
-    float inf) {
+    float inf, int nk, int qgroups) {
   constexpr int H = 4, CH = H * HD;
   static_assert(2 * NPM / 32 * 2048 + NW * 2048 <= 160 * 1024, "K^T, V^T and staging in one CU's LDS");
-  constexpr int NTM = NPM / 32;       // key tiles at most
+  constexpr int NTM = NPM / 32;       // key tiles in LDS
+  constexpr int ST = NTM / 2;         // STREAM: key tiles per stage (two stages)
+  constexpr int CPW = 4 * ST / NW;    // STREAM: copies of 1 KiB per wave and stage
   constexpr float kRescale = 8.0f;    // lazy-rescale threshold (log2 units)
-  static_assert(NTM <= 64, "excluded-key bits: one word per lane");
+  static_assert(NTM <= 64 && 64 % ST == 0, "excluded-key bits: one word per lane");
+  static_assert(!STREAM || ((4 * ST) % NW == 0 && CPW <= ST && ST % 2 == 0), "whole copies, at most one a tile");
   __shared__ __attribute__((aligned(1024))) char kv[2 * NTM * 2048];
   __shared__ __attribute__((aligned(1024))) char stg[NW][2048];
 
@@ -1148,32 +753,52 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
   const int t32 = lane & 31;
-  const int nt = Np / 32;             // key tiles (even: Np is a multiple of 128)
+  const int nt = Np / 32;             // tiles of a workspace row
   const int nq = (N + 31) / 32;       // query tiles holding real queries
-  const int64_t per_h = (int64_t)gridDim.x / H;
-  const int64_t lin = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = (int)(lin / per_h);
-  const int64_t rem = lin - h * per_h;
-  const int b = (int)(rem / nrows);
-  const int r = r0 + (int)(rem - (int64_t)b * nrows);
+  // nk: key tiles attended, those with real keys rounded up to a pair
+  const int lin = (int)xcd_remap(blockIdx.x, gridDim.x);
+  const int per_h = (int)gridDim.x / H;
+  const int h = lin / per_h;
+  int rem = lin - h * per_h;
+  int qg = 0;                         // STREAM: the block's group of query tiles
+  if constexpr (STREAM) {
+    const int rr = rem / qgroups;
+    qg = rem - rr * qgroups;
+    rem = rr;
+  }
+  const int b = rem / nrows;
+  const int r = r0 + (rem - b * nrows);
   const int64_t rowbase = ws.row(b, r);
 
-  // K^T / V^T of (row, head): 4 * nt copies of 1 KiB (kind, tile, row half)
-  {
-    const bf16* kbase = ws.k + (rowbase * H + h) * (int64_t)HD * Np;
-    const bf16* vbase = ws.vt + (rowbase * H + h) * (int64_t)HD * Np;
-    // tiled layout: key tile t is [32 d][32 keys], 2 KiB contiguous
-    const uint32_t ln = (uint32_t)lane;
-    const uint32_t rowoff = (ln >> 2) * 64;
-    const uint32_t voff_k = rowoff + (ln & 3) * 16;
-    const uint32_t voff_v = rowoff + (((ln & 3) ^ ((ln >> 4) & 3)) * 16);
-    const uint32_t kv_lds = lds_addr(kv);
-    for (int c = wave; c < 4 * nt; c += NW) {
-      const int kind = c >= 2 * nt;
-      const int cr = c - kind * 2 * nt;
-      const int t = cr >> 1, rh = cr & 1;
-      const bf16* src = (kind ? vbase : kbase) + t * 1024 + rh * 512;
-      g2lds16_sv_nt(src, kind ? voff_v : voff_k, kv_lds + ((kind * NTM + t) * 2 + rh) * 1024);
+  // K^T / V^T of (row, head) in copies of 1 KiB (kind, key tile, row half);
+  // tiled layout: key tile t is [32 d][32 keys], 2 KiB contiguous.  Tile t
+  // lands in slot t % NTM.
+  const bf16* kbase = ws.k + (rowbase * H + h) * (int64_t)HD * Np;
+  const bf16* vbase = ws.vt + (rowbase * H + h) * (int64_t)HD * Np;
+  const uint32_t kv_lds = lds_addr(kv);
+  auto copy_piece = [&](int kind, int t, int rh) {
+    const uint32_t ln = (uint32_t)(lane + opaque_zero());
+    const uint32_t p = kind ? (ln & 3) ^ ((ln >> 4) & 3) : ln & 3;
+    const bf16* src = (kind ? vbase : kbase) + t * 1024 + rh * 512;
+    const uint32_t dst = kv_lds + ((kind * NTM + t % NTM) * 2 + rh) * 1024;
+    // read once by this row's block, or (STREAM) by its few query groups
+    if constexpr (STREAM) g2lds16_sv(src, (ln >> 2) * 64 + p * 16, dst);
+    else g2lds16_sv_nt(src, (ln >> 2) * 64 + p * 16, dst);
+  };
+  // STREAM: this wave's copy i of stage s (key tiles ST s .. ST s + ST-1)
+  auto stage_piece = [&](int s, int i) {
+    const int c = wave * CPW + i;
+    const int kind = c / (2 * ST), t = s * ST + (c % (2 * ST)) / 2;
+    if (t < nk) copy_piece(kind, t, c & 1);
+  };
+  if constexpr (STREAM) {
+#pragma unroll
+    for (int i = 0; i < CPW; ++i) stage_piece(0, i);
+  } else {
+    for (int c = wave; c < 4 * nk; c += NW) {
+      const int kind = c >= 2 * nk;
+      const int cr = c - kind * 2 * nk;
+      copy_piece(kind, cr >> 1, cr & 1);
     }
   }
 
@@ -1189,9 +814,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // the same row.
   const float* mrow = mask ? mask + (int64_t)b * N * N + (starting ? (int64_t)r * N : r) : nullptr;
   const int64_t mks = starting ? 1 : N;
-  const int64_t mwi = ((int64_t)b * Np + r) * (Np / 32) + lane;
-  const uint32_t kmv = lane < nt ? ws.mbits[mwi] : 0u;
-  const int mfl = lane < nt ? ws.mflags[mwi] : 0;
+  const int64_t mwi = ((int64_t)b * Np + r) * (Np / 32);
+  // words of key tiles t0 .. t0+63, one a lane (STREAM: reloaded every 64 tiles)
+  auto mask_words = [&](int t0) { return t0 + lane < nk ? ws.mbits[mwi + t0 + lane] : 0u; };
+  uint32_t kmv = mask_words(0);
+  int mfl = lane < nk ? ws.mflags[mwi + lane] : 0;
+  if constexpr (STREAM)
+    for (int t = 64 + lane; t < nk; t += 64) mfl |= ws.mflags[mwi + t];
   const bool row_valid = __ballot((mfl & 1) != 0) != 0ull;
   const bool row_frac = __ballot((mfl & 2) != 0) != 0ull;
   const float madd0 = -inf * kLog2e;  // the bias of a key with mask == 0
@@ -1215,7 +844,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     return lds_read_tr16(sw + (c0 + (i >> 2)) * 64 + (16 * ((ln >> 4) & 1) + 4 * (i & 3)) * 2);
   };
   const bf16* q_row = ws.q + ((rowbase * H + h) * HD) * (int64_t)Np;
-  const bf16* g_row = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np;
+  bf16* g_row = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np;
   const bf16* b_head = ws.biasfr + (int64_t)(b * H + h) * Np * Np;  // wave-uniform
 
   // K fragments (transposing reads of K^T) and V^T fragments: per-lane offsets
@@ -1251,7 +880,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   };
   // K fragments of key tile t (transposing reads of K^T)
   auto k_read = [&](int t, Frag<bf16>* kf) {
-    const char* kt_base = kv + t * 2048 + kt_lane;
+    const char* kt_base = kv + (t % NTM) * 2048 + kt_lane;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       const s16x4 p0 = lds_read_tr16(kt_base + (m * 16) * 64);
@@ -1275,7 +904,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // exact pass runs rows with such values)
   auto mask_tile = [&](int t, f32x16& sc, auto frac_tag) {
     constexpr bool FRAC = decltype(frac_tag)::value;
-    const unsigned km_t = __builtin_amdgcn_readlane(kmv, t);
+    const unsigned km_t = __builtin_amdgcn_readlane(kmv, t & 63);
     const int nin = N - 32 * t;  // keys of tile t below N
     if (km_t != 0u || nin < 32) {
       // this lane's keys j = 8g + 4*half + rr: bits 8g + rr after the shift
@@ -1301,7 +930,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const bool fast_ok = row_valid && !row_frac;
   // P = 2^sc (bf16), l += row sums of P, O^T += V^T P^T
   auto pv_tile = [&](int t, const f32x16& sc, f32x16& o, float& l_run) {
-    const char* vt_base = kv + (NTM + t) * 2048;
+    const char* vt_base = kv + (NTM + t % NTM) * 2048;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       Frag<bf16> pf, vf;
@@ -1324,13 +953,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // tile, or again the current one at the end), so the compiler's waits
   // count them exactly.
   constexpr int KB = 2;
-  // Epilogue of query tile q0: o / l * gate, stored into og in the output
-  // projection's B-fragment order (og_frag_off): this head's 32 channels are
+  // Epilogue of query tile q0: o / l * gate, stored over the gate tile in the
+  // output projection's order (og_tile_off): this head's 32 channels are
   // 4 chunks of 8; the two half-waves trade quads (v_permlane32_swap) so that
   // the lower one writes chunks 0-1 and the upper one chunks 2-3, each store
   // 32 lanes x 16 bytes contiguous.  next_q: the q tile to copy into the
   // wave's region before the stores (null: none).
-  const int64_t og_tiles = rowbase * (int64_t)nt;  // og tile index of (row, query tile 0)
   auto finish = [&](int q0, const f32x16& o, float l_tot, const bf16* next_q) {
     const float inv = 1.0f / l_tot;
     const int lne = lane + opaque_zero();
@@ -1361,34 +989,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     const uint4 cB = up ? make_uint4(s1x[0], s1y[0], px[3], py[3]) : make_uint4(px[1], py[1], s1x[1], s1y[1]);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // gate read: the region is free for the next q copy
     if (next_q) issue_cq(next_q);
-    const int ks = (h & 1) * 4 + (up ? 2 : 0);  // chunk of cA; cB is ks + 1
-    const uint32_t o_off = (uint32_t)og_frag_off(og_tiles + (q0 >> 5), ks, (h >> 1) * 32 + (lne & 31)) * 2;
-    *reinterpret_cast<uint4*>(reinterpret_cast<char*>(ws.og) + o_off) = cA;
-    *reinterpret_cast<uint4*>(reinterpret_cast<char*>(ws.og) + o_off + 1024) = cB;
+    char* const og = reinterpret_cast<char*>(g_row + (q0 >> 5) * 1024);  // the gate tile, read above
+    const uint32_t o_off = (uint32_t)og_tile_off(up ? 2 : 0, lne & 31) * 2;  // chunk of cA; cB is the next
+    *reinterpret_cast<uint4*>(og + o_off) = cA;
+    *reinterpret_cast<uint4*>(og + o_off + og_tile_off(1, 0) * 2) = cB;
   };
 
   uint4 bq[KB][2];
-  // K fragments of the fast pass's next tile, read one tile ahead (the last
-  // tile of a query tile reads tile 0 for the next query tile)
+  // K fragments of the fast pass's next tile, read one tile ahead
   Frag<bf16> kn[2];
-  int qt = wave;
-  if (qt < nq) {
-    issue_cq(q_row + qt * 1024);
-    if (fast_ok) {
-#pragma unroll
-      for (int u = 0; u < KB; ++u) load_bias(bq[u], qt * 32, u);
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();  // K^T / V^T resident for every wave
-  k_read(0, kn);
-  for (; qt < nq; qt += NW) {
-    const int q0 = qt * 32;
-    const int q0n = (qt + NW < nq ? qt + NW : qt) * 32;  // the query tile to prefetch for
-    // this tile's q copy landed: behind it are, after the first tile, the
-    // previous tile's og stores (2)
-    if (qt != wave) __builtin_amdgcn_s_waitcnt(vmcnt_imm<2>());
-    Frag<bf16> qf[2];
+  auto read_q = [&](Frag<bf16>* qf) {
     const int lnq = lane + opaque_zero();
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
@@ -1397,73 +1007,200 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       qf[m].v = __builtin_bit_cast(bf16x8, v8);
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): q read back, the region is free
-    issue_cq(g_row + qt * 1024);                // the gate tile lands behind the key loop
+  };
+  // Fast pass, tile t in bias buffer u: P = 2^s with no running maximum.
+  // Exact (softmax is shift invariant, and fp32 / bf16 keep relative
+  // precision) while every 2^s stays in range; checked at the end through l,
+  // else the exact pass runs.  tk: the tile whose K fragments are read ahead;
+  // (qb, tb): the bias tile to fetch into buffer u.
+  auto fast_tile = [&](int t, int u, int tk, int qb, int tb, const Frag<bf16>* qf, f32x16& o, float& l_run) {
+    f32x16 sc;
+    widen_bias(sc, bq[u]);
+    s_mma(sc, kn, qf);
+    k_read(tk, kn);
+    mask_tile(t, sc, kBinary);
+    pv_tile(t, sc, o, l_run);
+    load_bias(bq[u], qb, tb);
+    // one sub-tile at a time: interleaving them would need several S
+    // tiles and their fragments live at once
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Exact pass, tile t: online softmax with a running maximum, lazily moved
+  // (only when a tile exceeds it by more than kRescale), bias loaded per tile.
+  auto exact_tile = [&](int t, int q0, const Frag<bf16>* qf, f32x16& o, float& l_run, float& m_ref,
+                        float& m_use) {
+    f32x16 sc;
+    {
+      uint4 bp[2];
+      load_bias(bp, q0, t);
+      widen_bias(sc, bp);
+    }
+    s_tile(t, sc, qf);
+    mask_tile(t, sc, kFrac);
+    // the tile max of the raw scores; the reference is subtracted
+    // afterwards.  (Subtracted first, a reference set by a tile of
+    // masked keys only, about -inf log2 e, would round the logits of the
+    // valid keys that follow to multiples of its fp32 ulp.)
+    float mt = fmaxf(fmaxf(sc[0], sc[1]), sc[2]);
+#pragma unroll
+    for (int e = 3; e < 15; e += 2) mt = fmaxf(fmaxf(mt, sc[e]), sc[e + 1]);
+    mt = lane_pair_max(fmaxf(mt, sc[15]));
+    if (__ballot(mt > m_ref + kRescale) != 0ull) {
+      const float m_new = fmaxf(m_ref, mt);
+      const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[e] *= alpha;
+      m_ref = m_new;
+      m_use = (m_ref == -INFINITY) ? 0.f : m_ref;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sc[e] -= m_use;
+    pv_tile(t, sc, o, l_run);
+  };
+  // In range: the largest term 2^max(s) is within [2^-69, 2^64], so no P
+  // overflows and no term that underflows matters.  Tested on the bits:
+  // positive floats order as unsigned integers, and a NaN, a zero, a
+  // negative value or infinity all fall outside.
+  auto in_range = [&](float l_tot) { return __ballot(!l_in_range(l_tot)) == 0ull; };
 
-    // Fast pass: P = 2^s with no running maximum.  Exact (softmax is shift
-    // invariant, and fp32 / bf16 keep relative precision) while every 2^s
-    // stays in range; checked at the end through l, else the exact pass runs.
+  if constexpr (STREAM) {
+    // The block's query tiles: qg * per_g .. +per_g-1, one a wave (the groups
+    // of a row are of equal size, within one tile).  A wave without a tile
+    // only moves its share of the stages.
+    const int per_g = (nq + qgroups - 1) / qgroups;
+    const int qt = qg * per_g + wave;
+    const bool active = wave < per_g && qt < nq;
+    const int q0 = qt * 32;
+    const int ns = (nk + ST - 1) / ST;
+    if (active) {
+      issue_cq(q_row + qt * 1024);
+      if (fast_ok) {
+#pragma unroll
+        for (int u = 0; u < KB; ++u) load_bias(bq[u], q0, u);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // stage 0 resident for every wave
+    Frag<bf16> qf[2];
+    if (active) {
+      read_q(qf);
+      issue_cq(g_row + qt * 1024);  // the gate tile lands behind the key loop
+    }
+    // Stage s is computed while stage s + 1 is copied into the other half of
+    // kv, which held stage s - 1.  Opening a stage, a wave waits for its own
+    // copies of it, issued during the stage before, ahead of the bias loads of
+    // that stage's last KB tiles (the only ones that may stay in flight); the
+    // barrier makes every wave's copies visible and ends all reads of stage
+    // s - 1.
+    auto open_stage = [&](int s) {
+      if (s > 0) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm<2 * KB>());
+        barrier_only();
+        if ((s * ST) % 64 == 0) kmv = mask_words(s * ST);
+      }
+    };
     f32x16 o = zero16();
-    float l_run = 0.f;
-    for (int t = 0; fast_ok && t < nt; t += KB) {
+    float l_tot = 0.f;
+    bool done = !active;  // nothing (more) to compute for this wave
+    if (fast_ok) {
+      if (active) {
+        float l_run = 0.f;
+        for (int s = 0; s < ns; ++s) {
+          open_stage(s);
+          const int t0 = s * ST, t1 = min(t0 + ST, nk);
+          k_read(t0, kn);
+          for (int t = t0; t < t1; t += KB) {
 #pragma unroll
-      for (int u = 0; u < KB; ++u) {
-        f32x16 sc;
-        widen_bias(sc, bq[u]);
-        s_mma(sc, kn, qf);
-        k_read(t + u + 1 < nt ? t + u + 1 : 0, kn);
-        mask_tile(t + u, sc, kBinary);
-        pv_tile(t + u, sc, o, l_run);
-        const bool wrap = t + u + KB >= nt;
-        load_bias(bq[u], wrap ? q0n : q0, wrap ? t + u + KB - nt : t + u + KB);
-        // one sub-tile at a time: interleaving them would need several S
-        // tiles and their fragments live at once
-        __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < KB; ++u) {
+              // one copy a tile: the wait for a bias tile loaded after it
+              // then has a tile's work to cover it
+              if (s + 1 < ns && t - t0 + u < CPW) stage_piece(s + 1, t - t0 + u);
+              // (the last KB tiles fetch the first KB again)
+              fast_tile(t + u, u, min(t + u + 1, t1 - 1), q0, t + u + KB < nk ? t + u + KB : t + u + KB - nk,
+                        qf, o, l_run);
+            }
+          }
+        }
+        l_tot = lane_pair_sum(l_run);
+        if (in_range(l_tot)) {
+          finish(q0, o, l_tot, nullptr);
+          done = true;
+        }
+      } else {
+        for (int s = 0; s < ns; ++s) {
+          if (s > 0) {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
+            barrier_only();
+          }
+          if (s + 1 < ns)
+            for (int i = 0; i < CPW; ++i) stage_piece(s + 1, i);
+        }
       }
     }
-    float l_tot = lane_pair_sum(l_run);
-    // In range: the largest term 2^max(s) is within [2^-69, 2^64], so no P
-    // overflows and no term that underflows matters.  Tested on the bits:
-    // positive floats order as unsigned integers, and a NaN, a zero, a
-    // negative value or infinity all fall outside.
-    if (!fast_ok || __ballot(!l_in_range(l_tot)) != 0ull) {
-      // Exact pass: online softmax with a running maximum, lazily moved (only
-      // when a tile exceeds it by more than kRescale), bias loaded per tile.
-      o = zero16();
-      l_run = 0.f;
-      float m_ref = -INFINITY, m_use = 0.f;
-      for (int t = 0; t < nt; ++t) {
-        f32x16 sc;
-        {
-          uint4 bp[2];
-          load_bias(bp, q0, t);
-          widen_bias(sc, bp);
-        }
-        s_tile(t, sc, qf);
-        mask_tile(t, sc, kFrac);
-        // the tile max of the raw scores; the reference is subtracted
-        // afterwards.  (Subtracted first, a reference set by a tile of
-        // masked keys only, about -inf log2 e, would round the logits of the
-        // valid keys that follow to multiples of its fp32 ulp.)
-        float mt = fmaxf(fmaxf(sc[0], sc[1]), sc[2]);
+    // Exact pass, for the waves that need it: all waves stream K and V again.
+    // (Whether any does goes through kv, free by then: LDS is full.)
+    __syncthreads();
+    int* const flags = reinterpret_cast<int*>(kv);
+    if (lane == 0) flags[wave] = done ? 0 : 1;
+    __syncthreads();
+    if (__ballot(lane < NW && flags[lane & (NW - 1)] != 0) == 0ull) return;
+    __syncthreads();
+    float l_run = 0.f, m_ref = -INFINITY, m_use = 0.f;
+    o = zero16();
+    for (int s = 0; s < ns; ++s) {
+      if (s > 0) __syncthreads();  // the stage before is read by every wave
 #pragma unroll
-        for (int e = 3; e < 15; e += 2) mt = fmaxf(fmaxf(mt, sc[e]), sc[e + 1]);
-        mt = lane_pair_max(fmaxf(mt, sc[15]));
-        if (__ballot(mt > m_ref + kRescale) != 0ull) {
-          const float m_new = fmaxf(m_ref, mt);
-          const float alpha = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
-          l_run *= alpha;
-#pragma unroll
-          for (int e = 0; e < 16; ++e) o[e] *= alpha;
-          m_ref = m_new;
-          m_use = (m_ref == -INFINITY) ? 0.f : m_ref;
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) sc[e] -= m_use;
-        pv_tile(t, sc, o, l_run);
-      }
-      l_tot = lane_pair_sum(l_run);
+      for (int i = 0; i < CPW; ++i) stage_piece(s, i);
+      if ((s * ST) % 64 == 0) kmv = mask_words(s * ST);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      if (!done)
+        for (int t = s * ST; t < min(s * ST + ST, nk); ++t) exact_tile(t, q0, qf, o, l_run, m_ref, m_use);
     }
-    finish(q0, o, l_tot, qt + NW < nq ? q_row + (qt + NW) * 1024 : nullptr);
+    if (!done) finish(q0, o, lane_pair_sum(l_run), nullptr);
+  } else {
+    int qt = wave;
+    if (qt < nq) {
+      issue_cq(q_row + qt * 1024);
+      if (fast_ok) {
+#pragma unroll
+        for (int u = 0; u < KB; ++u) load_bias(bq[u], qt * 32, u);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // K^T / V^T resident for every wave
+    k_read(0, kn);
+    for (; qt < nq; qt += NW) {
+      const int q0 = qt * 32;
+      const int q0n = (qt + NW < nq ? qt + NW : qt) * 32;  // the query tile to prefetch for
+      // this tile's q copy landed: behind it are, after the first tile, the
+      // previous tile's og stores (2)
+      if (qt != wave) __builtin_amdgcn_s_waitcnt(vmcnt_imm<2>());
+      Frag<bf16> qf[2];
+      read_q(qf);
+      issue_cq(g_row + qt * 1024);  // the gate tile lands behind the key loop
+      f32x16 o = zero16();
+      float l_run = 0.f;
+      for (int t = 0; fast_ok && t < nk; t += KB) {
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+          // the last tile reads tile 0's K fragments for the next query tile
+          const bool wrap = t + u + KB >= nk;
+          fast_tile(t + u, u, t + u + 1 < nk ? t + u + 1 : 0, wrap ? q0n : q0,
+                    wrap ? t + u + KB - nk : t + u + KB, qf, o, l_run);
+        }
+      }
+      float l_tot = lane_pair_sum(l_run);
+      if (!fast_ok || !in_range(l_tot)) {
+        o = zero16();
+        l_run = 0.f;
+        float m_ref = -INFINITY, m_use = 0.f;
+        for (int t = 0; t < nk; ++t) exact_tile(t, q0, qf, o, l_run, m_ref, m_use);
+        l_tot = lane_pair_sum(l_run);
+      }
+      finish(q0, o, l_tot, qt + NW < nq ? q_row + (qt + NW) * 1024 : nullptr);
+    }
   }
 }
 
@@ -1472,8 +1209,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
 //     out[pair] = og[row][q] . W_o^T + b_o (+ x[pair]) at the source pair of
 //     (row, q).  Persistent blocks of 8 waves (two per CU), W_o (packed, 32
 //     KiB) and b_o in LDS; one tile = 32 consecutive queries of one row.
-//   * og arrives in fragment order (og_frag_off): 8 loads of 1 KiB
-//     contiguous, issued with the residual rows at the start of the tile
+//   * og arrives in fragment order (og_tile_off): 8 loads of two 512-byte
+//     runs, issued with the residual rows at the start of the tile
 //     (four waves per SIMD hide their latency).
 //   * The result is transposed through the wave's 4 KiB LDS region in two
 //     halves of 64 channels (bf16 update, rows of 128 bytes, chunk c of row q
@@ -1505,20 +1242,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
   const int t32 = lane & 31;
   char* const sw = stg[wave];
   const int qtiles = (N + 31) / 32;
-  const int ntq = Np / 32;  // og tiles per workspace row
   const int64_t stride = (int64_t)gridDim.x * 8;
-  auto og_tile = [&](int64_t tile) {
-    const int qtl = (int)(tile % qtiles);
-    const int64_t br = tile / qtiles;
-    const int b = (int)(br / nrows);
-    const int r = r0 + (int)(br - (int64_t)b * nrows);
-    return ws.row(b, r) * ntq + qtl;
-  };
-  auto load_og = [&](Frag<bf16>* of, int64_t tile) {
-    const bf16* src = ws.og + og_frag_off(og_tile(tile), 0, lane);
-#pragma unroll
-    for (int ks = 0; ks < KC; ++ks) of[ks].load(src + ks * 512);
-  };
   for (int64_t tile = (int64_t)blockIdx.x * 8 + wave; tile < ntiles; tile += stride) {
     const int qtl = (int)(tile % qtiles);
     const int64_t br = tile / qtiles;
@@ -1527,10 +1251,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
     // row-pass lanes: query qq = 8i + lane/8 of the tile, 16-byte chunk lane%8
     // of a 64-channel half
     const int rq = lane >> 3, rc = lane & 7;
-    const auto ors = buf_rsrc(out + (int64_t)b * N * N * CIN, (uint32_t)((int64_t)N * N * CIN * 2));
-    auto pair_of = [&](int q) {  // source pair of (row r, query q), q < N
-      return starting ? ((int64_t)r * N + q) : ((int64_t)q * N + r);
-    };
+    // source pair of (row r, query qtl * 32 + qq): p0 + qq * pstep; the output
+    // descriptor spans the tile's 32 pairs, so its offsets fit 32 bits at any N
+    const int64_t p0 = (int64_t)b * N * N + (starting ? (int64_t)r * N + qtl * 32 : (int64_t)qtl * 32 * N + r);
+    const int pstep = starting ? 1 : N;
+    const auto ors = buf_rsrc(out + p0 * CIN, (uint32_t)pstep * (32 * CIN * 2));
     // residual rows of this tile (queries >= N read pair 0 and are not stored)
     uint4 xr[2][4];
     if (residual) {
@@ -1538,13 +1263,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
       for (int hp = 0; hp < 2; ++hp)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int q = qtl * 32 + 8 * i + rq;
-          const int64_t pr = q < N ? pair_of(q) : 0;
-          xr[hp][i] = *reinterpret_cast<const uint4*>(x + ((int64_t)b * N * N + pr) * CIN + hp * 64 + rc * 8);
+          const int qq = 8 * i + rq;
+          const int64_t pr = qtl * 32 + qq < N ? p0 + (int64_t)qq * pstep : 0;
+          xr[hp][i] = *reinterpret_cast<const uint4*>(x + pr * CIN + hp * 64 + rc * 8);
         }
     }
+    // chunk ks of lane (query t32, half): chunk ks & 3 of head 2 * half + ks / 4
     Frag<bf16> cur[KC];
-    load_og(cur, tile);
+    const bf16* og = ws.gate + (ws.row(b, r) * 4 + 2 * half) * (int64_t)HD * Np + qtl * 1024;
+#pragma unroll
+    for (int ks = 0; ks < KC; ++ks)
+      cur[ks].load(og + (ks >> 2) * (int64_t)HD * Np + og_tile_off(ks & 3, t32));
     const bf16* wlt = wl + opaque_zero();  // keep the W_o reads in the loop
 #pragma unroll
     for (int hp = 0; hp < 2; ++hp) {
@@ -1581,8 +1310,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
           v = make_uint4(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]),
                          pack_bf16x2(s[6], s[7]));
         }
-        const int q = qtl * 32 + qq;
-        buf_store16(ors, q < N ? (uint32_t)((pair_of(q) * CIN + hp * 64 + rc * 8) * 2) : kBufSkip, v);
+        const bool ok = qtl * 32 + qq < N;
+        buf_store16(ors, ok ? (uint32_t)((qq * pstep * CIN + hp * 64 + rc * 8) * 2) : kBufSkip, v);
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);  // the region is read back before the next half
     }
@@ -1768,60 +1497,56 @@ static int fwd_triattn(const void* x, const float* mask, void* out, const void* 
   const int64_t blocks = B * N * ((N + 31) / 32);
   GTK_REQUIRE(blocks < (1ll << 31), GTK_EUNSUPPORTED, "attention grid too large");
   if constexpr (kFast) {
-    constexpr int QT = 2;  // two 8-wave blocks of 64 queries per CU (Np > kFlashRhMaxNp)
-    const bool rh = Np <= kFlashRhMaxNp;  // (row, head) flash path, fragment-order bf16 bias
+    // position tiles that hold a pair, in twos (the flash kernel attends key
+    // tiles in pairs), of the rows below N rounded up to a query tile
+    const int vtiles = (int)round_up((N + 31) / 32, 2);
+    const int rows_all = (int)round_up(N, 32);
     auto prologue = [&](auto mode, int r0, int nrows) {
       constexpr int MODE = decltype(mode)::value;
-      const int64_t ptiles = B * (int64_t)nrows * (Np / 32);
+      const int64_t ptiles = B * (int64_t)nrows * vtiles;
       const int grid = (int)std::min<int64_t>(device_cus(), (ptiles + 7) / 8);
       StageTimer timer("triattn_prologue", st);
       triattn_prologue_bf16_kernel<CIN, H, MODE><<<grid, 1024, 0, st>>>(
-          (const bf16*)x, mask, w, a, (int)N, Np, starting, eps, ptiles, r0, nrows);
+          (const bf16*)x, mask, w, a, (int)N, Np, starting, eps, ptiles, r0, nrows, vtiles);
     };
     auto flash = [&](int r0, int nrows) {
-      if (rh) {
-        // (row, head) blocks, then the output projection
-        const int64_t fblocks = B * nrows * H;
-        {
-          StageTimer timer("triattn_flash", st);
-          if (Np <= 256)
-            triattn_flash_rh_kernel<256, 8><<<(unsigned)fblocks, 512, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf);
-          else if (Np <= 512)
-            triattn_flash_rh_kernel<512, 8><<<(unsigned)fblocks, 512, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf);
-          else
-            triattn_flash_rh_kernel<1024, 16><<<(unsigned)fblocks, 1024, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf);
-        }
-        GTK_HIP_CHECK(hipGetLastError());
-        const int64_t otiles = B * nrows * ((N + 31) / 32);
-        const int grid = (int)std::min<int64_t>(2 * device_cus(), (otiles + 7) / 8);
-        StageTimer timer("triattn_out", st);
-        triattn_out_kernel<CIN><<<grid, 512, 0, st>>>((const bf16*)x, (bf16*)out, w, a, (int)N, Np, starting,
-                                                      residual, r0, nrows, otiles);
-        return GTK_OK;
+      // (row, head) blocks, then the output projection.  Above Np = 1024 the
+      // keys of a row and head no longer fit in LDS: they stream through it,
+      // and a block takes up to 8 of the row's query tiles.
+      const int qgroups = Np > 1024 ? (int)((N + 255) / 256) : 1;
+      const int64_t fblocks = B * nrows * H * qgroups;
+      GTK_REQUIRE(fblocks < (1ll << 31), GTK_EUNSUPPORTED, "attention grid too large");
+      {
+        StageTimer timer("triattn_flash", st);
+        if (Np <= 256)
+          triattn_flash_rh_kernel<256, 8, false><<<(unsigned)fblocks, 512, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf, vtiles, 1);
+        else if (Np <= 512)
+          triattn_flash_rh_kernel<512, 8, false><<<(unsigned)fblocks, 512, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf, vtiles, 1);
+        else if (Np <= 1024)
+          triattn_flash_rh_kernel<1024, 16, false><<<(unsigned)fblocks, 1024, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf, vtiles, 1);
+        else
+          triattn_flash_rh_kernel<512, 8, true><<<(unsigned)fblocks, 512, 0, st>>>(mask, a, (int)N, Np, starting, r0, nrows, inf, vtiles, qgroups);
       }
-      const int64_t fblocks = B * nrows * ((N + 32 * QT - 1) / (32 * QT));
-      StageTimer timer("triattn_flash", st);
-      triattn_flash_kernel<CIN, H, QT><<<(unsigned)fblocks, 64 * H * QT, 0, st>>>(
-          (const bf16*)x, mask, (bf16*)out, w, a, (int)N, Np, starting, residual, r0, nrows, inf);
+      GTK_HIP_CHECK(hipGetLastError());
+      const int64_t otiles = B * nrows * ((N + 31) / 32);
+      const int grid = (int)std::min<int64_t>(2 * device_cus(), (otiles + 7) / 8);
+      StageTimer timer("triattn_out", st);
+      triattn_out_kernel<CIN><<<grid, 512, 0, st>>>((const bf16*)x, (bf16*)out, w, a, (int)N, Np, starting,
+                                                    residual, r0, nrows, otiles);
       return GTK_OK;
     };
     if (!chunked) {
-      // every row, padding included
-      if (rh) prologue(std::integral_constant<int, 15>(), 0, Np);
-      else prologue(std::integral_constant<int, 3>(), 0, Np);
+      prologue(std::integral_constant<int, 3>(), 0, rows_all);
       GTK_LAUNCH_CHECK();
       if (int rc = flash(0, (int)N)) return rc;
       GTK_LAUNCH_CHECK();
     } else {
-      // the bias over every row (padding rows and columns are written as zero)
-      if (rh) prologue(std::integral_constant<int, 6>(), 0, Np);
-      else prologue(std::integral_constant<int, 2>(), 0, Np);
+      prologue(std::integral_constant<int, 2>(), 0, rows_all);  // the bias over every row
       GTK_LAUNCH_CHECK();
       for (int64_t r0 = 0; r0 < N; r0 += chunk_rows) {
         const int nrows = (int)std::min<int64_t>(chunk_rows, N - r0);
         a.r0 = (int)r0;
-        if (rh) prologue(std::integral_constant<int, 9>(), (int)r0, nrows);
-        else prologue(std::integral_constant<int, 1>(), (int)r0, nrows);
+        prologue(std::integral_constant<int, 1>(), (int)r0, nrows);
         GTK_LAUNCH_CHECK();
         if (int rc = flash((int)r0, nrows)) return rc;
         GTK_LAUNCH_CHECK();

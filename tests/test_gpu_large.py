@@ -20,6 +20,7 @@ from oracle import grads, pair_ops
 from tests import helpers as H
 from tests.gpu_common import check_bf16, log, to_np, triattn_module, trimul_module
 from tests.test_gpu_grads import _check_grad
+from tests.test_gpu_kernels import logit_offset_qk_params
 
 pytestmark = pytest.mark.gpu
 
@@ -55,8 +56,8 @@ def _inputs(N: int):
 @pytest.mark.parametrize("starting", [True, False])
 @pytest.mark.parametrize("N", [1152, 2048])
 def test_tri_attn_forward_beyond_1024(starting, N):
-    """bf16 forward for Np > 1024 (the streaming flash kernel with the K/V ring,
-    the bf16 bias through the identity MFMA and W_o fused), sampled rows
+    """bf16 forward for Np > 1024 (the streamed form of the (row, head) flash
+    kernel), sampled rows
     against the oracle: fp32 arithmetic on the bf16-rounded inputs (float64
     at N = 1152)."""
     log(f"tri_attn forward N={N} starting={starting}")
@@ -176,3 +177,31 @@ def test_tri_mul_row_chunks_2048(outgoing):
     del y
     ref = pair_ops.tri_mul(x, m, P, outgoing, dtype=np.float32, rows=rows)
     check_bf16(got, ref, f"tri_mul chunks N={N} outgoing={outgoing}")
+
+
+@pytest.mark.parametrize("starting", [True, False])
+@pytest.mark.parametrize("N,offset", [(1025, 0.0), (1060, 200.0), (2100, 0.0)])
+def test_tri_attn_streamed_keys(starting, N, offset):
+    """The streamed form of the (row, head) kernel where it can go wrong: one
+    query and key tile past the resident form's range (a last stage of two
+    tiles), more than 64 key tiles (the key-mask words are read again), and
+    logits whose max-free pass overflows, so that every block streams its keys
+    a second time for the exact pass (mask None: with masked keys the oracle
+    holds only for |logit| < 32).  Sampled rows against the oracle."""
+    log(f"tri_attn streamed keys N={N} starting={starting} offset={offset}")
+    if offset:
+        P = logit_offset_qk_params(offset)
+        x, m = H.bf16_round(H.pair_input(1, N, 128, seed=N)), None
+    else:
+        x, m, P, _ = _inputs(N)
+    rows = sorted({0, 31, 100, 200, N - 38, N - 37, N - 1})
+    mod = triattn_module(P, starting, 4, torch.bfloat16)
+    with torch.no_grad():
+        y = mod(torch.from_numpy(x).to("cuda", torch.bfloat16),
+                None if m is None else torch.from_numpy(m).to("cuda"))
+    torch.cuda.synchronize()
+    sel = (lambda a: a[:, rows]) if starting else (lambda a: a[:, :, rows])
+    got = to_np(sel(y))
+    del y
+    ref = pair_ops.tri_attn(x, m, P, starting, 4, dtype=np.float32, rows=rows)
+    check_bf16(got, ref, f"tri_attn N={N} starting={starting} offset={offset}")
