@@ -269,15 +269,17 @@ __device__ __forceinline__ void ln_affine_to_frags(Frag<T>* frags, const RowHalf
 // LayerNorm (normalisation only) of the pair row held as raw bf16 fragments:
 // lane l holds channels (l>>5)*C/2 + 8*ch + e of its row in raw[ch]; the two
 // lanes of a row exchange partial sums with one lane^32 swap.
+// mean, rstd: the row's statistics.
 template <int C>
-__device__ __forceinline__ void ln_frags_bf16(Frag<bf16>* xf, const Frag<bf16>* raw, float eps) {
+__device__ __forceinline__ void ln_frags_bf16(Frag<bf16>* xf, const Frag<bf16>* raw, float eps, float& mean,
+                                              float& rstd) {
   float s = 0.f;
 #pragma unroll
   for (int ch = 0; ch < C / 16; ++ch)
 #pragma unroll
     for (int e = 0; e < 8; ++e) s += raw[ch].get(e);
   s += xor32(s);
-  const float mean = s * (1.0f / C);
+  mean = s * (1.0f / C);
   float q = 0.f;
 #pragma unroll
   for (int ch = 0; ch < C / 16; ++ch)
@@ -287,7 +289,7 @@ __device__ __forceinline__ void ln_frags_bf16(Frag<bf16>* xf, const Frag<bf16>* 
       q += d * d;
     }
   q += xor32(q);
-  const float rstd = __builtin_amdgcn_rsqf(q * (1.0f / C) + eps);  // v_rsq_f32 (1 ulp)
+  rstd = __builtin_amdgcn_rsqf(q * (1.0f / C) + eps);  // v_rsq_f32 (1 ulp)
 #pragma unroll
   for (int ch = 0; ch < C / 16; ++ch) {
     float f[8];
@@ -295,6 +297,11 @@ __device__ __forceinline__ void ln_frags_bf16(Frag<bf16>* xf, const Frag<bf16>* 
     for (int e = 0; e < 8; ++e) f[e] = (raw[ch].get(e) - mean) * rstd;
     xf[ch].set(f);
   }
+}
+template <int C>
+__device__ __forceinline__ void ln_frags_bf16(Frag<bf16>* xf, const Frag<bf16>* raw, float eps) {
+  float mean, rstd;
+  ln_frags_bf16<C>(xf, raw, eps, mean, rstd);
 }
 
 // Load and normalise the pair row at row_base (zeros when !valid).
