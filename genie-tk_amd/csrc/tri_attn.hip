@@ -80,9 +80,10 @@ template <typename T> struct AttnWs {
   T *q, *k, *vt, *gate, *bias;
   // (row, head) flash path (bf16 module forward), else null: the triangle
   // bias without its per-head constant in bf16, B x H x Np x Np in the flash
-  // kernel's fragment order (bias_frag_off; then bias is empty).  That path
-  // writes the gated attention output over the gate (og_tile_off).
+  // kernel's fragment order (bias_frag_off; then bias is empty), and the gated
+  // attention output (og_tile_off; the gate itself where Np > kOgOwnMaxNp)
   bf16* biasfr;
+  T* og;
   // (row, head) flash path, else null: the key-mask bits of every attention
   // row (B x Np x Np/32 words: bit j of word t is key 32t + j, set for a
   // mask value other than 1) and the flags of each key tile (B x Np x Np/32:
@@ -102,12 +103,17 @@ template <typename T> struct AttnWs {
 // Rows and positions are padded to a multiple of the flash kernel's query block.
 inline int64_t attn_pad(int64_t N) { return round_up(N, 128); }
 
-// Gated attention output og of the (row, head) path.  The wave that attends
-// (row, head, query tile) is the only reader of that 2 KiB tile of the gate,
-// so it writes its output tile there: 4 chunks of 8 channels, each [32
-// queries][8], which the output projection's B fragments read as 512-byte
-// runs (chunk ks & 3 of head 2 * (lane / 32) + ks / 4).  Element offset of
-// chunk k4, query q of a tile:
+// Gated attention output og of the (row, head) path, in 2 KiB tiles like the
+// gate's ([B][rows][H][Np/32] of 32 channels x 32 queries): 4 chunks of 8
+// channels, each [32 queries][8], which the output projection's B fragments
+// read as 512-byte runs (chunk ks & 3 of head 2 * (lane / 32) + ks / 4).  The
+// wave that attends (row, head, query tile) is the only reader of the gate
+// tile it replaces, so og may take the gate's place.  It does where the
+// workspace is large (N = 2048: 1 GiB less); below, a buffer of its own leaves
+// the next call's prologue 2 us faster at N = 200 (20 against 22 us), which
+// otherwise rewrites lines that the flash kernel's XCDs have just written.
+// Element offset of chunk k4, query q of a tile:
+constexpr int64_t kOgOwnMaxNp = 1024;
 __host__ __device__ __forceinline__ int og_tile_off(int k4, int q) { return (k4 * 32 + q) * 8; }
 
 // bf16 triangle bias of the (row, head) path, per batch element, in the
@@ -149,6 +155,7 @@ static AttnWs<T> carve_attn_ws(Carve& cv, int64_t B, int64_t Np, int H, int ch, 
   w.gate = cv.take<T>(ch > 0 ? B * w.rows * Np * ch : 0);
   const bool rh = fast && ch > 0 && sizeof(T) == 2;
   w.bias = rh ? nullptr : cv.take<T>(B * H * Np * Np);
+  w.og = rh && Np <= kOgOwnMaxNp ? cv.take<T>(B * w.rows * Np * ch) : w.gate;
   w.biasfr = rh ? cv.take<bf16>(B * H * Np * Np) : nullptr;
   w.mbits = rh ? cv.take<uint32_t>(B * Np * (Np / 32)) : nullptr;
   w.mflags = rh ? cv.take<int>(B * Np * (Np / 32)) : nullptr;
@@ -830,11 +837,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // q or gate tile [32 channels][32 queries] (2 KiB contiguous in the tiled
   // layout) -> the wave's region, 64-byte rows; copy j moves channels
   // 16j .. 16j+15, lane l takes channel 16j + l/4, queries 8*(l%4) .. +7
-  auto issue_cq = [&](const bf16* src) {
+  // (q is read once and for all: non-temporal.  The gate's copy goes plain: the
+  // flash kernel took 137 -> 132 us at N = 512 that way, 62 -> 60 at 384.)
+  auto issue_cq = [&](const bf16* src, bool nt_hint = true) {
     const uint32_t ln = (uint32_t)(lane + opaque_zero());
     const uint32_t voff = ln * 16;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) g2lds16_sv_nt(src + j * 512, voff, stg_lds + j * 1024);
+    for (int j = 0; j < 2; ++j) {
+      if (nt_hint) g2lds16_sv_nt(src + j * 512, voff, stg_lds + j * 1024);
+      else g2lds16_sv(src + j * 512, voff, stg_lds + j * 1024);
+    }
   };
   // channels c0 .. c0+3 of this lane's query t32 (transposing read); ln is
   // the lane id through opaque_zero, so that these per-lane addresses are
@@ -844,7 +856,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     return lds_read_tr16(sw + (c0 + (i >> 2)) * 64 + (16 * ((ln >> 4) & 1) + 4 * (i & 3)) * 2);
   };
   const bf16* q_row = ws.q + ((rowbase * H + h) * HD) * (int64_t)Np;
-  bf16* g_row = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np;
+  const bf16* g_row = ws.gate + (rowbase * CH + h * HD) * (int64_t)Np;
   const bf16* b_head = ws.biasfr + (int64_t)(b * H + h) * Np * Np;  // wave-uniform
 
   // K fragments (transposing reads of K^T) and V^T fragments: per-lane offsets
@@ -953,7 +965,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // tile, or again the current one at the end), so the compiler's waits
   // count them exactly.
   constexpr int KB = 2;
-  // Epilogue of query tile q0: o / l * gate, stored over the gate tile in the
+  // Epilogue of query tile q0: o / l * gate, stored into og in the
   // output projection's order (og_tile_off): this head's 32 channels are
   // 4 chunks of 8; the two half-waves trade quads (v_permlane32_swap) so that
   // the lower one writes chunks 0-1 and the upper one chunks 2-3, each store
@@ -989,7 +1001,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     const uint4 cB = up ? make_uint4(s1x[0], s1y[0], px[3], py[3]) : make_uint4(px[1], py[1], s1x[1], s1y[1]);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // gate read: the region is free for the next q copy
     if (next_q) issue_cq(next_q);
-    char* const og = reinterpret_cast<char*>(g_row + (q0 >> 5) * 1024);  // the gate tile, read above
+    // (og may be the gate: this tile of it was read above)
+    char* const og = reinterpret_cast<char*>(ws.og + (rowbase * CH + h * HD) * (int64_t)Np + (q0 >> 5) * 1024);
     const uint32_t o_off = (uint32_t)og_tile_off(up ? 2 : 0, lne & 31) * 2;  // chunk of cA; cB is the next
     *reinterpret_cast<uint4*>(og + o_off) = cA;
     *reinterpret_cast<uint4*>(og + o_off + og_tile_off(1, 0) * 2) = cB;
@@ -1085,7 +1098,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     Frag<bf16> qf[2];
     if (active) {
       read_q(qf);
-      issue_cq(g_row + qt * 1024);  // the gate tile lands behind the key loop
+      issue_cq(g_row + qt * 1024, false);  // the gate tile lands behind the key loop
     }
     // Stage s is computed while stage s + 1 is copied into the other half of
     // kv, which held stage s - 1.  Opening a stage, a wave waits for its own
@@ -1179,7 +1192,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       if (qt != wave) __builtin_amdgcn_s_waitcnt(vmcnt_imm<2>());
       Frag<bf16> qf[2];
       read_q(qf);
-      issue_cq(g_row + qt * 1024);  // the gate tile lands behind the key loop
+      issue_cq(g_row + qt * 1024, false);  // the gate tile lands behind the key loop
       f32x16 o = zero16();
       float l_run = 0.f;
       for (int t = 0; fast_ok && t < nk; t += KB) {
@@ -1243,11 +1256,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
   char* const sw = stg[wave];
   const int qtiles = (N + 31) / 32;
   const int64_t stride = (int64_t)gridDim.x * 8;
-  for (int64_t tile = (int64_t)blockIdx.x * 8 + wave; tile < ntiles; tile += stride) {
-    const int qtl = (int)(tile % qtiles);
-    const int64_t br = tile / qtiles;
-    const int b = (int)(br / nrows);
-    const int r = r0 + (int)(br - (int64_t)b * nrows);
+  const int64_t tile0 = (int64_t)blockIdx.x * 8 + wave;
+  TileWalk tw;
+  tw.init(tile0, stride, nrows, qtiles);
+  for (int64_t tile = tile0; tile < ntiles; tile += stride, tw.next()) {
+    const int qtl = tw.c;
+    const int b = tw.b;
+    const int r = r0 + tw.r;
     // row-pass lanes: query qq = 8i + lane/8 of the tile, 16-byte chunk lane%8
     // of a 64-channel half
     const int rq = lane >> 3, rc = lane & 7;
@@ -1270,10 +1285,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
     }
     // chunk ks of lane (query t32, half): chunk ks & 3 of head 2 * half + ks / 4
     Frag<bf16> cur[KC];
-    const bf16* og = ws.gate + (ws.row(b, r) * 4 + 2 * half) * (int64_t)HD * Np + qtl * 1024;
+    // (a wave-uniform base plus a 32-bit offset a lane)
+    const uint32_t og_lane = (uint32_t)(half * 2 * HD * Np + t32 * 8) * 2;
 #pragma unroll
-    for (int ks = 0; ks < KC; ++ks)
-      cur[ks].load(og + (ks >> 2) * (int64_t)HD * Np + og_tile_off(ks & 3, t32));
+    for (int h2 = 0; h2 < 2; ++h2) {
+      const char* og = reinterpret_cast<const char*>(ws.og + (ws.row(b, r) * 4 + h2) * (int64_t)HD * Np + qtl * 1024);
+#pragma unroll
+      for (int k4 = 0; k4 < 4; ++k4)
+        cur[4 * h2 + k4].load(reinterpret_cast<const bf16*>(og + og_lane + og_tile_off(k4, 0) * 2));
+    }
     const bf16* wlt = wl + opaque_zero();  // keep the W_o reads in the loop
 #pragma unroll
     for (int hp = 0; hp < 2; ++hp) {
@@ -1504,7 +1524,7 @@ static int fwd_triattn(const void* x, const float* mask, void* out, const void* 
     auto prologue = [&](auto mode, int r0, int nrows) {
       constexpr int MODE = decltype(mode)::value;
       const int64_t ptiles = B * (int64_t)nrows * vtiles;
-      const int grid = (int)std::min<int64_t>(device_cus(), (ptiles + 7) / 8);
+      const int grid = (int)std::min<int64_t>(device_cus(), (ptiles + 3) / 4);
       StageTimer timer("triattn_prologue", st);
       triattn_prologue_bf16_kernel<CIN, H, MODE><<<grid, 1024, 0, st>>>(
           (const bf16*)x, mask, w, a, (int)N, Np, starting, eps, ptiles, r0, nrows, vtiles);
