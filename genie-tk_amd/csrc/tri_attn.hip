@@ -763,7 +763,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const int nt = Np / 32;             // tiles of a workspace row
   const int nq = (N + 31) / 32;       // query tiles holding real queries
   // nk: key tiles attended, those with real keys rounded up to a pair
-  const int lin = (int)xcd_remap(blockIdx.x, gridDim.x);
+  const int lin = (int)(STREAM ? xcd_remap_any(blockIdx.x, gridDim.x) : xcd_remap(blockIdx.x, gridDim.x));
   const int per_h = (int)gridDim.x / H;
   const int h = lin / per_h;
   int rem = lin - h * per_h;
