@@ -44,8 +44,15 @@ inline int64_t plane_stride(int64_t rows, int64_t Np) {
 //    (0: A, 1: Bm).  Whole planes: r0 = 0, nrows = Np, sides 0 .. 1; the row
 //    chunks of the memory-bounded mode write Bm once over all rows and A one
 //    chunk of rows at a time.
+//
+// Generic form (fp32 and the shapes without a fast kernel): one wave per
+// 32-pair tile, weights from L2.  The 2 CH/32 (side, channel tile) units of a
+// tile are dealt over gridDim.y waves, each of which normalises the tile again:
+// a tile's products are a serial chain of 64 matrix instructions a unit and
+// projection, 30 us for all units in fp32, so a small problem needs its waves
+// (SPLIT, units_split).
 // ---------------------------------------------------------------------------
-template <typename T, int CZ, int CH>
+template <typename T, int CZ, int CH, bool SPLIT>
 __global__ __launch_bounds__(256) void trimul_prologue_kernel(
     const T* __restrict__ z, const float* __restrict__ mask, T* __restrict__ pa,
     T* __restrict__ pb, TriMulPacked<T> w, int B, int N, int Np, int outgoing, float eps,
@@ -75,27 +82,33 @@ __global__ __launch_bounds__(256) void trimul_prologue_kernel(
   const float m = valid ? (mask ? mask[pair] : 1.0f) : 0.0f;
 
   const int64_t off_fv = (int64_t)fl * Np + v;
-#pragma unroll 1
-  for (int side = side_lo; side < side_hi; ++side) {
+  auto unit = [&](int side, int nt) {
     const T* wp = side ? w.w_bp : w.w_ap;
     const T* wg = side ? w.w_bg : w.w_ag;
     const float* bp = side ? w.b_bp : w.b_ap;
     const float* bg = side ? w.b_bg : w.b_ag;
     T* dst = (side ? pb : pa) + (int64_t)b * CH * plane + off_fv;
-#pragma unroll 1
-    for (int nt = 0; nt < CH / 32; ++nt) {
-      const f32x16 ap = row_gemm_tile<T, CZ, true>(xf, wp, nt);
-      const f32x16 ag = row_gemm_tile<T, CZ, true>(xf, wg, nt);
+    const f32x16 ap = row_gemm_tile<T, CZ, true>(xf, wp, nt);
+    const f32x16 ag = row_gemm_tile<T, CZ, true>(xf, wg, nt);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < 4; ++g) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int c = nt * 32 + 8 * g + 4 * half + r;
-          const float val = (ap[4 * g + r] + bp[c]) * gate_from_u(ag[4 * g + r] + bg[c]) * m;
-          dst[(int64_t)c * plane] = cvt<T>(val);
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int c = nt * 32 + 8 * g + 4 * half + r;
+        const float val = (ap[4 * g + r] + bp[c]) * gate_from_u(ag[4 * g + r] + bg[c]) * m;
+        dst[(int64_t)c * plane] = cvt<T>(val);
       }
     }
+  };
+  if constexpr (SPLIT) {
+#pragma unroll 1
+    for (int u = blockIdx.y; u < (side_hi - side_lo) * (CH / 32); u += gridDim.y)
+      unit(side_lo + u / (CH / 32), u % (CH / 32));
+  } else {
+#pragma unroll 1
+    for (int side = side_lo; side < side_hi; ++side)
+#pragma unroll 1
+      for (int nt = 0; nt < CH / 32; ++nt) unit(side, nt);
   }
 }
 
@@ -788,8 +801,12 @@ __global__ __launch_bounds__(64 * (TI / 64) * (TJ / 64)) void trimul_contract_fp
 //    Both epilogues produce output rows i = r0 .. r0 + nrows - 1 from rows
 //    i - r0 of the x planes, which hold xrows x Np (whole planes: r0 = 0,
 //    nrows = N, xrows = Np).
+//
+// Generic form: one wave per 32-pair tile and NTB of its output channel tiles
+// (blockIdx.y), weights from L2.  NTB < CZ / 32 where the tiles alone would
+// leave the chip without waves (units_split; N = 64 fp32: 32 -> 18 us).
 // ---------------------------------------------------------------------------
-template <typename T, int CZ, int CH>
+template <typename T, int CZ, int CH, int NTB>
 __global__ __launch_bounds__(256) void trimul_epilogue_kernel(
     const T* __restrict__ z, const T* __restrict__ px, T* __restrict__ out, TriMulPacked<T> w,
     int B, int N, int Np, int residual, float eps_in, float eps_out, int r0, int nrows, int xrows,
@@ -812,7 +829,8 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(
   const int64_t pair = ((int64_t)b * N + i) * N + (valid ? j : 0);
 
   // Gate from z.
-  f32x16 gate[CZ / 32];
+  f32x16 gate[NTB];
+  const int nt0 = NTB == CZ / 32 ? 0 : blockIdx.y * NTB;
   {
     RowHalf<CZ> rh;
     load_row_half<T, CZ>(rh, z + pair * CZ, valid);
@@ -821,13 +839,13 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(
     if constexpr (trimul_folded<CZ, CH>()) ln_to_frags<T, CZ>(xf, rh, st);
     else ln_affine_to_frags<T, CZ>(xf, rh, st, w.ln_in_w, w.ln_in_b);
 #pragma unroll
-    for (int nt = 0; nt < CZ / 32; ++nt) {
-      gate[nt] = row_gemm_tile<T, CZ, true>(xf, w.w_g, nt);
+    for (int nt = 0; nt < NTB; ++nt) {
+      gate[nt] = row_gemm_tile<T, CZ, true>(xf, w.w_g, nt0 + nt);
 #pragma unroll
       for (int g = 0; g < 4; ++g)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int c = nt * 32 + 8 * g + 4 * half + r;
+          const int c = (nt0 + nt) * 32 + 8 * g + 4 * half + r;
           gate[nt][4 * g + r] = gate_from_u(gate[nt][4 * g + r] + w.b_g[c]);
         }
     }
@@ -869,12 +887,12 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(
   else ln_affine_to_frags<T, CH>(yf, xh, st, w.ln_out_w, w.ln_out_b);
 
 #pragma unroll
-  for (int nt = 0; nt < CZ / 32; ++nt) {
-    const f32x16 acc = row_gemm_tile<T, CH, true>(yf, w.w_z, nt);
+  for (int nt = 0; nt < NTB; ++nt) {
+    const f32x16 acc = row_gemm_tile<T, CH, true>(yf, w.w_z, nt0 + nt);
     if (valid) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int c0 = nt * 32 + 8 * g + 4 * half;
+        const int c0 = (nt0 + nt) * 32 + 8 * g + 4 * half;
         float o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = (acc[4 * g + r] + w.b_z[c0 + r]) * gate[nt][4 * g + r];
@@ -1300,6 +1318,16 @@ constexpr bool trimul_fast() {
 // Prologue over plane rows r0 .. r0 + nrows - 1 (default: all Np rows) for
 // sides side_lo .. side_hi - 1 (0: A, 1: Bm), into planes of stride ps
 // (default: the unpadded nrows * Np).
+// Parts that a row tile's `units` independent pieces are dealt to: as many as
+// keep the launch within `per_cu` waves a CU, at most one a unit.  Beyond that
+// the LayerNorm that each part repeats costs more than its waves give.  fp32,
+// times of the kernel unsplit / split: prologue (24 a CU) 63 / 17 us at N = 64,
+// 99 / 69 at 160, 101 / 103 at 256; epilogue (8 a CU, all or nothing) 32 / 18
+// at N = 64, 35 / 42 at 160, where it is not split any more.
+static int units_split(int64_t tiles, int units, int per_cu) {
+  return (int)std::min<int64_t>(units, std::max<int64_t>(1, per_cu * (int64_t)device_cus() / std::max<int64_t>(tiles, 1)));
+}
+
 template <typename T, int CZ, int CH>
 static int launch_trimul_prologue(const void* z, const float* mask, const TriMulPacked<T>& w, T* pa,
                                   T* pb, int64_t B, int64_t N, int Np, int outgoing, float eps_in,
@@ -1329,9 +1357,13 @@ static int launch_trimul_prologue(const void* z, const float* mask, const TriMul
     }
   } else {
     StageTimer timer("trimul_prologue", st);
-    trimul_prologue_kernel<T, CZ, CH><<<(unsigned)((ptiles + 3) / 4), 256, 0, st>>>(
-        (const T*)z, mask, pa, pb, w, (int)B, (int)N, Np, outgoing, eps_in, r0, nrows, side_lo,
-        side_hi, ps);
+    const int parts = units_split(ptiles, (side_hi - side_lo) * (CH / 32), 24);
+    auto go = [&](auto kern) {
+      kern<<<dim3((unsigned)((ptiles + 3) / 4), parts), 256, 0, st>>>((const T*)z, mask, pa, pb, w, (int)B, (int)N, Np,
+                                                                      outgoing, eps_in, r0, nrows, side_lo, side_hi, ps);
+    };
+    if (parts > 1) go(trimul_prologue_kernel<T, CZ, CH, true>);
+    else go(trimul_prologue_kernel<T, CZ, CH, false>);
   }
   GTK_LAUNCH_CHECK();
   return GTK_OK;
@@ -1356,9 +1388,13 @@ static int launch_trimul_epilogue(const void* z, const T* px, void* out, const T
                                etiles, r0, nrows, xrows, ps_x);
   } else {
     StageTimer timer("trimul_epilogue", st);
-    trimul_epilogue_kernel<T, CZ, CH><<<(unsigned)((etiles + 3) / 4), 256, 0, st>>>(
-        (const T*)z, px, (T*)out, w, (int)B, (int)N, Np, residual, eps_in, eps_out, r0, nrows,
-        xrows, ps_x);
+    auto go = [&](auto kern, int parts) {
+      kern<<<dim3((unsigned)((etiles + 3) / 4), parts), 256, 0, st>>>((const T*)z, px, (T*)out, w, (int)B, (int)N, Np,
+                                                                      residual, eps_in, eps_out, r0, nrows, xrows, ps_x);
+    };
+    constexpr int NT = CZ / 32;
+    if (NT > 1 && units_split(etiles, NT, 8) == NT) go(trimul_epilogue_kernel<T, CZ, CH, 1>, NT);
+    else go(trimul_epilogue_kernel<T, CZ, CH, NT>, 1);
   }
   GTK_LAUNCH_CHECK();
   return GTK_OK;
