@@ -167,8 +167,12 @@ static AttnWs<T> carve_attn_ws(Carve& cv, int64_t B, int64_t Np, int H, int ch, 
 //    mode bit 0: q, k, v^T and the gate (into the workspace rows of ws), bit
 //    1: the triangle bias (every row of it is read by every row's attention,
 //    so row chunks compute it over all rows first).
+//    SPLIT: the pieces of a tile (q, k and v of a head, the gate of a head, the
+//    bias) are dealt over gridDim.y waves, each of which normalises the tile
+//    again, where the tiles alone leave the chip without waves (fewer than 8 a
+//    CU; fp32, N = 128: 80 -> 51 us).
 // ---------------------------------------------------------------------------
-template <typename T, int CIN, int H>
+template <typename T, int CIN, int H, bool SPLIT>
 __global__ __launch_bounds__(256) void triattn_prologue_kernel(const T* __restrict__ x,
                                                                TriAttnPacked<T> w, AttnWs<T> ws,
                                                                int B, int N, int Np, int starting,
@@ -196,9 +200,9 @@ __global__ __launch_bounds__(256) void triattn_prologue_kernel(const T* __restri
   const float keep = valid ? 1.f : 0.f;
 
   const int64_t rowbase = ws.row(b, r);  // (b, r) in the workspace rows
-#pragma unroll 1
-  for (int h = 0; h < ((mode & 1) ? H : 0); ++h) {
-    // q, k: [b][r][h][j][d], lane holds d = 8g + 4*half + rr -> 4 consecutive d
+  // q, k: [b][r][h][j][d], lane holds d = 8g + 4*half + rr -> 4 consecutive d;
+  // v^T: [b][r][h][d][vt_pos(j)] (one unit: three independent product chains)
+  auto qkv = [&](int h) {
     const f32x16 aq = row_gemm_tile<T, CIN, true>(xf, w.w_q, h);
     const f32x16 ak = row_gemm_tile<T, CIN, true>(xf, w.w_k, h);
     const f32x16 av = row_gemm_tile<T, CIN, true>(xf, w.w_v, h);
@@ -218,11 +222,10 @@ __global__ __launch_bounds__(256) void triattn_prologue_kernel(const T* __restri
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) vd[(int64_t)(d0 + rr) * Np] = cvt<T>((av[4 * g + rr] + bv[rr]) * keep);
     }
-  }
+  };
   // gate: [b][r][j][CH]
-  T* gd = ws.gate + (rowbase * Np + j) * CH;
-#pragma unroll 1
-  for (int nt = 0; nt < ((mode & 1) ? CH / 32 : 0); ++nt) {
+  auto gate = [&](int nt) {
+    T* gd = ws.gate + (rowbase * Np + j) * CH;
     const f32x16 ag = row_gemm_tile<T, CIN, true>(xf, w.w_g, nt);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -230,24 +233,35 @@ __global__ __launch_bounds__(256) void triattn_prologue_kernel(const T* __restri
       store4(gd + c0, gate_from_u(ag[4 * g] + w.b_g[c0]), gate_from_u(ag[4 * g + 1] + w.b_g[c0 + 1]),
              gate_from_u(ag[4 * g + 2] + w.b_g[c0 + 2]), gate_from_u(ag[4 * g + 3] + w.b_g[c0 + 3]));
     }
-  }
+  };
   // triangle bias: [b][h][r][j] (rows h >= H of the packed tile are zero)
-  if (mode & 2) {
+  auto bias = [&]() {
     const f32x16 ab = row_gemm_tile<T, CIN, true>(xf, w.w_b, 0);
     if (half == 0) {
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr)
         if (rr < H) ws.bias[(((int64_t)b * H + rr) * Np + r) * Np + j] = cvt<T>((ab[rr] + w.b_b[rr]) * keep);
     }
-    if (H > 4) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int h = 8 * g + 4 * half + rr;
-          if (h >= 4 && h < H) ws.bias[(((int64_t)b * H + h) * Np + r) * Np + j] = cvt<T>((ab[4 * g + rr] + w.b_b[h]) * keep);
-        }
+  };
+  static_assert(H <= 4, "the bias of a tile sits in four registers");
+  if constexpr (SPLIT) {
+#pragma unroll 1
+    for (int u = blockIdx.y; u < 2 * H + 1; u += gridDim.y) {
+      if (u == 2 * H) {
+        if (mode & 2) bias();
+      } else if (mode & 1) {
+        if (u < H) qkv(u);
+        else gate(u - H);
+      }
     }
+  } else {
+    if (mode & 1) {
+#pragma unroll 1
+      for (int h = 0; h < H; ++h) qkv(h);
+#pragma unroll 1
+      for (int nt = 0; nt < CH / 32; ++nt) gate(nt);
+    }
+    if (mode & 2) bias();
   }
 }
 
@@ -1576,8 +1590,13 @@ static int fwd_triattn(const void* x, const float* mask, void* out, const void* 
     auto prologue = [&](int r0, int nrows, int mode) {
       const int64_t ptiles = B * (int64_t)nrows * (Np / 32);
       StageTimer timer("triattn_prologue", st);
-      triattn_prologue_kernel<T, CIN, H><<<(unsigned)((ptiles + 3) / 4), 256, 0, st>>>(
-          (const T*)x, w, a, (int)B, (int)N, Np, starting, eps, r0, nrows, mode);
+      const int parts = (int)std::min<int64_t>(2 * H + 1, std::max<int64_t>(1, 8 * (int64_t)device_cus() / ptiles));
+      auto go = [&](auto kern) {
+        kern<<<dim3((unsigned)((ptiles + 3) / 4), parts), 256, 0, st>>>((const T*)x, w, a, (int)B, (int)N, Np,
+                                                                        starting, eps, r0, nrows, mode);
+      };
+      if (parts > 1) go(triattn_prologue_kernel<T, CIN, H, true>);
+      else go(triattn_prologue_kernel<T, CIN, H, false>);
     };
     auto attend = [&](int r0, int nrows) {
       const int64_t ablocks = B * nrows * ((N + 31) / 32);

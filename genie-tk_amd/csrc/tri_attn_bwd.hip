@@ -61,7 +61,7 @@ template <typename T> struct AttnBwdBufs {
   float* kmask;                    // [B][N][np]: 1 valid key, 0 masked
   float *mrow, *linv, *dd;         // [B][N][H][np]
   float* db;                       // dL/dbias [B][H][N][N]
-  float* dbp;                      // dL/dbias partial sums per row chunk (bf16 path, np <= 512)
+  float* dbp;                      // dL/dbias partial sums per row chunk
   T *cm_stack, *cm_xh, *cm_dxn, *cm_dy, *cm_go, *cm_dtri;
   int64_t pitch;
 };
@@ -121,8 +121,13 @@ __host__ __device__ __forceinline__ int64_t bias_frag_elem(int h, int a, int k, 
 
 // ---------------------------------------------------------------------------
 // proj: one 32-position tile of one attention row per wave
+//
+// SPLIT: the 4 H + 1 projections of a tile (q, k, v and gate of each head, the
+// bias) are dealt over gridDim.y waves, each of which normalises the tile
+// again, where the tiles alone leave the chip without waves (attn_parts; N =
+// 128 in fp32: 103 -> 56 us).
 // ---------------------------------------------------------------------------
-template <typename T, int C, int H>
+template <typename T, int C, int H, bool SPLIT>
 __global__ __launch_bounds__(256) void attn_bwd_proj_kernel(const T* __restrict__ x,
                                                             const float* __restrict__ mask,
                                                             AttnBwdW<T> w, AttnBwdBufs<T> bf,
@@ -150,30 +155,25 @@ __global__ __launch_bounds__(256) void attn_bwd_proj_kernel(const T* __restrict_
   const float* bk[3] = {w.b_q, w.b_k, w.b_v};
   T* dr[3] = {bf.qr, bf.kr, bf.vr};
   T* dt[3] = {bf.qt, bf.kt, bf.vt};
-#pragma unroll 1
-  for (int kind = 0; kind < 3; ++kind) {
-#pragma unroll 1
-    for (int h = 0; h < H; ++h) {
-      const f32x16 acc = row_gemm_tile<T, C, true>(xf, wk[kind], h);
-      const int64_t rh_ = ((int64_t)b * N + r) * H + h;
-      T* rowm = dr[kind] + (rh_ * np + j) * AD;
-      T* dmaj = dt[kind] + rh_ * AD * np + j;
+  auto qkv = [&](int kind, int h) {
+    const f32x16 acc = row_gemm_tile<T, C, true>(xf, wk[kind], h);
+    const int64_t rh_ = ((int64_t)b * N + r) * H + h;
+    T* rowm = dr[kind] + (rh_ * np + j) * AD;
+    T* dmaj = dt[kind] + rh_ * AD * np + j;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d0 = 8 * g + 4 * half;
-        float v[4];
+    for (int g = 0; g < 4; ++g) {
+      const int d0 = 8 * g + 4 * half;
+      float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = valid ? acc[4 * g + q] + bk[kind][h * AD + d0 + q] : 0.f;
-        store4(rowm + d0, v[0], v[1], v[2], v[3]);
-        if (dmajor) {
+      for (int q = 0; q < 4; ++q) v[q] = valid ? acc[4 * g + q] + bk[kind][h * AD + d0 + q] : 0.f;
+      store4(rowm + d0, v[0], v[1], v[2], v[3]);
+      if (dmajor) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) dmaj[(int64_t)(d0 + q) * np] = cvt<T>(v[q]);
-        }
+        for (int q = 0; q < 4; ++q) dmaj[(int64_t)(d0 + q) * np] = cvt<T>(v[q]);
       }
     }
-  }
-#pragma unroll 1
-  for (int h = 0; h < H; ++h) {
+  };
+  auto gate = [&](int h) {
     const f32x16 acc = row_gemm_tile<T, C, true>(xf, w.w_g, h);
     T* gp = bf.gt + (((int64_t)b * N + r) * np + j) * CH + h * AD;
 #pragma unroll
@@ -184,8 +184,8 @@ __global__ __launch_bounds__(256) void attn_bwd_proj_kernel(const T* __restrict_
       for (int q = 0; q < 4; ++q) v[q] = sigmoidf_(acc[4 * g + q] + w.b_g[h * AD + d0 + q]);
       store4(gp + d0, v[0], v[1], v[2], v[3]);
     }
-  }
-  {
+  };
+  auto bias = [&]() {
     // triangle bias: outputs 0..H-1 sit in lanes of half 0, acc[0..H-1]
     const f32x16 acc = row_gemm_tile<T, C, true>(xf, w.w_b, 0);
     if (valid && half == 0) {
@@ -200,10 +200,32 @@ __global__ __launch_bounds__(256) void attn_bwd_proj_kernel(const T* __restrict_
         bS[bias_frag_elem(h, j, r, np)] = bs;
       }
     }
+    // 1 for a valid key (mask == 1: no bias); 0 for a masked key, whose bias
+    // 1e9 * (mask - 1) <= -60 takes it out of any row with a valid key
+    if (half == 0) bf.kmask[((int64_t)b * N + r) * np + j] = valid && (!mask || mask[xp] == 1.f) ? 1.f : 0.f;
+  };
+  if constexpr (SPLIT) {
+#pragma unroll 1
+    for (int u = blockIdx.y; u < 4 * H + 1; u += gridDim.y) {
+      if (u < 3 * H) qkv(u / H, u % H);
+      else if (u < 4 * H) gate(u - 3 * H);
+      else bias();
+    }
+  } else {
+#pragma unroll 1
+    for (int kind = 0; kind < 3; ++kind)
+#pragma unroll 1
+      for (int h = 0; h < H; ++h) qkv(kind, h);
+#pragma unroll 1
+    for (int h = 0; h < H; ++h) gate(h);
+    bias();
   }
-  // 1 for a valid key (mask == 1: no bias); 0 for a masked key, whose bias
-  // 1e9 * (mask - 1) <= -60 takes it out of any row with a valid key
-  if (half == 0) bf.kmask[((int64_t)b * N + r) * np + j] = valid && (!mask || mask[xp] == 1.f) ? 1.f : 0.f;
+}
+
+// Parts that a row tile's `units` independent pieces are dealt to: within
+// `per_cu` waves a CU, at most one part a unit.
+inline int attn_parts(int64_t tiles, int units, int per_cu) {
+  return (int)std::min<int64_t>(units, std::max<int64_t>(1, per_cu * (int64_t)device_cus() / std::max<int64_t>(tiles, 1)));
 }
 
 // ---------------------------------------------------------------------------
@@ -428,7 +450,9 @@ __device__ __forceinline__ void store_row32_bf16(bf16* row, const float* v) {
   }
 }
 
-template <typename T, int C, int H>
+// SPLIT: one head per wave (blockIdx.y), where the tiles alone leave the chip
+// without waves (N = 128 in fp32: 33 -> 26 us).
+template <typename T, int C, int H, bool SPLIT>
 __global__ __launch_bounds__(256) void attn_bwd_epi_kernel(const T* __restrict__ dy, AttnBwdW<T> w,
                                                            AttnBwdBufs<T> bf, int B, int N, int np,
                                                            int starting, int dmajor) {
@@ -453,7 +477,9 @@ __global__ __launch_bounds__(256) void attn_bwd_epi_kernel(const T* __restrict__
   Frag<T> fdy[C / 16];
 #pragma unroll
   for (int ch = 0; ch < C / 16; ++ch) fdy[ch].set(&dh.v[ch * 8]);
-  if constexpr (std::is_same<T, bf16>::value && C == 128) {
+  if (SPLIT && blockIdx.y != 0) {
+    // dy goes out once
+  } else if constexpr (std::is_same<T, bf16>::value && C == 128) {
     const CmTileRH cmr;  // whole transposed tiles of the lane's row half
     cmr.store(bf.cm_dy, pitch, p0, dh.v, fast, valid);
   } else if (valid) {
@@ -463,7 +489,7 @@ __global__ __launch_bounds__(256) void attn_bwd_epi_kernel(const T* __restrict__
   T* cm_dg = bf.cm_stack + (int64_t)3 * CH * pitch;
   const CmTile cmt;
 #pragma unroll 1
-  for (int h = 0; h < H; ++h) {
+  for (int h = SPLIT ? blockIdx.y : 0; h < (SPLIT ? (int)blockIdx.y + 1 : H); ++h) {
     const f32x16 dog = row_gemm_tile<T, C, true>(fdy, w.wt_o, h);
     const int64_t rh = ((int64_t)b * N + r) * H + h;
     const T* O = bf.o + (rh * np + j) * AD;
@@ -635,10 +661,30 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_kernel(AttnBwdBufs<T> bf, int
 
 // ---------------------------------------------------------------------------
 // dbias: per (batch, head, 32 queries, 32 keys), summed over the rows; lane = query
+//
+// The B H (np/32)^2 tiles are few (64 at N = 128) and each sums over all N rows,
+// so the rows are dealt to gridDim.y chunks, whose sums go to `dst` one after the
+// other ([chunk][B][H][N][N]) and are added by attn_bwd_dbias_sum_kernel.  N =
+// 128 in fp32: 345 us with one chunk, 40 with 32 (4096 waves' worth; chunks of
+// fewer than 4 rows would write more than they read).
 // ---------------------------------------------------------------------------
+constexpr int kDbWaves = 4096;
+inline int dbias_row_chunks(int64_t B, int64_t N, int H) {
+  const int64_t t1 = (N + 31) / 32, tiles = B * H * t1 * t1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>((N + 3) / 4, kDbWaves / std::max<int64_t>(tiles, 1)));
+}
+static __global__ void attn_bwd_dbias_sum_kernel(const float* __restrict__ part, float* __restrict__ db, int64_t n,
+                                                 int nch) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  float a = 0.f;
+#pragma unroll 4
+  for (int c = 0; c < nch; ++c) a += part[c * n + i];
+  db[i] = a;
+}
 template <typename T, int H>
-__global__ __launch_bounds__(256) void attn_bwd_dbias_kernel(AttnBwdBufs<T> bf, int B, int N, int np,
-                                                             float scale) {
+__global__ __launch_bounds__(256) void attn_bwd_dbias_kernel(AttnBwdBufs<T> bf, float* __restrict__ dst_all,
+                                                             int B, int N, int np, float scale) {
   const int lane = threadIdx.x & 63, half = lane >> 5, t32 = lane & 31;
   const int t1 = np / 32;
   const int64_t tile = (int64_t)blockIdx.x * 4 + wave_id();
@@ -660,7 +706,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dbias_kernel(AttnBwdBufs<T> bf, 
   float acc[16];
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-  for (int r = 0; r < N; ++r) {
+  const int rpc = (N + gridDim.y - 1) / gridDim.y;
+  const int r_end = min(N, (int)(blockIdx.y + 1) * rpc);
+  for (int r = blockIdx.y * rpc; r < r_end; ++r) {
     const int64_t br = (int64_t)b * N + r;
     const int64_t rh = br * H + h;
     const f32x16 sa = qk_tile<T>(bf.kr + (rh * np + (int64_t)kt * 32) * AD,
@@ -684,7 +732,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dbias_kernel(AttnBwdBufs<T> bf, 
     }
   }
   if (q >= N) return;
-  float* dst = bf.db + (((int64_t)b * H + h) * N + q) * N;
+  float* dst = dst_all + ((((int64_t)blockIdx.y * B + b) * H + h) * N + q) * N;
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -1850,7 +1898,9 @@ static AttnBwdWs<T> carve_attn_bwd(Carve& cv, int64_t B, int64_t N, int C, int H
   b.linv = cv.take<float>(B * N * H * np);
   b.dd = cv.take<float>(B * N * H * np);
   b.db = cv.take<float>(B * H * N * N);
-  b.dbp = (sizeof(T) == 2 && np <= 512) ? cv.take<float>(B * kDbChunks * H * np * np) : nullptr;
+  const int nch = dbias_row_chunks(B, N, H);
+  b.dbp = (sizeof(T) == 2 && np <= 512) ? cv.take<float>(B * kDbChunks * H * np * np)
+                                        : cv.take<float>(nch > 1 ? nch * B * H * N * N : 0);
   b.pitch = round_up(B * N * N, 64);
   // operands of the weight-gradient products: rows padded to their tiles
   b.cm_stack = cv.take<T>((int64_t)wgrad_rows(4 * CH) * b.pitch);
@@ -1930,9 +1980,15 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
                                                                   np, starting, eps, 1.0f / scale, rowtiles);
       }
     }
-    if (!std::is_same<T, bf16>::value || dmajor)
-      attn_bwd_proj_kernel<T, C, H><<<g4(rowtiles), 256, 0, st>>>(
-          (const T*)x, mask, a.w, a.b, (int)B, (int)N, np, starting, eps, 1.0f / scale, dmajor);
+    if (!std::is_same<T, bf16>::value || dmajor) {
+      const int parts = attn_parts(rowtiles, 4 * H + 1, 24);
+      auto go = [&](auto kern) {
+        kern<<<dim3(g4(rowtiles), parts), 256, 0, st>>>((const T*)x, mask, a.w, a.b, (int)B, (int)N, np, starting,
+                                                        eps, 1.0f / scale, dmajor);
+      };
+      if (parts > 1) go(attn_bwd_proj_kernel<T, C, H, true>);
+      else go(attn_bwd_proj_kernel<T, C, H, false>);
+    }
     GTK_LAUNCH_CHECK();
   }
   const int64_t rblocks = B * N * H;
@@ -1963,8 +2019,13 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
   }
   {
     StageTimer timer("triattn_bwd_epi", st);
-    attn_bwd_epi_kernel<T, C, H><<<g4(rowtiles), 256, 0, st>>>((const T*)dy, a.w, a.b, (int)B,
-                                                                (int)N, np, starting, dmajor);
+    const bool split = attn_parts(rowtiles, H, 8) == H;
+    auto go = [&](auto kern) {
+      kern<<<dim3(g4(rowtiles), split ? H : 1), 256, 0, st>>>((const T*)dy, a.w, a.b, (int)B, (int)N, np, starting,
+                                                             dmajor);
+    };
+    if (split) go(attn_bwd_epi_kernel<T, C, H, true>);
+    else go(attn_bwd_epi_kernel<T, C, H, false>);
     GTK_LAUNCH_CHECK();
   }
   bool rh_done = false;
@@ -1997,7 +2058,7 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
   }
   {
     StageTimer timer("triattn_bwd_dbias", st);
-    if (a.b.dbp) {
+    if (std::is_same<T, bf16>::value && np <= 512) {
       if constexpr (std::is_same<T, bf16>::value) {
         // row chunks of rpc rows (at most kDbChunks per batch element), partial
         // sums in fragment order, then the sum over the chunks
@@ -2016,7 +2077,14 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
         attn_bwd_dbias_reduce_kernel<<<(unsigned)rtiles, 256, 0, st>>>(a.b.dbp, a.b.db, (int)B, (int)N, np, nch);
       }
     } else {
-      attn_bwd_dbias_kernel<T, H><<<g4(pairtiles), 256, 0, st>>>(a.b, (int)B, (int)N, np, scale);
+      const int nch = dbias_row_chunks(B, N, H);
+      attn_bwd_dbias_kernel<T, H><<<dim3(g4(pairtiles), nch), 256, 0, st>>>(a.b, nch > 1 ? a.b.dbp : a.b.db, (int)B,
+                                                                            (int)N, np, scale);
+      if (nch > 1) {
+        GTK_LAUNCH_CHECK();
+        const int64_t n = B * H * N * N;
+        attn_bwd_dbias_sum_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(a.b.dbp, a.b.db, n, nch);
+      }
     }
     GTK_LAUNCH_CHECK();
   }
