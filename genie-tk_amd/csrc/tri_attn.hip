@@ -55,9 +55,14 @@ template <typename T> struct TriAttnPacked {
   float *ln_w, *ln_b;
 };
 
+// Head width in the packed weights: HD, or 8 for the narrow fp32 path.
+template <typename T> static int attn_head_pad(int64_t ch, int64_t H) {
+  return sizeof(T) == 4 && H == 4 && ch <= 8 * H ? 8 : HD;
+}
+
 template <typename T>
-static TriAttnPacked<T> carve_triattn(Carve& cv, int cin, int /*ch*/, int H) {
-  const int ch = H * HD;  // padded heads
+static TriAttnPacked<T> carve_triattn(Carve& cv, int cin, int c_h, int H) {
+  const int ch = H * attn_head_pad<T>(c_h, H);  // padded heads
   TriAttnPacked<T> p;
   p.w_q = cv.take<T>(packed_elems(ch, cin));
   p.w_k = cv.take<T>(packed_elems(ch, cin));
@@ -1353,6 +1358,292 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
 }
 
 // ---------------------------------------------------------------------------
+// Narrow heads in fp32 (four heads of d <= 8: the reference layer's default).
+//
+// Padded to 32 channels a head, the default attention computed four times the
+// projections, eight times the score products and four times the P V products
+// it needs.  Here a head is 8 channels, so the four heads of q, k, v or the gate
+// are one 32-channel tile:
+//   q, k  [row][H][Np][8], the even channels of a position before the odd ones,
+//         so that a lane's 16 bytes are the operands of four 32x32x2 products
+//         (step e takes channels 2e and 2e + 1 from the two half-waves);
+//   v     [row][H][8 d][Np], 16-byte chunk c of row d at chunk c ^ d (the eight
+//         rows of a chunk then sit in distinct LDS banks);
+//   gate  [row][Np][32];
+//   bias  [B][H] in fp32 tiles of 32 x 32 in S^T accumulator order, 4 KiB each
+//         (attn8_bias_off).
+// ---------------------------------------------------------------------------
+struct Attn8Ws {
+  float *q, *k, *v, *gate, *bias;
+  int64_t rows;  // workspace rows per batch element, from row r0 on (see AttnWs)
+  int r0;
+  __host__ __device__ int64_t row(int b, int r) const { return (int64_t)b * rows + (r - r0); }
+};
+static Attn8Ws carve_attn8_ws(Carve& cv, int64_t B, int64_t Np, int64_t rows) {
+  Attn8Ws w;
+  w.rows = rows > 0 ? rows : Np;
+  w.r0 = 0;
+  float** t[] = {&w.q, &w.k, &w.v, &w.gate};
+  for (float** p : t) *p = cv.take<float>(B * w.rows * Np * 32);
+  w.bias = cv.take<float>(B * 4 * Np * Np);
+  return w;
+}
+// Element (h, query q, key k): tile (q/32, k/32), register 4g + rr of lane 32 hh
+// + q % 32 holds key 8g + 4 hh + rr of the tile.
+__host__ __device__ __forceinline__ int64_t attn8_bias_off(int h, int q, int k, int Np) {
+  const int nt = Np / 32;
+  const int64_t tile = ((int64_t)h * nt + (q >> 5)) * nt + (k >> 5);
+  return (((tile * 4 + ((k & 31) >> 3)) * 64 + ((k >> 2) & 1) * 32 + (q & 31)) << 2) + (k & 3);
+}
+
+// Prologue: one wave per tile of 32 positions of a row (rows r0 .. r0 + nrows -
+// 1, vtiles tiles each); mode bit 0: q, k, v and the gate, bit 1: the bias.  The
+// five projections are dealt over gridDim.y waves (1 or 5), each of which
+// normalises the tile again.
+template <int CIN>
+__global__ __launch_bounds__(256) void attn8_prologue_kernel(const float* __restrict__ x, TriAttnPacked<float> w,
+                                                             Attn8Ws ws, int B, int N, int Np, int starting,
+                                                             float eps, int r0, int nrows, int vtiles, int mode) {
+  const int lane = threadIdx.x & 63;
+  const int half = lane >> 5;
+  const int t32 = lane & 31;
+  const int64_t tile = (int64_t)blockIdx.x * 4 + wave_id();
+  if (tile >= (int64_t)B * nrows * vtiles) return;
+  const int vt = (int)(tile % vtiles);
+  const int r = r0 + (int)((tile / vtiles) % nrows);  // destination row
+  const int b = (int)(tile / ((int64_t)vtiles * nrows));
+  const int j = vt * 32 + t32;                // destination position
+  const bool valid = r < N && j < N;
+  const int p = starting ? r : j, q = starting ? j : r;  // source pair
+  const int64_t pair = ((int64_t)b * N + (valid ? p : 0)) * N + (valid ? q : 0);
+  RowHalf<CIN> rh;
+  load_row_half<float, CIN>(rh, x + pair * CIN, valid);
+  const f32x2 st = row_stats<CIN>(rh, eps);
+  Frag<float> xf[CIN / 16];
+  ln_to_frags<float, CIN>(xf, rh, st);
+  const float keep = valid ? 1.f : 0.f;
+  const int64_t rowbase = ws.row(b, r);
+  // accumulator register 4h + rr: channel 4 * half + rr of head h, position j
+#pragma unroll 1
+  for (int u = blockIdx.y; u < 5; u += gridDim.y) {
+    if (!(mode & (u == 4 ? 2 : 1))) continue;
+    const f32x16 a = row_gemm_tile<float, CIN, true>(
+        xf, u == 0 ? w.w_q : u == 1 ? w.w_k : u == 2 ? w.w_v : u == 3 ? w.w_g : w.w_b, 0);
+    if (u == 4) {  // rows h >= 4 of the packed tile are zero
+      if (half == 0) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          ws.bias[(int64_t)b * 4 * Np * Np + attn8_bias_off(h, r, j, Np)] = (a[h] + w.b_b[h]) * keep;
+      }
+      continue;
+    }
+    const float* bias = (u == 0 ? w.b_q : u == 1 ? w.b_k : u == 2 ? w.b_v : w.b_g) + 4 * half;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      float v[4];
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) v[rr] = a[4 * h + rr] + bias[8 * h + rr];
+      if (u == 3) {
+        store4(ws.gate + (rowbase * Np + j) * 32 + 8 * h + 4 * half, gate_from_u(v[0]), gate_from_u(v[1]),
+               gate_from_u(v[2]), gate_from_u(v[3]));
+      } else if (u == 2) {
+        float* vd = ws.v + (rowbase * 4 + h) * 8 * (int64_t)Np;
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+          const int d = 4 * half + rr;
+          vd[(int64_t)d * Np + (((j >> 2) ^ d) << 2) + (j & 3)] = v[rr] * keep;
+        }
+      } else {
+        float* pd = (u == 0 ? ws.q : ws.k) + ((rowbase * 4 + h) * Np + j) * 8 + 2 * half;
+        *reinterpret_cast<f32x2*>(pd) = f32x2{v[0] * keep, v[2] * keep};
+        *reinterpret_cast<f32x2*>(pd + 4) = f32x2{v[1] * keep, v[3] * keep};
+      }
+    }
+  }
+}
+
+// Attention and output projection: a block is one row and up to blockDim/64
+// query tiles of it, one a wave; a wave attends its 32 queries in all four heads
+// and projects them, so heads never meet in LDS.  The keys of the row pass
+// through LDS in segments of KS positions (k and v of the four heads, 256 KS
+// bytes), read by every wave.
+//   S^T = bias + K Q^T: four 32x32x2 products a 32-key tile (lane = query, 16
+//   keys a half-wave).  Online softmax whose reference maximum moves only when a
+//   tile exceeds it by more than 8 (log2 units).  O^T += V^T P^T with the
+//   16-block 4x4x1 product, one key a step: block 4 * half-row of channels x 4
+//   queries, so 8 channels cost 8 passes of 8 cycles where a 32-row product
+//   would spend 64; the half-waves' P meet by v_permlane32_swap.  The 8 output
+//   channels a half-wave holds are the operand of the projection as they are.
+// N = 256, c_in = 128: 60 us (and 44 for the prologue); with heads padded to 32
+// and one wave per head and query tile reading K, V, the mask and a row-major bias
+// from L2 these took 240 and 114 us.
+template <int CIN, int KS>
+__global__ __launch_bounds__(512) void attn8_flash_kernel(const float* __restrict__ x, const float* __restrict__ mask,
+                                                          float* __restrict__ out, TriAttnPacked<float> w, Attn8Ws ws,
+                                                          int N, int Np, int starting, int residual, int r0, int nrows,
+                                                          float inf, int qgroups) {
+  constexpr int H = 4;
+  constexpr float kRescale = 8.0f;
+  __shared__ __attribute__((aligned(1024))) float ks[H][KS * 8];
+  __shared__ __attribute__((aligned(1024))) float vs[H][8 * KS];
+  __shared__ __attribute__((aligned(16))) float kb[KS];  // what a key's scores take: 0, its mask bias, -inf past N
+  __shared__ int dirty[KS / 64];                         // bits 0, 1: some kb of the two tiles of 64 keys is not 0
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();
+  const int nwaves = blockDim.x >> 6;
+  const int half = lane >> 5;
+  const int t32 = lane & 31;
+  const int nq = (N + 31) / 32;
+  const int nt = Np / 32;
+  const int lin = (int)xcd_remap_any(blockIdx.x, gridDim.x);
+  const int qg = lin % qgroups, br = lin / qgroups;
+  const int b = br / nrows;
+  const int r = r0 + (br - b * nrows);
+  const int64_t rowbase = ws.row(b, r);
+  const int qt = qg * nwaves + wave;
+  const bool active = qt < nq;
+  const float* mrow = mask ? mask + (int64_t)b * N * N + (starting ? (int64_t)r * N : r) : nullptr;
+  const int64_t mks = starting ? 1 : N;
+  const int q = (active ? qt : 0) * 32 + t32;
+
+  f32x4 qf[H], o0[H], o1[H];
+  float m_ref[H], l_run[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    qf[h] = load4f(ws.q + ((rowbase * H + h) * Np + q) * 8 + 4 * half);
+    o0[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    o1[h] = o0[h];
+    m_ref[h] = -INFINITY;
+    l_run[h] = 0.f;
+  }
+  for (int k0 = 0; k0 < N; k0 += KS) {
+    const int kn = min(KS, Np - k0);  // positions of the segment (a multiple of 64)
+    if (k0 > 0) __syncthreads();      // the segment before is read by every wave
+    // k: kn * 8 floats a head, contiguous; v: 8 rows of kn floats a head
+    for (int c = threadIdx.x; c < H * 2 * kn; c += blockDim.x) {
+      const int h = c / (2 * kn), i = c - h * 2 * kn;
+      *reinterpret_cast<f32x4*>(&ks[h][i * 4]) = load4f(ws.k + ((rowbase * H + h) * Np + k0) * 8 + i * 4);
+      const int d = i / (kn / 4), cc = i - d * (kn / 4);
+      *reinterpret_cast<f32x4*>(&vs[h][d * KS + cc * 4]) =
+          load4f(ws.v + ((rowbase * H + h) * 8 + d) * (int64_t)Np + k0 + cc * 4);
+    }
+    for (int i = wave * 64; i < kn; i += nwaves * 64) {
+      const int k = k0 + i + lane;
+      const float mval = mrow && k < N ? mrow[k * mks] : 1.f;
+      const float add = k >= N ? -INFINITY : mval != 1.f ? (inf * (mval - 1.f)) * kLog2e : 0.f;
+      kb[i + lane] = add;
+      const unsigned long long bits = __ballot(add != 0.f);
+      if (lane == 0) dirty[i / 64] = ((uint32_t)bits != 0u ? 1 : 0) | ((bits >> 32) != 0ull ? 2 : 0);
+    }
+    __syncthreads();
+    if (!active) continue;
+    const int tn = min(kn / 32, nq - k0 / 32);  // key tiles of the segment with real keys
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const float* bh = ws.bias + (int64_t)b * H * Np * Np + (((int64_t)h * nt + qt) * nt + k0 / 32) * 1024 + lane * 4;
+      f32x4 bn[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) bn[g] = load4f(bh + g * 256);
+      const float* vlane = vs[h] + (4 * half + (lane & 3)) * KS;
+      const int vx = 4 * half + (lane & 3);  // chunk swizzle of this lane's row
+      for (int t = 0; t < tn; ++t) {
+        f32x16 s;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) s[4 * g + rr] = bn[g][rr];
+        // the next tile's bias (the last one again)
+        const float* bt = bh + min(t + 1, tn - 1) * 1024;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) bn[g] = load4f(bt + g * 256);
+        const f32x4 kf = load4f(&ks[h][(t * 32 + t32) * 8 + 4 * half]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qf[h][e], s, 0, 0, 0);
+        if ((__builtin_amdgcn_readfirstlane(dirty[t >> 1]) >> (t & 1)) & 1) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 add = load4f(kb + t * 32 + 8 * g + 4 * half);
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) s[4 * g + rr] += add[rr];
+          }
+        }
+        float mt = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+        for (int e = 3; e < 15; e += 2) mt = fmaxf(fmaxf(mt, s[e]), s[e + 1]);
+        mt = lane_pair_max(fmaxf(mt, s[15]));
+        if (__ballot(mt > m_ref[h] + kRescale) != 0ull) {
+          const float m_new = fmaxf(m_ref[h], mt);
+          const float alpha = __builtin_amdgcn_exp2f(m_ref[h] - m_new);
+          l_run[h] *= alpha;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            o0[h][e] *= alpha;
+            o1[h][e] *= alpha;
+          }
+          m_ref[h] = m_new;
+        }
+        const float m_use = m_ref[h];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int c = t * 8 + 2 * g;
+          const f32x4 va = load4f(vlane + ((c ^ vx) << 2));
+          const f32x4 vb = load4f(vlane + (((c + 1) ^ vx) << 2));
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {
+            const float pv = __builtin_amdgcn_exp2f(s[4 * g + rr] - m_use);
+            l_run[h] += pv;
+            const uint32_t pu = __float_as_uint(pv);
+            const auto sw = __builtin_amdgcn_permlane32_swap(pu, pu, false, false);
+            o0[h] = __builtin_amdgcn_mfma_f32_4x4x1f32(va[rr], __uint_as_float(sw[0]), o0[h], 0, 0, 0);
+            o1[h] = __builtin_amdgcn_mfma_f32_4x4x1f32(vb[rr], __uint_as_float(sw[1]), o1[h], 0, 0, 0);
+          }
+        }
+      }
+    }
+  }
+  if (!active) return;
+  f32x4 og[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const float inv = 1.0f / lane_pair_sum(l_run[h]);
+    const f32x4 gv = load4f(ws.gate + (rowbase * Np + q) * 32 + 8 * h + 4 * half);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) og[h][e] = (o0[h][e] + o1[h][e]) * inv * gv[e];
+  }
+  const bool qvalid = q < N;
+  const int p0 = starting ? r : q, p1 = starting ? q : r;
+  const int64_t pair = ((int64_t)b * N + (qvalid ? p0 : 0)) * N + (qvalid ? p1 : 0);
+#pragma unroll
+  for (int ot = 0; ot < CIN / 32; ++ot) {
+    f32x16 acc = zero16();
+#pragma unroll
+    for (int ck = 0; ck < 2; ++ck) {
+      Frag<float> wf;
+      load_wfrag<float>(wf, w.w_o, ot, ck, 2);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wf.lo[e], og[2 * ck][e], acc, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wf.hi[e], og[2 * ck + 1][e], acc, 0, 0, 0);
+    }
+    if (qvalid) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int c0 = ot * 32 + 8 * g + 4 * half;
+        float v[4];
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) v[rr] = acc[4 * g + rr] + w.b_o[c0 + rr];
+        if (residual) {
+          const f32x4 xr = load4f(x + pair * CIN + c0);
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) v[rr] += xr[rr];
+        }
+        store4(out + pair * CIN + c0, v[0], v[1], v[2], v[3]);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // 3b. Raw attention op: relayout of q/k/v/bias, then flash per (row, head).
 // ---------------------------------------------------------------------------
 // src: [B][H][N][N][D]; element (b, h, a1, a2, d).  Destination row/position:
@@ -1483,9 +1774,10 @@ static int pack_triattn(const gtk_tri_attn_weights* w, int cin, int ch, int H, v
   TriAttnPacked<T> p = carve_triattn<T>(cv, cin, ch, H);
   const int wd = w->dtype;
   const int d = ch / H;           // channels of a head
-  const int chp = H * HD;         // padded to HD per head
+  const int hd = attn_head_pad<T>(ch, H);
+  const int chp = H * hd;         // padded to hd per head
   Pad heads;
-  heads.gp = HD;
+  heads.gp = hd;
   heads.g = d;
   const float qscale = kLog2e / sqrtf((float)d);
   int rc;
@@ -1505,7 +1797,14 @@ static int pack_triattn(const gtk_tri_attn_weights* w, int cin, int ch, int H, v
   }
   // output projection acts on the gated attention output (no LayerNorm);
   // its input channels are the padded heads
-  if ((rc = launch_pack<T>(p.w_o, w->o_w, wd, cin, chp, ch, 1, 1.f, st, nullptr, Pad(), heads))) return rc;
+  if (hd == HD) {
+    if ((rc = launch_pack<T>(p.w_o, w->o_w, wd, cin, chp, ch, 1, 1.f, st, nullptr, Pad(), heads))) return rc;
+  } else {
+    // in the order in which attn8_flash_kernel holds its output: lane half f,
+    // element e of chunk ks <-> channel 16 ks + 8 (e >> 2) + 4 f + (e & 3)
+    batch_wjob(*pack_batch(), sizeof(T) == 2, wd,
+               WJob{p.w_o, w->o_w, cin, chp, ch, 1, 1.f, nullptr, packed_elems(cin, chp), Pad(), heads, 1});
+  }
   if ((rc = launch_to_f32(p.b_o, w->o_b, wd, cin, 1.f, 0.f, st))) return rc;
   return batch.flush();
 }
@@ -1625,6 +1924,67 @@ static int fwd_triattn(const void* x, const float* mask, void* out, const void* 
   return GTK_OK;
 }
 
+// The narrow fp32 path (attn_head_pad): four heads of at most 8 channels.
+template <int CIN>
+static int fwd_attn8(const void* x, const float* mask, void* out, const void* packed, int64_t B, int64_t N,
+                     int64_t ch, int starting, int residual, float eps, float inf, int64_t chunk_rows, void* ws,
+                     hipStream_t st) {
+  Carve pc((void*)packed, SIZE_MAX);
+  const TriAttnPacked<float> w = carve_triattn<float>(pc, CIN, (int)ch, 4);
+  const int Np = (int)attn_pad(N);
+  const bool chunked = chunk_rows > 0 && chunk_rows < N;
+  Carve cv(ws, SIZE_MAX);
+  Attn8Ws a = carve_attn8_ws(cv, B, Np, chunked ? chunk_rows : 0);
+  const int nq = (int)((N + 31) / 32);
+  // position tiles that are read: those with a pair, up to the pairs of tiles
+  // (64 keys) that the attention copies; rows below N rounded up to a query tile
+  const int vtiles = (int)round_up(nq, 2);
+  auto prologue = [&](int r0, int nrows, int mode) {
+    const int64_t ptiles = B * (int64_t)nrows * vtiles;
+    const int parts = ptiles * 5 <= 24 * (int64_t)device_cus() ? 5 : 1;
+    StageTimer timer("triattn_prologue", st);
+    attn8_prologue_kernel<CIN><<<dim3((unsigned)((ptiles + 3) / 4), parts), 256, 0, st>>>(
+        (const float*)x, w, a, (int)B, (int)N, Np, starting, eps, r0, nrows, vtiles, mode);
+  };
+  auto attend = [&](int r0, int nrows) {
+    // waves a block: 8, or fewer where a block per row would leave CUs without one
+    const int64_t tiles = B * (int64_t)nrows * nq;
+    const int wpb = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(8, nq), tiles / device_cus()));
+    const int qgroups = (nq + wpb - 1) / wpb;
+    const int waves = (nq + qgroups - 1) / qgroups;  // evenly
+    const int64_t blocks = B * (int64_t)nrows * qgroups;
+    GTK_REQUIRE(blocks < (1ll << 31), GTK_EUNSUPPORTED, "attention grid too large");
+    StageTimer timer("triattn_flash", st);
+    auto go = [&](auto kern) {
+      kern<<<(unsigned)blocks, 64 * waves, 0, st>>>((const float*)x, mask, (float*)out, w, a, (int)N, Np, starting,
+                                                    residual, r0, nrows, inf, qgroups);
+    };
+    if (Np <= 128) go(attn8_flash_kernel<CIN, 128>);
+    else go(attn8_flash_kernel<CIN, 256>);
+    return GTK_OK;
+  };
+  int rc;
+  const int rows_all = (int)round_up(N, 32);
+  if (!chunked) {
+    prologue(0, rows_all, 3);
+    GTK_LAUNCH_CHECK();
+    if ((rc = attend(0, (int)N))) return rc;
+    GTK_LAUNCH_CHECK();
+    return GTK_OK;
+  }
+  prologue(0, rows_all, 2);  // the bias over every row
+  GTK_LAUNCH_CHECK();
+  for (int64_t r0 = 0; r0 < N; r0 += chunk_rows) {
+    const int nrows = (int)std::min<int64_t>(chunk_rows, N - r0);
+    a.r0 = (int)r0;
+    prologue((int)r0, nrows, 1);
+    GTK_LAUNCH_CHECK();
+    if ((rc = attend((int)r0, nrows))) return rc;
+    GTK_LAUNCH_CHECK();
+  }
+  return GTK_OK;
+}
+
 // c_in in {32, 64, 128}, H in {1, 2, 4}, d = c_h / H in [1, 32] (heads are
 // padded to 32 channels); the bf16 kernels built for the module's headline
 // shape (c_in = 128, H = 4) run every d, the others run the generic kernels.
@@ -1635,9 +1995,20 @@ static bool triattn_shape_ok(int64_t cin, int64_t ch, int64_t H) {
 static bool triattn_fast_shape(int64_t cin, int64_t H) { return cin == 128 && H == 4; }
 
 template <typename T>
-static int fwd_triattn_any(int64_t cin, int64_t H, const void* x, const float* mask, void* out,
+static int fwd_triattn_any(int64_t cin, int64_t c_h, int64_t H, const void* x, const float* mask, void* out,
                            const void* packed, int64_t B, int64_t N, int starting, int residual,
                            float eps, float inf, int64_t chunk_rows, void* ws, hipStream_t st) {
+  if constexpr (sizeof(T) == 4) {
+    if (attn_head_pad<T>(c_h, H) == 8) {
+      auto go = [&](auto c) {
+        return fwd_attn8<decltype(c)::value>(x, mask, out, packed, B, N, c_h, starting, residual, eps, inf,
+                                             chunk_rows, ws, st);
+      };
+      if (cin == 128) return go(std::integral_constant<int, 128>());
+      if (cin == 64) return go(std::integral_constant<int, 64>());
+      if (cin == 32) return go(std::integral_constant<int, 32>());
+    }
+  }
 #define GTK_TA(C, HH)                                                                               \
   if (cin == C && H == HH)                                                                       \
     return fwd_triattn<T, C, HH>(x, mask, out, packed, B, N, starting, residual, eps, inf, chunk_rows, \
@@ -1716,7 +2087,8 @@ extern "C" size_t gtk_tri_attn_workspace_size_chunked(int64_t B, int64_t N, int6
   Carve cv(nullptr, SIZE_MAX);
   const int64_t rows = chunk_rows > 0 && chunk_rows < N ? chunk_rows : 0;
   const int chp = (int)H * HD;
-  if (dtype == GTK_F32) carve_attn_ws<float>(cv, B, attn_pad(N), (int)H, chp, rows, false);
+  if (dtype == GTK_F32 && attn_head_pad<float>(c_h, H) == 8) carve_attn8_ws(cv, B, attn_pad(N), rows);
+  else if (dtype == GTK_F32) carve_attn_ws<float>(cv, B, attn_pad(N), (int)H, chp, rows, false);
   else carve_attn_ws<bf16>(cv, B, attn_pad(N), (int)H, chp, rows, fast);
   return cv.off;
 }
@@ -1747,9 +2119,9 @@ extern "C" int gtk_tri_attn_forward_chunked(const void* x, const float* mask, vo
               ws_bytes, need);
   hipStream_t st = (hipStream_t)stream;
   if (dtype == GTK_F32)
-    return fwd_triattn_any<float>(c_in, H, x, mask, out, packed, B, N, starting, residual, eps, inf,
+    return fwd_triattn_any<float>(c_in, c_h, H, x, mask, out, packed, B, N, starting, residual, eps, inf,
                                   chunk_rows, ws, st);
-  return fwd_triattn_any<bf16>(c_in, H, x, mask, out, packed, B, N, starting, residual, eps, inf,
+  return fwd_triattn_any<bf16>(c_in, c_h, H, x, mask, out, packed, B, N, starting, residual, eps, inf,
                                chunk_rows, ws, st);
 }
 
