@@ -856,16 +856,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // q or gate tile [32 channels][32 queries] (2 KiB contiguous in the tiled
   // layout) -> the wave's region, 64-byte rows; copy j moves channels
   // 16j .. 16j+15, lane l takes channel 16j + l/4, queries 8*(l%4) .. +7
-  // (q is read once and for all: non-temporal.  The gate's copy goes plain: the
-  // flash kernel took 137 -> 132 us at N = 512 that way, 62 -> 60 at 384.)
-  auto issue_cq = [&](const bf16* src, bool nt_hint = true) {
+  // (Both are read once and for all: non-temporal.  With plain copies of the
+  // gate the flash kernel alone took 137 -> 132 us at N = 512, but the lines
+  // they leave in the cache cost the kernels after it more: a layer at B = 2,
+  // N = 384 took 1008 -> 1052 us.)
+  auto issue_cq = [&](const bf16* src) {
     const uint32_t ln = (uint32_t)(lane + opaque_zero());
     const uint32_t voff = ln * 16;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if (nt_hint) g2lds16_sv_nt(src + j * 512, voff, stg_lds + j * 1024);
-      else g2lds16_sv(src + j * 512, voff, stg_lds + j * 1024);
-    }
+    for (int j = 0; j < 2; ++j) g2lds16_sv_nt(src + j * 512, voff, stg_lds + j * 1024);
   };
   // channels c0 .. c0+3 of this lane's query t32 (transposing read); ln is
   // the lane id through opaque_zero, so that these per-lane addresses are
@@ -1117,7 +1116,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     Frag<bf16> qf[2];
     if (active) {
       read_q(qf);
-      issue_cq(g_row + qt * 1024, false);  // the gate tile lands behind the key loop
+      issue_cq(g_row + qt * 1024);  // the gate tile lands behind the key loop
     }
     // Stage s is computed while stage s + 1 is copied into the other half of
     // kv, which held stage s - 1.  Opening a stage, a wave waits for its own
@@ -1211,7 +1210,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       if (qt != wave) __builtin_amdgcn_s_waitcnt(vmcnt_imm<2>());
       Frag<bf16> qf[2];
       read_q(qf);
-      issue_cq(g_row + qt * 1024, false);  // the gate tile lands behind the key loop
+      issue_cq(g_row + qt * 1024);  // the gate tile lands behind the key loop
       f32x16 o = zero16();
       float l_run = 0.f;
       for (int t = 0; fast_ok && t < nk; t += KB) {
