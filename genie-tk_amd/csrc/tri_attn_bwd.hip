@@ -344,6 +344,12 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_proj_lds_kernel(const bf16* 
           bT[bias_frag_elem(h, r, j, np)] = bs;
           bS[bias_frag_elem(h, j, r, np)] = bs;
         }
+        // queries N .. np - 1 of this key, dealt over the rows: the dK / dV
+        // kernel drops them through lse2 = +inf, which needs a finite score
+        // (a NaN that the workspace happened to hold would reach every key)
+        for (int q = N + r; q < np; q += N)
+#pragma unroll
+          for (int h = 0; h < H; ++h) bS[bias_frag_elem(h, j, q, np)] = 0.f;
       }
     }
     // 1 for a valid key (mask == 1: no bias); 0 for a masked key
