@@ -333,23 +333,28 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_proj_lds_kernel(const bf16* 
     {
       // triangle bias: outputs 0..H-1 sit in lanes of half 0, acc[0..H-1]
       const f32x16 acc = gemm(wl + 4 * PW, 0);
-      if (valid && half == 0) {
+      if (half == 0) {
         float* bT = bf.biasT + (int64_t)b * H * np * np;
         float* bS = bf.biasS + (int64_t)b * H * np * np;
 #pragma unroll
         for (int h = 0; h < H; ++h) {
           const bf16 bv = cvt<bf16>(acc[h] + bl[4 * CH + h + oz]);
-          bf.bias[(((int64_t)b * H + h) * N + r) * N + j] = bv;
-          const float bs = to_f32(bv) * inv_scale;  // query r, key j
+          if (valid) bf.bias[(((int64_t)b * H + h) * N + r) * N + j] = bv;
+          const float bs = valid ? to_f32(bv) * inv_scale : 0.f;  // query r, key j
           bT[bias_frag_elem(h, r, j, np)] = bs;
           bS[bias_frag_elem(h, j, r, np)] = bs;
         }
-        // queries N .. np - 1 of this key, dealt over the rows: the dK / dV
-        // kernel drops them through lse2 = +inf, which needs a finite score
-        // (a NaN that the workspace happened to hold would reach every key)
+        // Queries N .. np - 1 of this key, dealt over the rows.  The kernels
+        // drop padded queries and keys after their scores (the dK / dV kernel
+        // through lse2 = +inf), which have to be finite for that: a NaN that
+        // the workspace happened to hold would reach every key, and a large
+        // value would send its tile to the exact softmax.
         for (int q = N + r; q < np; q += N)
 #pragma unroll
-          for (int h = 0; h < H; ++h) bS[bias_frag_elem(h, j, q, np)] = 0.f;
+          for (int h = 0; h < H; ++h) {
+            bT[bias_frag_elem(h, q, j, np)] = 0.f;
+            bS[bias_frag_elem(h, j, q, np)] = 0.f;
+          }
       }
     }
     // 1 for a valid key (mask == 1: no bias); 0 for a masked key
