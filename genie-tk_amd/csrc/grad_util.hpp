@@ -43,11 +43,11 @@ __global__ void pack_acc_kernel(Tout* __restrict__ dst, const Tin* __restrict__ 
 
 template <typename Tout>
 inline int launch_pack_acc(Tout* dst, const void* src, int wdtype, int out_dim, int k_dim,
-                           int64_t s_out, int64_t s_in, hipStream_t st) {
+                           int64_t s_out, int64_t s_in, hipStream_t st, Pad pk = Pad()) {
   if (PackBatch* b = pack_batch()) {
     batch_wjob(*b, sizeof(Tout) == 2, wdtype,
                WJob{dst, src, out_dim, k_dim, s_out, s_in, 1.f, nullptr, packed_elems(out_dim, k_dim), Pad(),
-                    Pad(), 1});
+                    pk, 1});
     return GTK_OK;
   }
   const int64_t total = packed_elems(out_dim, k_dim);
@@ -325,20 +325,34 @@ inline int launch_transpose_planes(const T* in, T* out, int Np, int64_t nplanes,
   return GTK_OK;
 }
 
-// Zero columns [P, pitch) of `rows` CM rows.
+// Zero columns [P, pitch) of the rows of several sets of CM rows, in one launch
+// (block y = set): nobody else writes those columns, so one launch a backward
+// pass does for all of its operands (five of 4.6 us each at N = 250 before).
+template <typename T> struct TailJobs {
+  static constexpr int kMax = 5;
+  T* base[kMax];
+  int64_t rows[kMax];
+  int count = 0;
+  int64_t most = 0;
+  void add(T* b, int64_t r) {
+    base[count] = b;
+    rows[count++] = r;
+    most = r > most ? r : most;
+  }
+};
 template <typename T>
-__global__ void zero_tail_kernel(T* __restrict__ base, int64_t rows, int64_t pitch, int64_t P) {
+__global__ void zero_tail_kernel(TailJobs<T> L, int64_t pitch, int64_t P) {
   const int64_t w = pitch - P;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= rows * w) return;
-  base[(idx / w) * pitch + P + idx % w] = cvt<T>(0.f);
+  if (idx >= L.rows[blockIdx.y] * w) return;
+  L.base[blockIdx.y][(idx / w) * pitch + P + idx % w] = cvt<T>(0.f);
 }
 
 template <typename T>
-inline int launch_zero_tail(T* base, int64_t rows, int64_t pitch, int64_t P, hipStream_t st) {
-  const int64_t n = rows * (pitch - P);
+inline int launch_zero_tails(const TailJobs<T>& L, int64_t pitch, int64_t P, hipStream_t st) {
+  const int64_t n = L.most * (pitch - P);
   if (n <= 0) return GTK_OK;
-  zero_tail_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(base, rows, pitch, P);
+  zero_tail_kernel<T><<<dim3((unsigned)((n + 255) / 256), L.count), 256, 0, st>>>(L, pitch, P);
   GTK_LAUNCH_CHECK();
   return GTK_OK;
 }
@@ -628,90 +642,151 @@ inline size_t wgrad_rowsum_floats(int M, int64_t pitch) {
   return (size_t)wgrad_plan(M, pitch).nsplit * wgrad_m_rows(M);
 }
 
-// Row ranges of one product's output, each finished into its own tensor.
-struct WgradSegs {
-  static constexpr int kMax = 8;
-  float* dst[kMax];
-  int m0[kMax];
-  int rows[kMax];
+// ---------------------------------------------------------------------------
+// Closing sums.  Every gradient of a backward pass ends as a sum over partials:
+// the splits of a product, the splits of its row sums, the segments of a row
+// reduction.  Each of these sums is a few microseconds of launch and load
+// latency, so all of a pass run in one launch (8 launches of 4.6 us at N = 250
+// before, 36.6 us; one of 8 now), each reading its partials directly:
+//   dst[m][n] = sum_s src[s * step + row(m) * sm + col(n) * sn] * (gamma ? gamma[n] : 1)
+//             + (rs ? beta[n] * sum_s rs[s * rs_step + row(m) * rs_m] : 0)
+// row and col map an index of the gradient to the padded one of the product
+// (Pad::pos).  With rs, cols is a multiple of kSumOuts: a block's outputs then
+// share their row.
+// ---------------------------------------------------------------------------
+constexpr int kSumOuts = 32, kSumChunks = 16;
+struct SumJob {
+  float* dst = nullptr;
+  const float* src = nullptr;
+  int64_t step = 0;
+  int nsplit = 0, sm = 0, sn = 0, rows = 0, cols = 1;
+  Pad row, col;
+  const float *gamma = nullptr, *beta = nullptr;
+  const float* rs = nullptr;
+  int64_t rs_step = 0;
+  int rs_m = 0, rs_n = 0;
+};
+struct SumJobs {
+  static constexpr int kMax = 16;
+  SumJob j[kMax];
+  int first[kMax + 1] = {0};  // first block of each job
   int count = 0;
-  void add(float* d, int m, int r) {
-    if (!d || r == 0) return;
-    dst[count] = d;
-    m0[count] = m;
-    rows[count] = r;
+  bool overflow = false;
+  void add(const SumJob& job) {
+    if (!job.dst || job.rows == 0) return;
+    if (count == kMax || (job.rs && job.cols % kSumOuts != 0)) {
+      overflow = true;
+      return;
+    }
+    j[count] = job;
+    first[count + 1] = first[count] + (job.rows * job.cols + kSumOuts - 1) / kSumOuts;
     ++count;
   }
 };
 
-// Segment k = blockIdx.y: dst_k[(m - m0_k)][n] = sum_s part[s][m][n] * (gamma ? gamma[n] : 1)
-//   + (rowsum && beta ? rowsum[m] * beta[n] : 0),  m in [m0_k, m0_k + rows_k),
-// n < Nn, with part laid out as [nsplit][Mp][Np] (the padded product).
-// Block: 32 consecutive outputs x 8 chunks of the splits (chunk c takes s = c,
-// c + 8, ..., four loads in flight), the 8 partial sums of each output added
-// through LDS.
-static __global__ __launch_bounds__(256) void wgrad_finish_kernel(
-    const float* __restrict__ part, int nsplit, int Mp, int Np, int Nn, WgradSegs segs,
-    const float* __restrict__ rowsum, const float* __restrict__ gamma, const float* __restrict__ beta) {
-  __shared__ float red[8][32];
-  const int k = blockIdx.y;
-  const int o = threadIdx.x & 31, ch = threadIdx.x >> 5;
-  const int idx = blockIdx.x * 32 + o;
-  if (blockIdx.x * 32 >= segs.rows[k] * Nn) return;  // block-uniform
-  const bool live = idx < segs.rows[k] * Nn;
-  const int m = segs.m0[k] + (live ? idx / Nn : 0), n = live ? idx % Nn : 0;
+// Block: 32 consecutive outputs x 16 chunks of the splits (chunk c takes s = c,
+// c + 16, ..., eight loads in flight), the chunks' sums added through LDS.
+static __global__ __launch_bounds__(kSumOuts * kSumChunks) void grad_sums_kernel(SumJobs L) {
+  __shared__ float red[kSumChunks][kSumOuts];
+  __shared__ float rsw[kSumOuts * kSumChunks / 64];
+  int k = 0;
+  while (k + 1 < L.count && (int)blockIdx.x >= L.first[k + 1]) ++k;
+  const SumJob& J = L.j[k];
+  const int o = threadIdx.x % kSumOuts, ch = threadIdx.x / kSumOuts;
+  const int idx0 = ((int)blockIdx.x - L.first[k]) * kSumOuts, idx = idx0 + o;
+  const bool live = idx < J.rows * J.cols;
+  const int m = live ? idx / J.cols : 0, n = live ? idx % J.cols : 0;
   float acc = 0.f;
   if (live) {
-    const float* src = part + (int64_t)m * Np + n;
-    const int64_t step = (int64_t)Mp * Np;
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
-    int sp = ch;
-    for (; sp + 24 < nsplit; sp += 32)
+    const float* src = J.src + (int64_t)J.row.pos(m) * J.sm + (int64_t)J.col.pos(n) * J.sn;
+    const int last = J.nsplit - 1;
+    float a[8] = {};
+    for (int s = ch; s <= last; s += 8 * kSumChunks)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) a[u] += src[(sp + 8 * u) * step];
-    for (; sp < nsplit; sp += 8) a[0] += src[sp * step];
-    acc = (a[0] + a[1]) + (a[2] + a[3]);
+      for (int u = 0; u < 8; ++u) {
+        const int su = s + u * kSumChunks;
+        const float v = src[(su < last ? su : last) * J.step];
+        a[u] += su <= last ? v : 0.f;
+      }
+    acc = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
   }
   red[ch][o] = acc;
+  if (J.rs) {  // block-uniform
+    const float* rs = J.rs + (int64_t)J.row.pos(idx0 / J.cols) * J.rs_m;
+    float v = 0.f;
+    for (int s = threadIdx.x; s < J.rs_n; s += kSumOuts * kSumChunks) v += rs[s * J.rs_step];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if ((threadIdx.x & 63) == 0) rsw[threadIdx.x / 64] = v;
+  }
   __syncthreads();
   if (ch != 0 || !live) return;
 #pragma unroll
-  for (int c = 1; c < 8; ++c) acc += red[c][o];
-  if (gamma) acc *= gamma[n];
-  if (rowsum && beta) acc += rowsum[m] * beta[n];
-  segs.dst[k][idx] = acc;
+  for (int c = 1; c < kSumChunks; ++c) acc += red[c][o];
+  if (J.gamma) acc *= J.gamma[n];
+  if (J.rs) {
+    float r = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSumOuts * kSumChunks / 64; ++w) r += rsw[w];
+    acc += r * J.beta[n];
+  }
+  J.dst[idx] = acc;
 }
 
-inline int launch_wgrad_finish(const float* part, int M, int Nn, int64_t pitch, const WgradSegs& segs,
-                               const float* rowsum, const float* gamma, const float* beta, hipStream_t st) {
-  if (segs.count == 0) return GTK_OK;
-  int most = 0;
-  for (int k = 0; k < segs.count; ++k) most = segs.rows[k] > most ? segs.rows[k] : most;
-  const int n = most * Nn;
-  wgrad_finish_kernel<<<dim3((n + 31) / 32, segs.count), 256, 0, st>>>(
-      part, wgrad_plan(M, pitch).nsplit, wgrad_m_rows(M), wgrad_n_rows(Nn), Nn, segs, rowsum, gamma, beta);
+inline int launch_grad_sums(const SumJobs& L, hipStream_t st) {
+  GTK_REQUIRE(!L.overflow, GTK_EINVAL, "closing sums: too many jobs or an unsupported row length");
+  if (L.count == 0) return GTK_OK;
+  grad_sums_kernel<<<(unsigned)L.first[L.count], kSumOuts * kSumChunks, 0, st>>>(L);
   GTK_LAUNCH_CHECK();
   return GTK_OK;
 }
 
-inline int launch_wgrad_finish(const float* part, int M, int Nn, int64_t pitch, int m0, int rows,
-                               const float* rowsum, const float* gamma, const float* beta,
-                               float* dst, hipStream_t st) {
-  WgradSegs segs;
-  segs.add(dst, m0, rows);
-  return launch_wgrad_finish(part, M, Nn, pitch, segs, rowsum, gamma, beta, st);
+// Rows m0 .. m0 + rows - 1 of the product that launch_wgrad left in part.
+inline SumJob sum_of_product(float* dst, const float* part, int M, int Nn, int64_t pitch, int m0, int rows) {
+  SumJob j;
+  j.dst = dst;
+  j.sm = wgrad_n_rows(Nn);
+  j.sn = 1;
+  j.src = part + (int64_t)m0 * j.sm;
+  j.step = (int64_t)wgrad_m_rows(M) * j.sm;
+  j.nsplit = wgrad_plan(M, pitch).nsplit;
+  j.rows = rows;
+  j.cols = Nn;
+  return j;
+}
+// The affine fold of a LayerNorm in front: dW = W diag(gamma) + s beta^T with
+// s the row sums rs of the same launch_wgrad (null: no beta term).
+inline SumJob with_affine(SumJob j, const float* gamma, const float* beta, const float* rs, int M, int64_t pitch,
+                          int m0) {
+  j.gamma = gamma;
+  j.beta = beta;
+  j.rs = rs + m0;
+  j.rs_step = wgrad_m_rows(M);
+  j.rs_m = 1;
+  j.rs_n = wgrad_plan(M, pitch).nsplit;
+  return j;
+}
+// Rows m0 .. m0 + rows - 1 of the row sums that launch_wgrad left in rs.
+inline SumJob sum_of_rows(float* dst, const float* rs, int M, int64_t pitch, int m0, int rows) {
+  SumJob j;
+  j.dst = dst;
+  j.src = rs + m0;
+  j.step = wgrad_m_rows(M);
+  j.nsplit = wgrad_plan(M, pitch).nsplit;
+  j.sm = 1;
+  j.rows = rows;
+  return j;
 }
 
 // part[s][m][n] (m < wgrad_m_rows(M), n < wgrad_n_rows(Nn)): split s of
-// sum_k G[m][k] X[n][k].  With rs and sums: also sums[m] = sum_k G[m][k] for
-// m < M (rs: wgrad_rowsum_floats(M, pitch) floats of partials).
+// sum_k G[m][k] X[n][k].  With rs (wgrad_rowsum_floats(M, pitch) floats): also
+// rs[s][m], split s of sum_k G[m][k].
 template <typename T>
 inline int launch_wgrad(const T* G, const T* X, float* part, int M, int Nn, int64_t pitch,
-                        hipStream_t st, float* rs = nullptr, float* sums = nullptr) {
+                        hipStream_t st, float* rs = nullptr) {
   GTK_REQUIRE(M >= 1 && Nn >= 1, GTK_EUNSUPPORTED, "weight gradient shape %d x %d unsupported", M, Nn);
   const int Mp = wgrad_m_rows(M), Np = wgrad_n_rows(Nn);
   const WgradPlan pl = wgrad_plan(M, pitch);
-  const bool with_rs = rs && sums;
   auto go = [&](auto tn, auto r) {
     constexpr int TN = decltype(tn)::value;
     const int64_t blocks = (int64_t)pl.nsplit * (Mp / 128) * (TN == 128 ? Np / 128 : 1);
@@ -725,21 +800,13 @@ inline int launch_wgrad(const T* G, const T* X, float* part, int M, int Nn, int6
   using I128 = std::integral_constant<int, 128>;
   using I64 = std::integral_constant<int, 64>;
   if (Np % 128 == 0) {
-    if (with_rs) go(I128{}, std::true_type{});
+    if (rs) go(I128{}, std::true_type{});
     else go(I128{}, std::false_type{});
   } else {
-    if (with_rs) go(I64{}, std::true_type{});
+    if (rs) go(I64{}, std::true_type{});
     else go(I64{}, std::false_type{});
   }
   GTK_LAUNCH_CHECK();
-  if (with_rs) {
-    // rs is a product output of one column: the same split reduction
-    WgradSegs one;
-    one.add(sums, 0, M);
-    wgrad_finish_kernel<<<dim3((M + 31) / 32, 1), 256, 0, st>>>(rs, pl.nsplit, Mp, 1, 1, one, nullptr, nullptr,
-                                                                nullptr);
-    GTK_LAUNCH_CHECK();
-  }
   return GTK_OK;
 }
 
@@ -750,14 +817,22 @@ inline int launch_wgrad(const T* G, const T* X, float* part, int M, int Nn, int6
 // ---------------------------------------------------------------------------
 constexpr int kRowSegs = 8;
 
+struct RowJobs {  // rows of G, with or without X
+  static constexpr int kMax = 2;
+  const void *G[kMax], *X[kMax];
+  float *ps[kMax], *pd[kMax];
+  int nseg[kMax];
+  int first[kMax + 1] = {0};  // first block of each job
+  int count = 0;
+};
+
 template <typename T, bool DOT>
-__global__ __launch_bounds__(256) void rowred_kernel(const T* __restrict__ G, const T* __restrict__ X,
-                                                     int rows, int64_t pitch, int64_t P,
-                                                     float* __restrict__ psum, float* __restrict__ pdot) {
+__device__ __forceinline__ void rowred_block(const T* __restrict__ G, const T* __restrict__ X, int block, int nseg,
+                                             int64_t pitch, int64_t P, float* __restrict__ psum,
+                                             float* __restrict__ pdot) {
   __shared__ float red[2][4];
   constexpr int STEP = 8 * 256;  // entries a block reads per pass
-  const int nseg = (int)(gridDim.x / rows);
-  const int r = blockIdx.x / nseg, s = blockIdx.x % nseg;
+  const int r = block / nseg, s = block % nseg;
   const int64_t seg = ((P + nseg - 1) / nseg + 7) / 8 * 8;
   const int64_t b0 = s * seg;
   const int64_t b1 = b0 + seg < P ? b0 + seg : P;
@@ -813,25 +888,14 @@ __global__ __launch_bounds__(256) void rowred_kernel(const T* __restrict__ G, co
   }
 }
 
-// One wave a row: lane l adds segments l, l + 64, ...
-static __global__ __launch_bounds__(64) void rowred_finish_kernel(const float* __restrict__ ps,
-                                                                 const float* __restrict__ pd, int rows, int nseg,
-                                                                 float* __restrict__ sums, float* __restrict__ dots) {
-  const int r = blockIdx.x, l = threadIdx.x;
-  float a = 0.f, d = 0.f;
-  for (int s = l; s < nseg; s += 64) {
-    a += ps[(int64_t)r * nseg + s];
-    if (dots) d += pd[(int64_t)r * nseg + s];
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_xor(a, o, 64);
-    d += __shfl_xor(d, o, 64);
-  }
-  if (l == 0) {
-    sums[r] = a;
-    if (dots) dots[r] = d;
-  }
+// One launch for a pass's row reductions, each block a segment of one row.
+template <typename T>
+__global__ __launch_bounds__(256) void rowred_kernel(RowJobs L, int64_t pitch, int64_t P) {
+  const int k = L.count > 1 && (int)blockIdx.x >= L.first[1] ? 1 : 0;
+  const int block = (int)blockIdx.x - L.first[k];
+  const T *G = (const T*)L.G[k], *X = (const T*)L.X[k];
+  if (X) rowred_block<T, true>(G, X, block, L.nseg[k], pitch, P, L.ps[k], L.pd[k]);
+  else rowred_block<T, false>(G, nullptr, block, L.nseg[k], pitch, P, L.ps[k], nullptr);
 }
 
 // Segments a row is split into: kRowSegs, or more for few rows (so that the
@@ -839,58 +903,38 @@ static __global__ __launch_bounds__(64) void rowred_finish_kernel(const float* _
 // which bounds the partials in tmp (2 x that many floats).
 inline int rowred_segs(int rows) { return rows >= 128 ? kRowSegs : 1024 / rows; }
 
-// sums[r] (and dots[r] when X is given) for rows [0, rows) of G; tmp holds
-// 2 * rows * rowred_segs(rows) floats of partials.
+// Floats of the partials of a reduction of `rows` rows: the sums, then the dots.
+inline int64_t rowred_floats(int rows) { return (int64_t)2 * rows * rowred_segs(rows); }
+
+// The reduction of rows [0, rows) of G (with X: the dot products too) into the
+// rowred_floats(rows) partials tmp; the closing sums into the gradients sums
+// and dots (X given).
 template <typename T>
-inline int launch_rowred(const T* G, const T* X, int rows, int64_t pitch, int64_t P, float* tmp,
-                         float* sums, float* dots, hipStream_t st) {
-  if (rows == 0) return GTK_OK;
-  const int nseg = rowred_segs(rows);
-  float* ps = tmp;
-  float* pd = tmp + (size_t)rows * nseg;
-  if (X) rowred_kernel<T, true><<<rows * nseg, 256, 0, st>>>(G, X, rows, pitch, P, ps, pd);
-  else rowred_kernel<T, false><<<rows * nseg, 256, 0, st>>>(G, nullptr, rows, pitch, P, ps, nullptr);
-  GTK_LAUNCH_CHECK();
-  rowred_finish_kernel<<<rows, 64, 0, st>>>(ps, pd, rows, nseg, sums, X ? dots : nullptr);
-  GTK_LAUNCH_CHECK();
-  return GTK_OK;
+inline void add_rowred(RowJobs& R, SumJobs& S, const T* G, const T* X, int rows, float* tmp, float* sums,
+                       float* dots) {
+  const int k = R.count++, nseg = rowred_segs(rows);
+  R.G[k] = G;
+  R.X[k] = X;
+  R.ps[k] = tmp;
+  R.pd[k] = tmp + (int64_t)rows * nseg;
+  R.nseg[k] = nseg;
+  R.first[k + 1] = R.first[k] + rows * nseg;
+  SumJob j;
+  j.step = 1;
+  j.nsplit = j.sm = nseg;
+  j.rows = rows;
+  j.dst = sums;
+  j.src = R.ps[k];
+  S.add(j);
+  j.dst = X ? dots : nullptr;
+  j.src = R.pd[k];
+  S.add(j);
 }
 
-static __global__ void copy_f32_kernel(float* __restrict__ dst, const float* __restrict__ src, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-inline int launch_copy_f32(float* dst, const float* src, int n, hipStream_t st) {
-  if (!dst || n == 0) return GTK_OK;
-  copy_f32_kernel<<<(n + 255) / 256, 256, 0, st>>>(dst, src, n);
-  GTK_LAUNCH_CHECK();
-  return GTK_OK;
-}
-
-// Several small fp32 copies in one launch (block y = copy k).
-struct CopyList {
-  static constexpr int kMax = 8;
-  float* dst[kMax];
-  const float* src[kMax];
-  int n[kMax];
-  int count = 0;
-  void add(float* d, const float* s, int len) {
-    if (!d || len == 0) return;
-    dst[count] = d;
-    src[count] = s;
-    n[count] = len;
-    ++count;
-  }
-};
-static __global__ void copy_list_kernel(CopyList l) {
-  const int k = blockIdx.y;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < l.n[k]; i += gridDim.x * blockDim.x)
-    l.dst[k][i] = l.src[k][i];
-}
-inline int launch_copy_list(const CopyList& l, hipStream_t st) {
-  if (l.count == 0) return GTK_OK;
-  GTK_REQUIRE(l.count <= CopyList::kMax, GTK_EINVAL, "copy list overflow");
-  copy_list_kernel<<<dim3(1, l.count), 256, 0, st>>>(l);
+template <typename T>
+inline int launch_rowred(const RowJobs& R, int64_t pitch, int64_t P, hipStream_t st) {
+  if (R.count == 0) return GTK_OK;
+  rowred_kernel<T><<<(unsigned)R.first[R.count], 256, 0, st>>>(R, pitch, P);
   GTK_LAUNCH_CHECK();
   return GTK_OK;
 }

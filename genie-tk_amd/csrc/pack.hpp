@@ -14,15 +14,18 @@
 namespace gtk {
 
 // Grouped padding of one dimension: padded index i is element (i / gp) * g +
-// (i % gp) of the source, or zero when i % gp >= g.  Multi-head attention
-// pads each head of g channels to gp; {kNoPad, kNoPad} is the identity.
+// (i % gp) of the source, or zero when i % gp >= g or that element is not one
+// of the source's n.  Multi-head attention pads each head of g channels to gp;
+// the default is the identity.
 constexpr int kNoPad = 1 << 30;
 struct Pad {
-  int gp = kNoPad, g = kNoPad;
+  int gp = kNoPad, g = kNoPad, n = kNoPad;
   __host__ __device__ __forceinline__ int src(int i) const {
     const int q = i / gp, r = i - q * gp;
-    return r < g ? q * g + r : -1;
+    return r < g && q * g + r < n ? q * g + r : -1;
   }
+  // the padded index of source element i
+  __host__ __device__ __forceinline__ int pos(int i) const { return i / g * gp + i % g; }
 };
 
 inline int64_t packed_elems(int64_t out_dim, int64_t k_dim) {

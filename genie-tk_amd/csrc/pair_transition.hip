@@ -862,7 +862,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void p
 }
 
 // dst_k[i] = sum_s src_k[s * n_k + i], job k = blockIdx.y: 32 outputs x 8 chunks
-// of the splits a block (the order of wgrad_finish_kernel).
+// of the splits a block.
 struct PtSums {
   static constexpr int kJobs = 4;
   const float* src[kJobs];
@@ -978,7 +978,7 @@ static int launch_pt_generic(const void* p, const float* mask, void* out, const 
 template <typename T> struct PtBwdWs {
   void* packed;
   T *w2t, *w1t, *cm_xh, *cm_dxn, *cm_dy, *cm_a, *cm_dh;
-  float *part1, *part2, *red, *rs, *sums_dh, *sums_dy, *sums_dxn, *dots_dxn;
+  float *part1, *part2, *red_dy, *red_dxn, *rs;
   int64_t pitch;
 };
 
@@ -998,12 +998,9 @@ static PtBwdWs<T> carve_pt_bwd(Carve& cv, int64_t rows, int c, int hid) {
   a.cm_dh = cv.take<T>(hid * a.pitch);
   a.part1 = cv.take<float>(wgrad_part_floats(hid, c, a.pitch));
   a.part2 = cv.take<float>(wgrad_part_floats(hid, c, a.pitch));
-  a.red = cv.take<float>((int64_t)2 * hid * kRowSegs);
+  a.red_dy = cv.take<float>(rowred_floats(c));
+  a.red_dxn = cv.take<float>(rowred_floats(c));
   a.rs = cv.take<float>(wgrad_rowsum_floats(hid, a.pitch));
-  a.sums_dh = cv.take<float>(hid);
-  a.sums_dy = cv.take<float>(c);
-  a.sums_dxn = cv.take<float>(c);
-  a.dots_dxn = cv.take<float>(c);
   return a;
 }
 
@@ -1117,32 +1114,34 @@ static int bwd_pt(const void* p, const void* dy, const gtk_pair_transition_weigh
         a.w1t, rows, pitch, eps);
     GTK_LAUNCH_CHECK();
   }
-  T* planes[5] = {a.cm_xh, a.cm_dxn, a.cm_dy, a.cm_a, a.cm_dh};
-  const int prow[5] = {C, C, C, HID, HID};
-  for (int k = 0; k < 5; ++k)
-    if ((rc = launch_zero_tail<T>(planes[k], prow[k], pitch, rows, st))) return rc;
-  // bias and LayerNorm gradients straight into the outputs where requested
-  auto or_tmp = [](float* dst, float* tmp) { return dst ? dst : tmp; };
-  if ((rc = launch_rowred<T>(a.cm_dy, nullptr, C, pitch, rows, a.red, or_tmp(gr->b2, a.sums_dy), nullptr, st)))
-    return rc;
-  if ((rc = launch_rowred<T>(a.cm_dxn, a.cm_xh, C, pitch, rows, a.red, or_tmp(gr->ln_b, a.sums_dxn),
-                             or_tmp(gr->ln_w, a.dots_dxn), st)))
-    return rc;
+  TailJobs<T> tails;
+  tails.add(a.cm_xh, C);
+  tails.add(a.cm_dxn, C);
+  tails.add(a.cm_dy, C);
+  tails.add(a.cm_a, HID);
+  tails.add(a.cm_dh, HID);
+  if ((rc = launch_zero_tails<T>(tails, pitch, rows, st))) return rc;
+  RowJobs rowsums;
+  SumJobs sums;
+  add_rowred<T>(rowsums, sums, a.cm_dy, nullptr, C, a.red_dy, gr->b2, nullptr);
+  add_rowred<T>(rowsums, sums, a.cm_dxn, a.cm_xh, C, a.red_dxn, gr->ln_b, gr->ln_w);
+  if ((rc = launch_rowred<T>(rowsums, pitch, rows, st))) return rc;
   {
     // the first product also sums its G rows (dh): the b1 gradient
     StageTimer timer("pair_transition_bwd_wgrad", st);
-    if ((rc = launch_wgrad<T>(a.cm_dh, a.cm_xh, a.part1, HID, C, pitch, st, a.rs, a.sums_dh))) return rc;
+    if ((rc = launch_wgrad<T>(a.cm_dh, a.cm_xh, a.part1, HID, C, pitch, st, a.rs))) return rc;
     if ((rc = launch_wgrad<T>(a.cm_a, a.cm_dy, a.part2, HID, C, pitch, st))) return rc;
   }
   // dW1 = (sum dh x_hat^T) diag(g) + (sum dh) beta^T
-  if ((rc = launch_wgrad_finish(a.part1, HID, C, pitch, 0, HID, a.sums_dh, w.ln_w, w.ln_b, gr->w1, st)))
-    return rc;
+  sums.add(with_affine(sum_of_product(gr->w1, a.part1, HID, C, pitch, 0, HID), w.ln_w, w.ln_b, a.rs, HID, pitch, 0));
+  sums.add(sum_of_rows(gr->b1, a.rs, HID, pitch, 0, HID));
+  if ((rc = launch_grad_sums(sums, st))) return rc;
   if (gr->w2) {
     wgrad_finish_t_kernel<<<(HID * C + 255) / 256, 256, 0, st>>>(a.part2, wgrad_plan(HID, pitch).nsplit,
                                                                  HID, C, gr->w2);
     GTK_LAUNCH_CHECK();
   }
-  return launch_copy_f32(gr->b1, a.sums_dh, HID, st);
+  return GTK_OK;
 }
 
 }  // namespace gtk

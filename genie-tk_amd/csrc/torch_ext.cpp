@@ -311,10 +311,13 @@ std::vector<at::Tensor> tri_mul_backward(const at::Tensor& z, const c10::optiona
 // Backward of tri_attn_forward (update only): returns [dx, then the gradients of
 // the 10 parameters in tri_attn_pack's order (fp32 views of one buffer), then
 // that buffer].
-std::vector<at::Tensor> tri_attn_backward(const at::Tensor& x, const c10::optional<at::Tensor>& mask,
-                                          const at::Tensor& dy, std::vector<at::Tensor> ps,
-                                          int64_t c_in, int64_t c_h, int64_t H, bool starting,
-                                          double eps) {
+// `entry` is the C function: gtk_tri_attn_backward (four heads of 32) or
+// gtk_tri_attn_backward_heads (every head shape of the forward kernels), whose
+// workspace is that of four heads of 32.
+std::vector<at::Tensor> tri_attn_backward_with(decltype(&gtk_tri_attn_backward) entry, const at::Tensor& x,
+                                               const c10::optional<at::Tensor>& mask, const at::Tensor& dy,
+                                               std::vector<at::Tensor> ps, int64_t c_in, int64_t c_h, int64_t H,
+                                               bool starting, double eps) {
   TORCH_CHECK(ps.size() == 10, "tri_attn_backward expects 10 parameter tensors");
   check_gpu(x, "x");
   check_on(mask, x, "mask");
@@ -346,15 +349,30 @@ std::vector<at::Tensor> tri_attn_backward(const at::Tensor& x, const c10::option
              {{c_in}, {c_in}, {H, c_in}, {c_h, c_in}, {c_h, c_in}, {c_h, c_in}, {c_h, c_in}, {c_h},
               {c_in, c_h}, {c_in}},
              gs);
-  const size_t bytes = gtk_tri_attn_backward_workspace_size(B, N, c_in, c_h, H, dt);
+  const bool heads = entry == &gtk_tri_attn_backward_heads;
+  const size_t bytes = gtk_tri_attn_backward_workspace_size(B, N, c_in, heads ? 128 : c_h, heads ? 4 : H, dt);
   TORCH_CHECK(bytes > 0, "genie_tk._C: tri_attn backward shape c_in=", c_in, " c_h=", c_h, " H=", H,
               " unsupported");
   auto ws = workspace(xc, bytes);
-  check_rc(gtk_tri_attn_backward(xc.data_ptr(), mask.has_value() ? mc.data_ptr<float>() : nullptr,
-                                 dyc.data_ptr(), &w, out[0].data_ptr(), &g, B, N, c_in, c_h, H,
-                                 starting ? 1 : 0, (float)eps, dt, ws.data_ptr(), ws.numel(),
-                                 cur_stream(xc)));
+  check_rc(entry(xc.data_ptr(), mask.has_value() ? mc.data_ptr<float>() : nullptr, dyc.data_ptr(), &w,
+                 out[0].data_ptr(), &g, B, N, c_in, c_h, H, starting ? 1 : 0, (float)eps, dt, ws.data_ptr(),
+                 ws.numel(), cur_stream(xc)));
   return out;
+}
+
+std::vector<at::Tensor> tri_attn_backward(const at::Tensor& x, const c10::optional<at::Tensor>& mask,
+                                          const at::Tensor& dy, std::vector<at::Tensor> ps,
+                                          int64_t c_in, int64_t c_h, int64_t H, bool starting,
+                                          double eps) {
+  return tri_attn_backward_with(&gtk_tri_attn_backward, x, mask, dy, std::move(ps), c_in, c_h, H, starting, eps);
+}
+
+std::vector<at::Tensor> tri_attn_backward_heads(const at::Tensor& x, const c10::optional<at::Tensor>& mask,
+                                                const at::Tensor& dy, std::vector<at::Tensor> ps,
+                                                int64_t c_in, int64_t c_h, int64_t H, bool starting,
+                                                double eps) {
+  return tri_attn_backward_with(&gtk_tri_attn_backward_heads, x, mask, dy, std::move(ps), c_in, c_h, H, starting,
+                                eps);
 }
 
 // chunk_rows > 0: the memory-bounded mode (output rows that many at a time)
@@ -620,6 +638,10 @@ PYBIND11_MODULE(_C, m) {
         "TriangleAttention backward: [dx, 10 parameter gradients (fp32), their buffer]", py::arg("x"),
         py::arg("mask"), py::arg("dy"), py::arg("params"), py::arg("c_in"), py::arg("c_h"),
         py::arg("no_heads"), py::arg("starting"), py::arg("eps") = 1e-5);
+  m.def("tri_attn_backward_heads", &tri_attn_backward_heads,
+        "tri_attn_backward for every head shape of the forward kernels", py::arg("x"), py::arg("mask"),
+        py::arg("dy"), py::arg("params"), py::arg("c_in"), py::arg("c_h"), py::arg("no_heads"),
+        py::arg("starting"), py::arg("eps") = 1e-5);
   m.def("pair_transition_pack", &pair_transition_pack, "Pack PairTransition parameters",
         py::arg("params"), py::arg("c"), py::arg("n"), py::arg("fp32") = false);
   m.def("pair_transition_forward", &pair_transition_forward,

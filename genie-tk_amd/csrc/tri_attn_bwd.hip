@@ -1831,45 +1831,13 @@ __global__ __launch_bounds__(512) void attn_bwd_pro_lds_kernel(const bf16* __res
   }
 }
 
-// dW_b[h][c] = W3[c][h] gamma[c] + s[h] beta[c]  (W3 = sum_s part[s][c][h]: the
-// product's layout [nsplit][Cp][64], Cp = C rounded up to its row tile)
-__global__ __launch_bounds__(256) void attn_dwb_finish_kernel(const float* __restrict__ part, int nsplit, int C,
-                                                            int Cp, int H, const float* __restrict__ gamma,
-                                                            const float* __restrict__ beta,
-                                                            const float* __restrict__ sums, float* __restrict__ dst) {
-  // 8 outputs x 32 chunks of the splits per block (four loads in flight a
-  // thread), partial sums added through LDS
-  __shared__ float red[32][8];
-  const int o = threadIdx.x & 7, ch = threadIdx.x >> 3;
-  const int idx = blockIdx.x * 8 + o;
-  const bool live = idx < H * C;
-  const int h = live ? idx / C : 0, c = live ? idx % C : 0;
-  float acc = 0.f;
-  if (live) {
-    const float* src = part + (int64_t)c * 64 + h;
-    const int64_t step = (int64_t)Cp * 64;
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
-    int s = ch;
-    for (; s + 96 < nsplit; s += 128)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) a[u] += src[(s + 32 * u) * step];
-    for (; s < nsplit; s += 32) a[0] += src[s * step];
-    acc = (a[0] + a[1]) + (a[2] + a[3]);
-  }
-  red[ch][o] = acc;
-  __syncthreads();
-  if (ch != 0 || !live) return;
-  for (int k = 1; k < 32; ++k) acc += red[k][o];
-  dst[idx] = acc * gamma[c] + sums[h] * beta[c];
-}
-
 // ---------------------------------------------------------------------------
 // Workspace
 // ---------------------------------------------------------------------------
 template <typename T> struct AttnBwdWs {
   AttnBwdW<T> w;
   AttnBwdBufs<T> b;
-  float *part1, *part2, *part3, *red, *rs, *sums_stack, *sums_dy, *sums_dxn, *dots_dxn, *sums_dtri;
+  float *part1, *part2, *part3, *red_dxn, *red_dtri, *rs1, *rs2;
 };
 
 template <typename T>
@@ -1919,57 +1887,60 @@ static AttnBwdWs<T> carve_attn_bwd(Carve& cv, int64_t B, int64_t N, int C, int H
   b.cm_dxn = cv.take<T>(C * b.pitch);
   b.cm_dy = cv.take<T>((int64_t)wgrad_rows(C) * b.pitch);
   b.cm_go = cv.take<T>((int64_t)wgrad_rows(CH) * b.pitch);
-  b.cm_dtri = cv.take<T>(64 * b.pitch);
+  b.cm_dtri = cv.take<T>((int64_t)wgrad_n_rows(H) * b.pitch);
   a.part1 = cv.take<float>(wgrad_part_floats(4 * CH, C, b.pitch));
   a.part2 = cv.take<float>(wgrad_part_floats(C, CH, b.pitch));
-  a.part3 = cv.take<float>(wgrad_part_floats(C, 64, b.pitch));
-  a.red = cv.take<float>((int64_t)2 * 4 * CH * kRowSegs);
-  a.rs = cv.take<float>(std::max(wgrad_rowsum_floats(4 * CH, b.pitch), wgrad_rowsum_floats(C, b.pitch)));
-  a.sums_stack = cv.take<float>(4 * CH);
-  a.sums_dy = cv.take<float>(C);
-  a.sums_dxn = cv.take<float>(C);
-  a.dots_dxn = cv.take<float>(C);
-  a.sums_dtri = cv.take<float>(64);
+  a.part3 = cv.take<float>(wgrad_part_floats(C, H, b.pitch));
+  a.red_dxn = cv.take<float>(rowred_floats(C));
+  a.red_dtri = cv.take<float>(rowred_floats(H));
+  a.rs1 = cv.take<float>(wgrad_rowsum_floats(4 * CH, b.pitch));
+  a.rs2 = cv.take<float>(wgrad_rowsum_floats(C, b.pitch));
   return a;
 }
 
+// The module's heads (nh of d channels, nh <= H, d <= AD) take channels AD h ..
+// AD h + d - 1 of the kernels' H heads of AD; the other channels and heads get
+// zero weights, so they add nothing to a gradient of the real ones.
 template <typename T>
-static int pack_attn_bwd(const gtk_tri_attn_weights* wt, AttnBwdW<T>& w, int C, int H,
+static int pack_attn_bwd(const gtk_tri_attn_weights* wt, AttnBwdW<T>& w, int C, int H, int nh, int d,
                          hipStream_t st) {
-  const int CH = H * AD, wd = wt->dtype;
+  const int CH = H * AD, wd = wt->dtype, c_h = nh * d;
+  const Pad heads{AD, d, c_h}, tri{kNoPad, kNoPad, nh};
   PackScope batch(st);  // the packing launches issued as 3
   int rc;
   if ((rc = launch_to_f32(w.ln_w, wt->ln_w, wd, C, 1.f, 1.f, st))) return rc;
   if ((rc = launch_to_f32(w.ln_b, wt->ln_b, wd, C, 1.f, 0.f, st))) return rc;
-  struct Lin { T* dst; float* bdst; const void* wsrc; const void* bsrc; int out; };
-  const Lin lins[5] = {{w.w_q, w.b_q, wt->q_w, nullptr, CH}, {w.w_k, w.b_k, wt->k_w, nullptr, CH},
-                       {w.w_v, w.b_v, wt->v_w, nullptr, CH}, {w.w_g, w.b_g, wt->g_w, wt->g_b, CH},
-                       {w.w_b, w.b_b, wt->tri_w, nullptr, H}};
+  struct Lin { T* dst; float* bdst; const void* wsrc; const void* bsrc; int out; Pad pad; };
+  const Lin lins[5] = {{w.w_q, w.b_q, wt->q_w, nullptr, CH, heads}, {w.w_k, w.b_k, wt->k_w, nullptr, CH, heads},
+                       {w.w_v, w.b_v, wt->v_w, nullptr, CH, heads}, {w.w_g, w.b_g, wt->g_w, wt->g_b, CH, heads},
+                       {w.w_b, w.b_b, wt->tri_w, nullptr, H, tri}};
   for (const Lin& l : lins) {
-    if ((rc = launch_pack<T>(l.dst, l.wsrc, wd, l.out, C, C, 1, 1.f, st, w.ln_w))) return rc;
-    if ((rc = launch_fold_bias(l.bdst, l.wsrc, l.bsrc, wd, w.ln_b, l.out, C, C, 1, 1.f, st))) return rc;
+    if ((rc = launch_pack<T>(l.dst, l.wsrc, wd, l.out, C, C, 1, 1.f, st, w.ln_w, l.pad))) return rc;
+    if ((rc = launch_fold_bias(l.bdst, l.wsrc, l.bsrc, wd, w.ln_b, l.out, C, C, 1, 1.f, st, l.pad))) return rc;
   }
   T* wts[4] = {w.wt_q, w.wt_k, w.wt_v, w.wt_g};
   const void* srcs[4] = {wt->q_w, wt->k_w, wt->v_w, wt->g_w};
   for (int k = 0; k < 4; ++k)
-    if ((rc = launch_pack_acc<T>(wts[k], srcs[k], wd, C, CH, 1, C, st))) return rc;
-  if ((rc = launch_pack<T>(w.wt_o, wt->o_w, wd, CH, C, 1, CH, 1.f, st))) return rc;
-  if ((rc = launch_to_f32(w.wb_raw, wt->tri_w, wd, H * C, 1.f, 0.f, st))) return rc;
+    if ((rc = launch_pack_acc<T>(wts[k], srcs[k], wd, C, CH, 1, C, st, heads))) return rc;
+  if ((rc = launch_pack<T>(w.wt_o, wt->o_w, wd, CH, C, 1, c_h, 1.f, st, nullptr, heads))) return rc;
+  if ((rc = launch_to_f32(w.wb_raw, wt->tri_w, wd, nh * C, 1.f, 0.f, st))) return rc;
+  if (nh < H && (rc = launch_to_f32(w.wb_raw + nh * C, nullptr, wd, (H - nh) * C, 1.f, 0.f, st))) return rc;
   return batch.flush();
 }
 
 template <typename T, int C, int H>
 static int bwd_triattn(const void* x, const float* mask, const void* dy,
                        const gtk_tri_attn_weights* wts, void* dx, const gtk_tri_attn_grads* gr,
-                       int64_t B, int64_t N, int starting, float eps, void* ws, hipStream_t st) {
+                       int64_t B, int64_t N, int nh, int d, int starting, float eps, void* ws,
+                       hipStream_t st) {
   constexpr int CH = H * AD;
   Carve cv(ws, SIZE_MAX);
   AttnBwdWs<T> a = carve_attn_bwd<T>(cv, B, N, C, H);
   int rc;
-  if ((rc = pack_attn_bwd<T>(wts, a.w, C, H, st))) return rc;
+  if ((rc = pack_attn_bwd<T>(wts, a.w, C, H, nh, d, st))) return rc;
   const int np = (int)round_up(N, 32);
   const int64_t P = B * N * N, pitch = a.b.pitch;
-  const float scale = 1.0f / sqrtf((float)AD);
+  const float scale = 1.0f / sqrtf((float)d);
   const int64_t rowtiles = B * N * (np / 32);
   const int64_t headtiles = B * N * H * (np / 32);
   const int64_t pairtiles = B * H * (int64_t)(np / 32) * (np / 32);
@@ -2099,9 +2070,6 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
     }
     GTK_LAUNCH_CHECK();
   }
-  // rows H..63 of the dtri operand stay zero
-  if ((rc = launch_zero(a.b.cm_dtri + (int64_t)H * pitch, (size_t)(64 - H) * pitch * sizeof(T), st)))
-    return rc;
   {
     StageTimer timer("triattn_bwd_pro", st);
     bool lds = false;
@@ -2123,36 +2091,54 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
     GTK_LAUNCH_CHECK();
   }
   const AttnBwdBufs<T>& b = a.b;
-  if ((rc = launch_zero_tail<T>(b.cm_stack, 4 * CH, pitch, P, st))) return rc;
-  if ((rc = launch_zero_tail<T>(b.cm_xh, C, pitch, P, st))) return rc;
-  if ((rc = launch_zero_tail<T>(b.cm_dy, C, pitch, P, st))) return rc;
-  if ((rc = launch_zero_tail<T>(b.cm_go, CH, pitch, P, st))) return rc;
-  if ((rc = launch_zero_tail<T>(b.cm_dtri, H, pitch, P, st))) return rc;
-  // LayerNorm parameter gradients straight into the outputs where requested
-  auto or_tmp = [](float* dst, float* tmp) { return dst ? dst : tmp; };
-  if ((rc = launch_rowred<T>(b.cm_dxn, b.cm_xh, C, pitch, P, a.red, or_tmp(gr->ln_b, a.sums_dxn),
-                             or_tmp(gr->ln_w, a.dots_dxn), st)))
-    return rc;
-  if ((rc = launch_rowred<T>(b.cm_dtri, nullptr, H, pitch, P, a.red, a.sums_dtri, nullptr, st))) return rc;
+  TailJobs<T> tails;
+  tails.add(b.cm_stack, 4 * CH);
+  tails.add(b.cm_xh, C);
+  tails.add(b.cm_dy, C);
+  tails.add(b.cm_go, CH);
+  tails.add(b.cm_dtri, H);
+  if ((rc = launch_zero_tails<T>(tails, pitch, P, st))) return rc;
+  RowJobs rows;
+  SumJobs sums;
+  add_rowred<T>(rows, sums, b.cm_dxn, b.cm_xh, C, a.red_dxn, gr->ln_b, gr->ln_w);
+  add_rowred<T>(rows, sums, b.cm_dtri, nullptr, H, a.red_dtri, nullptr, nullptr);
+  if ((rc = launch_rowred<T>(rows, pitch, P, st))) return rc;
   // the weight-gradient products also sum their G rows: the bias gradients
   {
     StageTimer timer("triattn_bwd_wgrad", st);
-    if ((rc = launch_wgrad<T>(b.cm_stack, b.cm_xh, a.part1, 4 * CH, C, pitch, st, a.rs, a.sums_stack))) return rc;
-    if ((rc = launch_wgrad<T>(b.cm_dy, b.cm_go, a.part2, C, CH, pitch, st, a.rs, or_tmp(gr->o_b, a.sums_dy))))
-      return rc;
-    if ((rc = launch_wgrad<T>(b.cm_xh, b.cm_dtri, a.part3, C, 64, pitch, st))) return rc;
+    if ((rc = launch_wgrad<T>(b.cm_stack, b.cm_xh, a.part1, 4 * CH, C, pitch, st, a.rs1))) return rc;
+    if ((rc = launch_wgrad<T>(b.cm_dy, b.cm_go, a.part2, C, CH, pitch, st, a.rs2))) return rc;
+    // (the operand's rows from H on are whatever the workspace held: their outputs are never read)
+    if ((rc = launch_wgrad<T>(b.cm_xh, b.cm_dtri, a.part3, C, H, pitch, st))) return rc;
   }
+  const Pad heads{AD, d, kNoPad};
   float* wdst[4] = {gr->q_w, gr->k_w, gr->v_w, gr->g_w};
-  WgradSegs wsegs;
-  for (int k = 0; k < 4; ++k) wsegs.add(wdst[k], k * CH, CH);
-  if ((rc = launch_wgrad_finish(a.part1, 4 * CH, C, pitch, wsegs, a.sums_stack, a.w.ln_w, a.w.ln_b, st)))
-    return rc;
-  if ((rc = launch_copy_f32(gr->g_b, a.sums_stack + 3 * CH, CH, st))) return rc;
-  if ((rc = launch_wgrad_finish(a.part2, C, CH, pitch, 0, C, nullptr, nullptr, nullptr, gr->o_w, st)))
-    return rc;
-  attn_dwb_finish_kernel<<<(H * C + 7) / 8, 256, 0, st>>>(
-      a.part3, wgrad_plan(C, pitch).nsplit, C, wgrad_m_rows(C), H, a.w.ln_w, a.w.ln_b, a.sums_dtri, gr->tri_w);
-  GTK_LAUNCH_CHECK();
+  for (int k = 0; k < 4; ++k) {
+    SumJob j = with_affine(sum_of_product(wdst[k], a.part1, 4 * CH, C, pitch, k * CH, nh * d), a.w.ln_w, a.w.ln_b,
+                           a.rs1, 4 * CH, pitch, k * CH);
+    j.row = heads;
+    sums.add(j);
+  }
+  SumJob gb = sum_of_rows(gr->g_b, a.rs1, 4 * CH, pitch, 3 * CH, nh * d);
+  gb.row = heads;
+  sums.add(gb);
+  SumJob ow = sum_of_product(gr->o_w, a.part2, C, CH, pitch, 0, C);
+  ow.cols = nh * d;
+  ow.col = heads;
+  sums.add(ow);
+  sums.add(sum_of_rows(gr->o_b, a.rs2, C, pitch, 0, C));
+  // dW_b[h][c] = W3[c][h] gamma[c] + s[h] beta[c]: the product transposed
+  SumJob tw = sum_of_product(gr->tri_w, a.part3, C, H, pitch, 0, nh);
+  tw.sn = tw.sm;
+  tw.sm = 1;
+  tw.cols = C;
+  tw.gamma = a.w.ln_w;
+  tw.beta = a.w.ln_b;
+  tw.rs = a.red_dtri;
+  tw.rs_step = 1;
+  tw.rs_m = tw.rs_n = rowred_segs(H);
+  sums.add(tw);
+  if ((rc = launch_grad_sums(sums, st))) return rc;
   return GTK_OK;
 }
 
@@ -2169,11 +2155,12 @@ static bool attn_bwd_shape_ok(int64_t c_in, int64_t c_h, int64_t H) {
 template <typename T>
 static int bwd_triattn_any(int64_t c_in, const void* x, const float* mask, const void* dy,
                            const gtk_tri_attn_weights* w, void* dx, const gtk_tri_attn_grads* grads,
-                           int64_t B, int64_t N, int starting, float eps, void* ws, hipStream_t st) {
+                           int64_t B, int64_t N, int nh, int d, int starting, float eps, void* ws,
+                           hipStream_t st) {
   switch (c_in) {
-    case 32: return bwd_triattn<T, 32, 4>(x, mask, dy, w, dx, grads, B, N, starting, eps, ws, st);
-    case 64: return bwd_triattn<T, 64, 4>(x, mask, dy, w, dx, grads, B, N, starting, eps, ws, st);
-    default: return bwd_triattn<T, 128, 4>(x, mask, dy, w, dx, grads, B, N, starting, eps, ws, st);
+    case 32: return bwd_triattn<T, 32, 4>(x, mask, dy, w, dx, grads, B, N, nh, d, starting, eps, ws, st);
+    case 64: return bwd_triattn<T, 64, 4>(x, mask, dy, w, dx, grads, B, N, nh, d, starting, eps, ws, st);
+    default: return bwd_triattn<T, 128, 4>(x, mask, dy, w, dx, grads, B, N, nh, d, starting, eps, ws, st);
   }
 }
 
@@ -2187,6 +2174,27 @@ extern "C" size_t gtk_tri_attn_backward_workspace_size(int64_t B, int64_t N, int
   return cv.off;
 }
 
+// The checks that both entries share, then the pass.
+static int attn_bwd_entry(const char* name, const void* x, const float* mask, const void* dy,
+                          const gtk_tri_attn_weights* w, void* dx, const gtk_tri_attn_grads* grads, int64_t B,
+                          int64_t N, int64_t c_in, int nh, int d, int starting, float eps, int dtype, void* ws,
+                          size_t ws_bytes, void* stream) {
+  GTK_REQUIRE(B >= 0 && N >= 0 && N <= 4096, GTK_EINVAL, "%s: bad shape", name);
+  if (B == 0 || N == 0) return GTK_OK;
+  GTK_REQUIRE(x && dy && w && dx && grads && ws, GTK_EINVAL, "%s: null pointer", name);
+  GTK_REQUIRE(w->dtype == GTK_F32 || w->dtype == GTK_BF16, GTK_EINVAL, "%s: bad weight dtype %d", name, w->dtype);
+  GTK_REQUIRE(w->tri_w && w->q_w && w->k_w && w->v_w && w->g_w && w->o_w, GTK_EINVAL, "%s: null weight", name);
+  const float* gp[] = {grads->ln_w, grads->ln_b, grads->tri_w, grads->q_w, grads->k_w,
+                       grads->v_w,  grads->g_w,  grads->g_b,   grads->o_w, grads->o_b};
+  for (const float* p : gp) GTK_REQUIRE(p, GTK_EINVAL, "%s: null gradient pointer", name);
+  const size_t need = gtk_tri_attn_backward_workspace_size(B, N, c_in, 4 * AD, 4, dtype);
+  GTK_REQUIRE(ws_bytes >= need, GTK_EWORKSPACE, "%s: workspace %zu < %zu bytes", name, ws_bytes, need);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == GTK_F32)
+    return bwd_triattn_any<float>(c_in, x, mask, dy, w, dx, grads, B, N, nh, d, starting, eps, ws, st);
+  return bwd_triattn_any<bf16>(c_in, x, mask, dy, w, dx, grads, B, N, nh, d, starting, eps, ws, st);
+}
+
 extern "C" int gtk_tri_attn_backward(const void* x, const float* mask, const void* dy,
                                      const gtk_tri_attn_weights* w, void* dx,
                                      const gtk_tri_attn_grads* grads, int64_t B, int64_t N,
@@ -2197,20 +2205,23 @@ extern "C" int gtk_tri_attn_backward(const void* x, const float* mask, const voi
   GTK_REQUIRE(attn_bwd_shape_ok(c_in, c_h, H), GTK_EUNSUPPORTED,
               "gtk_tri_attn_backward: c_in=%lld c_h=%lld H=%lld unsupported (c_in in {32, 64, 128}, H=4, d=32)",
               (long long)c_in, (long long)c_h, (long long)H);
-  GTK_REQUIRE(B >= 0 && N >= 0 && N <= 4096, GTK_EINVAL, "gtk_tri_attn_backward: bad shape");
-  if (B == 0 || N == 0) return GTK_OK;
-  GTK_REQUIRE(x && dy && w && dx && grads && ws, GTK_EINVAL, "gtk_tri_attn_backward: null pointer");
-  GTK_REQUIRE(w->dtype == GTK_F32 || w->dtype == GTK_BF16, GTK_EINVAL,
-              "gtk_tri_attn_backward: bad weight dtype %d", w->dtype);
-  GTK_REQUIRE(w->tri_w && w->q_w && w->k_w && w->v_w && w->g_w && w->o_w, GTK_EINVAL,
-              "gtk_tri_attn_backward: null weight");
-  const float* gp[] = {grads->ln_w, grads->ln_b, grads->tri_w, grads->q_w, grads->k_w,
-                       grads->v_w,  grads->g_w,  grads->g_b,   grads->o_w, grads->o_b};
-  for (const float* p : gp) GTK_REQUIRE(p, GTK_EINVAL, "gtk_tri_attn_backward: null gradient pointer");
-  const size_t need = gtk_tri_attn_backward_workspace_size(B, N, c_in, c_h, H, dtype);
-  GTK_REQUIRE(ws_bytes >= need, GTK_EWORKSPACE, "gtk_tri_attn_backward: workspace %zu < %zu bytes",
-              ws_bytes, need);
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == GTK_F32) return bwd_triattn_any<float>(c_in, x, mask, dy, w, dx, grads, B, N, starting, eps, ws, st);
-  return bwd_triattn_any<bf16>(c_in, x, mask, dy, w, dx, grads, B, N, starting, eps, ws, st);
+  return attn_bwd_entry("gtk_tri_attn_backward", x, mask, dy, w, dx, grads, B, N, c_in, (int)H, AD, starting, eps,
+                        dtype, ws, ws_bytes, stream);
+}
+
+extern "C" int gtk_tri_attn_backward_heads(const void* x, const float* mask, const void* dy,
+                                           const gtk_tri_attn_weights* w, void* dx,
+                                           const gtk_tri_attn_grads* grads, int64_t B, int64_t N, int64_t c_in,
+                                           int64_t c_h, int64_t H, int starting, float eps, int dtype, void* ws,
+                                           size_t ws_bytes, void* stream) {
+  GTK_REQUIRE(dtype == GTK_F32 || dtype == GTK_BF16, GTK_EINVAL,
+              "gtk_tri_attn_backward_heads: bad dtype %d", dtype);
+  GTK_REQUIRE((H == 1 || H == 2 || H == 4) && c_h >= H && c_h % H == 0 && c_h / H <= AD &&
+                  attn_bwd_shape_ok(c_in, 4 * AD, 4),
+              GTK_EUNSUPPORTED,
+              "gtk_tri_attn_backward_heads: c_in=%lld c_h=%lld H=%lld unsupported (c_in in {32, 64, 128}, H in "
+              "{1, 2, 4}, d <= 32)",
+              (long long)c_in, (long long)c_h, (long long)H);
+  return attn_bwd_entry("gtk_tri_attn_backward_heads", x, mask, dy, w, dx, grads, B, N, c_in, (int)H,
+                        (int)(c_h / H), starting, eps, dtype, ws, ws_bytes, stream);
 }

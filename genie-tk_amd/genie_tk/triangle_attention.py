@@ -9,7 +9,7 @@ Kernel path (``use_fused_kernel=True``, GPU tensor):
 triangle-bias projections on the matrix cores) and a flash-style kernel
 (online softmax, bias streamed from HBM, gate and output projection fused).
 When autograd needs gradients the same forward runs inside
-``_TriAttnFunction``, whose backward is ``genie_tk._C.tri_attn_backward``.
+``_TriAttnFunction``, whose backward is ``genie_tk._C.tri_attn_backward_heads``.
 PyTorch path: ``_forward_pytorch``, the reference fallback semantics
 (triangle_attention.py:100-143).
 
@@ -52,7 +52,9 @@ def _pad_heads(params, H: int, ch: int):
     1/sqrt(d).  The zero channels and heads add nothing to the output (their
     v and their W_o columns are zero), so the padded module's gradients
     restricted to the real parameters are the module's own.  Returns the
-    padded list and the channel index of the real ones."""
+    padded list and the channel index of the real ones.  (The kernels pad in
+    their packing, with the score scale of the real heads in place of the
+    scaled W_q; this is the same map in PyTorch.)"""
     ln_w, ln_b, tri_w, q_w, k_w, v_w, g_w, g_b, o_w, o_b = params
     d = ch // H
     idx = (torch.arange(H, device=q_w.device)[:, None] * HD_BWD
@@ -81,7 +83,9 @@ class _TriAttnFunction(torch.autograd.Function):
     same gradients on the kernels.  Activations are recomputed in the backward
     from x (only x, the mask and the parameters are saved).  Modules with
     fewer than four heads, or heads narrower than 32 channels, run the
-    backward on their weights padded to four heads of 32 (_pad_heads)."""
+    backward on their weights padded to four heads of 32 as _pad_heads
+    describes; the kernels' packing and closing sums do that on the fly (in
+    PyTorch it took some 20 launches, 70 us a call)."""
 
     @staticmethod
     def forward(ctx, module, x, mask, chunk_size, *params):
@@ -94,24 +98,11 @@ class _TriAttnFunction(torch.autograd.Function):
         x, mask, *params = ctx.saved_tensors
         mod = ctx.module
         xb, mb, lead = _dispatch.flatten_batch(x, mask)
-        padded = (mod.no_heads, mod.c_hidden) != (H_BWD, H_BWD * HD_BWD)
-        bparams = list(params)
-        if padded:
-            with torch.no_grad():
-                bparams, idx, scale = _pad_heads(params, mod.no_heads, mod.c_hidden)
-        res = _ext.require().tri_attn_backward(
-            xb, mb, dy.reshape(xb.shape).to(x.dtype), bparams, mod.c_in, H_BWD * HD_BWD,
-            H_BWD, mod.starting, mod.layer_norm.eps)
+        res = _ext.require().tri_attn_backward_heads(
+            xb, mb, dy.reshape(xb.shape).to(x.dtype), params, mod.c_in, mod.c_hidden,
+            mod.no_heads, mod.starting, mod.layer_norm.eps)
         dx = res[0].reshape(x.shape) if ctx.needs_input_grad[1] else None
         g, flat = list(res[1:-1]), res[-1]
-        if padded:
-            flat = None
-            # back to the module's parameters (order of _PARAMS)
-            g[2] = g[2][:mod.no_heads]
-            g[3] = g[3][idx] * scale
-            for k in (4, 5, 6, 7):
-                g[k] = g[k][idx]
-            g[8] = g[8][:, idx]
         g = _dispatch.grads_as_params(g, flat, params)
         grads = [gk if ctx.needs_input_grad[4 + k] else None for k, gk in enumerate(g)]
         return (None, dx, None, None, *grads)

@@ -311,12 +311,12 @@ int gtk_tri_attn_forward_chunked(const void* x, const float* mask, void* out, co
  * forward gives them the bias inf * (mask - 1), which this backward does
  * not model, so callers must send such masks elsewhere (the genie_tk
  * modules use autograd of their PyTorch path for them).  c_in in
- * {32, 64, 128}, H == 4, d == 32 (c_h == 128), N <= 4096.  Other head
- * shapes (the reference layer's default of four heads of 8, two heads of 8)
- * are computed here by padding: zero q/k/v/gate/output weight columns up
- * to four heads of 32, W_q scaled by sqrt(32 / d) so the scores keep
- * their 1/sqrt(d), the triangle bias of the missing heads zero, and the
- * padded gradients dropped (genie_tk.triangle_attention does this). */
+ * {32, 64, 128}, H == 4, d == 32 (c_h == 128), N <= 4096.
+ * gtk_tri_attn_backward_heads takes every head shape of the forward kernels
+ * (H in {1, 2, 4}, d = c_h / H <= 32; the reference layer's default is four
+ * heads of 8) with weights and gradients in the module's own shapes: the
+ * packing pads them to four heads of 32 whose extra weights are zero.  Its
+ * workspace is that of c_h = 128, H = 4. */
 typedef struct gtk_tri_attn_grads {
   float *ln_w, *ln_b, *tri_w, *q_w, *k_w, *v_w, *g_w, *g_b, *o_w, *o_b;
 } gtk_tri_attn_grads;
@@ -328,6 +328,11 @@ int gtk_tri_attn_backward(const void* x, const float* mask, const void* dy,
                           int64_t B, int64_t N, int64_t c_in, int64_t c_h, int64_t H, int starting,
                           float eps, int dtype, void* workspace, size_t workspace_bytes,
                           void* stream);
+int gtk_tri_attn_backward_heads(const void* x, const float* mask, const void* dy,
+                                const gtk_tri_attn_weights* w, void* dx, const gtk_tri_attn_grads* grads,
+                                int64_t B, int64_t N, int64_t c_in, int64_t c_h, int64_t H, int starting,
+                                float eps, int dtype, void* workspace, size_t workspace_bytes,
+                                void* stream);
 
 /* ------------------------------------------------------------------------
  * PairTransition fused with the pair-stack residual and mask.
