@@ -1249,8 +1249,18 @@ __global__ __launch_bounds__(64 * kRhWaves) __attribute__((amdgpu_waves_per_eu(4
 // (b, chunk, head) are consecutive, so the blocks that read the same K and V
 // rows share an XCD's L2.  Two query tiles a block halve the K/V bytes moved
 // per unit of work and make the launch one round of blocks at N = 512.
-constexpr int kDbChunks = 8;  // row chunks per batch element (at most)
-constexpr int kDbQt = 2;      // query tiles per block
+constexpr int kDbQt = 2;  // query tiles per block
+
+// Row chunks per batch element.  A block's two buffers of a row leave room for
+// one block a CU (two at np <= 128), so as many chunks as make one block a CU:
+// 8 at N = 512, 16 at N = 250 (with 8, 128 blocks, 70 us; with 16, 41 us and 2
+// us more in the reduction; N = 384, 8 -> 10: 118 -> 101).  At most 16: 32 at N
+// = 128 took 11 + 12 us for the sums and the reduction against 26 + 5 with 8.
+inline int dbias_rh_chunks(int64_t B, int64_t N, int H) {
+  const int64_t blocks = B * H * (((N + 31) / 32 + kDbQt - 1) / kDbQt);
+  const int64_t want = std::min<int64_t>(std::max<int64_t>(256 / blocks, 8), 16);
+  return (int)std::min<int64_t>(want, std::max<int64_t>((N + 3) / 4, 8));
+}
 
 template <int NPM>
 __global__ __launch_bounds__(64 * kRhWaves) void attn_bwd_dbias_rh_kernel(AttnBwdBufs<bf16> bf,
@@ -1503,15 +1513,25 @@ __global__ __launch_bounds__(256) void attn_bwd_dbias_reduce_kernel(const float*
 
 // ---------------------------------------------------------------------------
 // pro: dxn and the LayerNorm backward; per 32-position tile of one row
+//
+// SPLIT (fp32): a block's four waves share a tile.  Wave k takes the products
+// of kind k (q, k, v or gate), the partial dxn meet in LDS, and wave k finishes
+// channel tile k: a quarter of the serial chain, where one wave a tile leaves
+// SIMDs without a wave.  Up to 5 tiles a CU (kProSplitPerCu): N = 64 62 -> 22
+// us, N = 128 64 -> 45, N = 192 (1152 tiles) 137 -> 107; with 2048 tiles (N =
+// 256) the exchange and the repeated statistics cost more, 150 -> 173.
 // ---------------------------------------------------------------------------
-template <typename T, int C, int H>
+constexpr int kProSplitPerCu = 5;
+
+template <typename T, int C, int H, bool SPLIT>
 __global__ __launch_bounds__(256) void attn_bwd_pro_kernel(const T* __restrict__ x, T* __restrict__ dx,
                                                            AttnBwdW<T> w, AttnBwdBufs<T> bf, int B,
                                                            int N, int np, int starting, float eps) {
   constexpr int CH = H * AD;
   const int lane = threadIdx.x & 63, half = lane >> 5, t32 = lane & 31;
   const int jtiles = np / 32;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + wave_id();
+  const int wave = wave_id();
+  const int64_t tile = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
   if (tile >= (int64_t)B * N * jtiles) return;
   const int jt = (int)(tile % jtiles);
   const int r = (int)((tile / jtiles) % N);
@@ -1536,7 +1556,7 @@ __global__ __launch_bounds__(256) void attn_bwd_pro_kernel(const T* __restrict__
   const T* src[3] = {bf.dq, bf.dk, bf.dv};
   const T* wts[4] = {w.wt_q, w.wt_k, w.wt_v, w.wt_g};
 #pragma unroll 1
-  for (int kind = 0; kind < 4; ++kind) {
+  for (int kind = SPLIT ? wave : 0; kind < (SPLIT ? wave + 1 : 4); ++kind) {
 #pragma unroll 1
     for (int h = 0; h < H; ++h) {
       // this (kind, head)'s weight fragments first: their loads overlap the operand loads
@@ -1585,20 +1605,35 @@ __global__ __launch_bounds__(256) void attn_bwd_pro_kernel(const T* __restrict__
         for (int gp = 0; gp < 2; ++gp) mma(dzn[nt2], wf[nt2][gp], f[gp]);
     }
   }
+  // the channel tiles that this wave finishes: dzn[i] is tile ct(i)
+  constexpr int NT = SPLIT ? 1 : C / 32;
+  const bool act = !SPLIT || wave < C / 32;
+  auto ct = [&](int nt) { return SPLIT ? (act ? wave : 0) : nt; };
+  if constexpr (SPLIT) {
+    __shared__ float red[4][C / 32][16][64];
+#pragma unroll
+    for (int nt = 0; nt < C / 32; ++nt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) red[wave][nt][e][lane] = dzn[nt][e];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      dzn[0][e] = (red[0][ct(0)][e][lane] + red[1][ct(0)][e][lane]) + (red[2][ct(0)][e][lane] + red[3][ct(0)][e][lane]);
+  }
   // triangle bias: dxn += sum_h dB[h][r][j] W_b[h][.]
   float dtri[H];
 #pragma unroll
   for (int h = 0; h < H; ++h) {
     dtri[h] = valid ? bf.db[(((int64_t)b * H + h) * N + r) * N + j] : 0.f;
-    if (valid && half == 0) bf.cm_dtri[(int64_t)h * pitch + p] = cvt<T>(dtri[h]);
+    if (valid && half == 0 && (!SPLIT || wave == 0)) bf.cm_dtri[(int64_t)h * pitch + p] = cvt<T>(dtri[h]);
   }
-  float xh[C / 2];
+  float xh[NT * 16];
   float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-  for (int nt = 0; nt < C / 32; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const int c0 = nt * 32 + 8 * g + 4 * half;
+      const int c0 = ct(nt) * 32 + 8 * g + 4 * half;
       const f32x4 x4 = valid ? load4f(x + xp * C + c0) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -1615,10 +1650,20 @@ __global__ __launch_bounds__(256) void attn_bwd_pro_kernel(const T* __restrict__
     }
   s1 += xor32(s1);
   s2 += xor32(s2);
+  if constexpr (SPLIT) {
+    __shared__ float sums[4][2][32];
+    if (half == 0) {
+      sums[wave][0][t32] = act ? s1 : 0.f;
+      sums[wave][1][t32] = act ? s2 : 0.f;
+    }
+    __syncthreads();
+    s1 = (sums[0][0][t32] + sums[1][0][t32]) + (sums[2][0][t32] + sums[3][0][t32]);
+    s2 = (sums[0][1][t32] + sums[1][1][t32]) + (sums[2][1][t32] + sums[3][1][t32]);
+  }
   const float m1 = s1 * (1.0f / C), m2 = s2 * (1.0f / C);
   if constexpr (std::is_same<T, bf16>::value) {
 #pragma unroll
-    for (int nt = 0; nt < C / 32; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       float vt[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) vt[e] = dzn[nt][e];
@@ -1626,12 +1671,12 @@ __global__ __launch_bounds__(256) void attn_bwd_pro_kernel(const T* __restrict__
       cmt.store(bf.cm_dxn, pitch, p0, nt * 32, vt, fast, valid);
     }
   }
-  if (!valid) return;
+  if (!valid || !act) return;
 #pragma unroll
-  for (int nt = 0; nt < C / 32; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const int c0 = nt * 32 + 8 * g + 4 * half;
+      const int c0 = ct(nt) * 32 + 8 * g + 4 * half;
       float o[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -1878,7 +1923,7 @@ static AttnBwdWs<T> carve_attn_bwd(Carve& cv, int64_t B, int64_t N, int C, int H
   b.dd = cv.take<float>(B * N * H * np);
   b.db = cv.take<float>(B * H * N * N);
   const int nch = dbias_row_chunks(B, N, H);
-  b.dbp = (sizeof(T) == 2 && np <= 512) ? cv.take<float>(B * kDbChunks * H * np * np)
+  b.dbp = (sizeof(T) == 2 && np <= 512) ? cv.take<float>(B * dbias_rh_chunks(B, N, H) * H * np * np)
                                         : cv.take<float>(nch > 1 ? nch * B * H * N * N : 0);
   b.pitch = round_up(B * N * N, 64);
   // operands of the weight-gradient products: rows padded to their tiles
@@ -2042,9 +2087,10 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
     StageTimer timer("triattn_bwd_dbias", st);
     if (std::is_same<T, bf16>::value && np <= 512) {
       if constexpr (std::is_same<T, bf16>::value) {
-        // row chunks of rpc rows (at most kDbChunks per batch element), partial
-        // sums in fragment order, then the sum over the chunks
-        const int rpc = (int)((N + kDbChunks - 1) / kDbChunks);
+        // row chunks of rpc rows, partial sums in fragment order, then the sum
+        // over the chunks
+        const int chunks = dbias_rh_chunks(B, N, H);
+        const int rpc = (int)((N + chunks - 1) / chunks);
         const int nch = (int)((N + rpc - 1) / rpc);
         const int64_t dblocks = B * nch * H * (((N + 31) / 32 + kDbQt - 1) / kDbQt);
         GTK_REQUIRE(dblocks < (1ll << 31), GTK_EUNSUPPORTED, "attention backward grid too large");
@@ -2085,9 +2131,15 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
         lds = true;
       }
     }
-    if (!lds)
-      attn_bwd_pro_kernel<T, C, H><<<g4(rowtiles), 256, 0, st>>>((const T*)x, (T*)dx, a.w, a.b,
-                                                                  (int)B, (int)N, np, starting, eps);
+    if (!lds) {
+      auto go = [&](auto kern, unsigned grid) {
+        kern<<<grid, 256, 0, st>>>((const T*)x, (T*)dx, a.w, a.b, (int)B, (int)N, np, starting, eps);
+      };
+      if (sizeof(T) == 4 && rowtiles <= kProSplitPerCu * (int64_t)device_cus())
+        go(attn_bwd_pro_kernel<T, C, H, sizeof(T) == 4>, (unsigned)rowtiles);
+      else
+        go(attn_bwd_pro_kernel<T, C, H, false>, g4(rowtiles));
+    }
     GTK_LAUNCH_CHECK();
   }
   const AttnBwdBufs<T>& b = a.b;
