@@ -358,7 +358,12 @@ __global__ __launch_bounds__(512) void trimul_prologue_bf16_kernel(
 // 2. Per-channel contraction  X = A . Bm^T   (Bm: [Np][Np] planes; A, X:
 //    [Mi][Np], Mi = Np for whole planes, fewer rows for a row chunk)
 // ---------------------------------------------------------------------------
-template <typename T, int TILE>
+// LT / RT: the operand is given transposed, as the plane L^T [k][i] (R^T
+// [k][j]) of whole Np x Np planes, as in the bf16 tile kernel below: its stage
+// sits in LDS as 64 k rows and its fragments come from transposing reads.  (N =
+// 301: forward + backward 568 -> 527 us without the three plane transposes of the
+// contraction backward.)
+template <typename T, int TILE, bool LT = false, bool RT = false>
 __global__ __launch_bounds__(256) void trimul_contract_kernel(const T* __restrict__ pa,
                                                               const T* __restrict__ pb,
                                                               T* __restrict__ px, int Np, int Mi,
@@ -371,6 +376,8 @@ __global__ __launch_bounds__(256) void trimul_contract_kernel(const T* __restric
   constexpr int CHUNKS = TILE * 8;               // 16-byte chunks per operand per stage
   constexpr int CPT = CHUNKS / 256;              // chunks per thread per operand
   constexpr int EPC = 16 / sizeof(T);            // elements per 16-byte chunk
+  // a transposed operand's stage is BK rows of TILE columns: the same LDS shape
+  static_assert((!LT && !RT) || (sizeof(T) == 2 && TILE == BK), "transposed operands: bf16, 64 x 64 tiles");
   __shared__ __attribute__((aligned(16))) char smem[2][2][TILE * PITCH];
 
   const int ti_n = Mi / TILE, tj_n = Np / TILE;
@@ -402,8 +409,10 @@ __global__ __launch_bounds__(256) void trimul_contract_kernel(const T* __restric
     for (int u = 0; u < CPT; ++u) {
       const int id = tid + 256 * u;
       const int row = id >> 3, cc = id & 7;
-      ra[u] = *reinterpret_cast<const f32x4*>(A + (int64_t)(i0 + row) * Np + k0 + cc * EPC);
-      rb[u] = *reinterpret_cast<const f32x4*>(Bm + (int64_t)(j0 + row) * Np + k0 + cc * EPC);
+      const T* sa = LT ? A + (int64_t)(k0 + row) * Np + i0 : A + (int64_t)(i0 + row) * Np + k0;
+      const T* sb = RT ? Bm + (int64_t)(k0 + row) * Np + j0 : Bm + (int64_t)(j0 + row) * Np + k0;
+      ra[u] = *reinterpret_cast<const f32x4*>(sa + cc * EPC);
+      rb[u] = *reinterpret_cast<const f32x4*>(sb + cc * EPC);
     }
   };
   auto sstore = [&](int buf) {
@@ -414,6 +423,19 @@ __global__ __launch_bounds__(256) void trimul_contract_kernel(const T* __restric
       *reinterpret_cast<f32x4*>(&smem[buf][0][row * PITCH + cc * 16]) = ra[u];
       *reinterpret_cast<f32x4*>(&smem[buf][1][row * PITCH + cc * 16]) = rb[u];
     }
+  };
+
+  // fragment of a transposed panel (64 k rows): lane l takes column c0 + (l & 31),
+  // k 16 kc + 8 (l >> 5) .. +7, from two transposing reads (see the bf16 tile
+  // kernel)
+  auto tfrag = [&](Frag<T>& f, const char* panel, int c0, int kc) {
+    const int G = lane >> 4, sl = lane & 15;
+    const int col = c0 + 16 * (G & 1) + 4 * (sl & 3);
+    const char* at = panel + (16 * kc + 8 * (G >> 1) + (sl >> 2)) * PITCH + col * 2;
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const s16x4 p0 = lds_read_tr16(at), p1 = lds_read_tr16(at + 4 * PITCH);
+    if constexpr (sizeof(T) == 2)
+      f.v = __builtin_bit_cast(bf16x8, s16x8{p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]});
   };
 
   const int KT = Np / BK;
@@ -432,8 +454,10 @@ __global__ __launch_bounds__(256) void trimul_contract_kernel(const T* __restric
         const int ra_row = wi + x * 32 + (lane & 31);
         const int rb_row = wj + x * 32 + (lane & 31);
         const int koff = (kc * 16 + half * 8) * (int)sizeof(T);
-        fa[x].load(reinterpret_cast<const T*>(&smem[cur][0][ra_row * PITCH + koff]));
-        fb[x].load(reinterpret_cast<const T*>(&smem[cur][1][rb_row * PITCH + koff]));
+        if constexpr (LT) tfrag(fa[x], smem[cur][0], wi + x * 32, kc);
+        else fa[x].load(reinterpret_cast<const T*>(&smem[cur][0][ra_row * PITCH + koff]));
+        if constexpr (RT) tfrag(fb[x], smem[cur][1], wj + x * 32, kc);
+        else fb[x].load(reinterpret_cast<const T*>(&smem[cur][1][rb_row * PITCH + koff]));
       }
 #pragma unroll
       for (int x = 0; x < MB; ++x)
@@ -1534,14 +1558,10 @@ int trimul_contract_planes(const void* pl, const void* pr, void* out, int Np, in
   return launch_contract<bf16>((const bf16*)pl, (const bf16*)pr, (bf16*)out, Np, nplanes, st);
 }
 
-bool trimul_contract_t_ok(int Np, int64_t nplanes, int dtype) {
-  return dtype != GTK_F32 && contract_tile<bf16>(Np, nplanes) >= 128;
-}
+bool trimul_contract_t_ok(int dtype) { return dtype != GTK_F32; }
 
 int trimul_contract_planes_t(const void* pl, const void* pr, void* out, int Np, int64_t nplanes, bool lt,
                              bool rt, hipStream_t st) {
-  GTK_REQUIRE(trimul_contract_t_ok(Np, nplanes, GTK_BF16), GTK_EUNSUPPORTED,
-              "transposed-operand contraction: Np %d", Np);
   const int tile = contract_tile<bf16>(Np, nplanes);
   const int64_t blocks = (int64_t)(Np / tile) * (Np / tile) * nplanes;
   GTK_REQUIRE(blocks < (1ll << 31), GTK_EUNSUPPORTED, "contraction grid too large");
@@ -1558,6 +1578,11 @@ int trimul_contract_planes_t(const void* pl, const void* pr, void* out, int Np, 
     else if (lt) go(trimul_contract_bf16_kernel<256, 256, true, false>, 1024, device_cus());
     else if (rt) go(trimul_contract_bf16_kernel<256, 256, false, true>, 1024, device_cus());
     else go(trimul_contract_bf16_kernel<256, 256>, 1024, device_cus());
+  } else if (tile == 64) {
+    if (lt && rt) go(trimul_contract_kernel<bf16, 64, true, true>, 256, blocks);
+    else if (lt) go(trimul_contract_kernel<bf16, 64, true, false>, 256, blocks);
+    else if (rt) go(trimul_contract_kernel<bf16, 64, false, true>, 256, blocks);
+    else go(trimul_contract_kernel<bf16, 64>, 256, blocks);
   } else {
     if (lt && rt) go(trimul_contract_bf16_kernel<128, 128, true, true>, 256, 2 * device_cus());
     else if (lt) go(trimul_contract_bf16_kernel<128, 128, true, false>, 256, 2 * device_cus());

@@ -881,14 +881,14 @@ template <typename T> struct TriMulBwdWs {
   int64_t pitch;
 };
 
-// Does the contraction backward transpose its planes first?  Only where the
-// tile kernels cannot read the operands transposed, or when the test switch
+// Does the contraction backward transpose its planes first?  Only in fp32,
+// whose kernels cannot read the operands transposed, or when the test switch
 // GENIE_TK_TRANSPOSE_PLANES=1 asks for it (the transposed planes then take
 // workspace).
-static bool trimul_bwd_transposes(int64_t B, int64_t N, int c, int dtype) {
+static bool trimul_bwd_transposes(int dtype) {
   const char* tp = std::getenv("GENIE_TK_TRANSPOSE_PLANES");
   if (tp && tp[0] == '1') return true;
-  return !trimul_contract_t_ok((int)round_up(N, 64), B * c, dtype);
+  return !trimul_contract_t_ok(dtype);
 }
 
 template <typename T>
@@ -906,7 +906,7 @@ static TriMulBwdWs<T> carve_trimul_bwd(Carve& cv, int64_t B, int64_t N, int cz, 
   T** planes[] = {&w.pa, &w.pb, &w.px, &w.pdx, &w.pda, &w.pdb};
   for (T** p : planes) *p = cv.take<T>(pe);
   w.pat = w.pbt = nullptr;
-  if (trimul_bwd_transposes(B, N, c, dtype)) {
+  if (trimul_bwd_transposes(dtype)) {
     w.pat = cv.take<T>(pe);
     w.pbt = cv.take<T>(pe);
   }
@@ -1002,7 +1002,7 @@ static int bwd_trimul(const void* z, const float* mask, const void* dy,
   }
   // 3. contraction backward.  Outgoing: dA = dX Bm, dB = dX^T A; incoming
   // (planes stored so that X = A Bm^T as well): dA^T = Bm^T dX, dB^T =
-  // A^T dX^T.  The bf16 tile kernels read the operands that enter
+  // A^T dX^T.  The bf16 kernels read the operands that enter
   // transposed straight from the planes (trimul_contract_planes_t);
   // otherwise the planes are transposed first (px is free from here on: it
   // takes dX^T).  GENIE_TK_TRANSPOSE_PLANES=1 selects the transposing form

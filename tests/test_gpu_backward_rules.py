@@ -1,0 +1,54 @@
+"""The backward kernels on both sides of the rules that choose between their
+forms: the same gradients either way."""
+import pytest
+import torch
+
+from tests import helpers as H
+from tests.gpu_common import trimul_module, triattn_module
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(B, N, dt, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(1, N, N, 128, generator=gen, device="cuda").to(dt)
+    dy = torch.randn(1, N, N, 128, generator=gen, device="cuda").to(dt)
+    m = torch.ones(1, N, N, device="cuda")
+    m[:, N - 5:] = 0
+    m[:, :, N - 5:] = 0
+    return (t.expand(B, *t.shape[1:]).contiguous() for t in (x, dy, m))
+
+
+@pytest.mark.parametrize("outgoing", [True, False])
+@pytest.mark.parametrize("B,N", [(1, 33), (2, 50), (1, 150), (1, 301)])
+def test_contraction_backward_on_64_tiles(monkeypatch, outgoing, B, N):
+    """Planes of an odd multiple of 64: operands read transposed give the bits
+    of planes transposed first (the same products in the same order)."""
+    mod = trimul_module(H.draw_params(H.tri_mul_shapes(128, 128), seed=N, bias_random=True), outgoing,
+                        torch.bfloat16)
+    x, dy, m = _inputs(B, N, torch.bfloat16, N)
+    x.requires_grad_()
+    runs = []
+    for force in ("0", "1"):
+        monkeypatch.setenv("GENIE_TK_TRANSPOSE_PLANES", force)
+        runs.append(torch.autograd.grad(mod(x, m), [x, *mod.parameters()], dy))
+    for a, b in zip(*runs):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("starting", [True, False])
+def test_attention_backward_split_tiles(starting):
+    """fp32, N = 72: 216 row tiles take the prologue backward that four waves
+    share, 8 copies (1728 tiles) the one of a wave a tile.  Each copy's dx is
+    the single call's up to the order of four partial sums of 32-bit values."""
+    mod = triattn_module(H.draw_params(H.tri_attn_shapes(128, 32, 4), seed=9, bias_random=True), starting, 4,
+                         torch.float32)
+    dx = []
+    for B in (1, 8):
+        x, dy, m = _inputs(B, 72, torch.float32, 72)
+        x.requires_grad_()
+        dx.append(torch.autograd.grad(mod(x, m), x, dy)[0])
+    one, many = dx
+    for k in range(8):
+        err = (many[k] - one[0]).norm() / one[0].norm()
+        assert err < 1e-6, err
