@@ -646,8 +646,9 @@ inline size_t wgrad_rowsum_floats(int M, int64_t pitch) {
 // Closing sums.  Every gradient of a backward pass ends as a sum over partials:
 // the splits of a product, the splits of its row sums, the segments of a row
 // reduction.  Each of these sums is a few microseconds of launch and load
-// latency, so all of a pass run in one launch (8 launches of 4.6 us at N = 250
-// before, 36.6 us; one of 8 now), each reading its partials directly:
+// latency, so all of a pass run in one launch (attention at N = 250: 8 launches of
+// 4.6 to 5.6 us before, one of 14 now, bound by the 40 MB of partials), each
+// reading its partials directly:
 //   dst[m][n] = sum_s src[s * step + row(m) * sm + col(n) * sn] * (gamma ? gamma[n] : 1)
 //             + (rs ? beta[n] * sum_s rs[s * rs_step + row(m) * rs_m] : 0)
 // row and col map an index of the gradient to the padded one of the product
