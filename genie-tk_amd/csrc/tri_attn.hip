@@ -29,6 +29,7 @@
 // valid key attends uniformly over all N keys: that is what the reference's
 // additive -1e9 bias produces in fp32 (every logit rounds to -1e9).
 #include <algorithm>
+#include <cfloat>
 #include <type_traits>
 
 #include "capi_util.hpp"
@@ -1512,7 +1513,10 @@ __global__ __launch_bounds__(512) void attn8_flash_kernel(const float* __restric
     qf[h] = load4f(ws.q + ((rowbase * H + h) * Np + q) * 8 + 4 * half);
     o0[h] = f32x4{0.f, 0.f, 0.f, 0.f};
     o1[h] = o0[h];
-    m_ref[h] = -INFINITY;
+    // Finite: keys whose mask bias overflows (-inf, such as inf * (lowest - 1))
+    // may fill the first tiles, and a reference of -inf would turn their scores
+    // into NaN.  No finite score lies below it.
+    m_ref[h] = -FLT_MAX;
     l_run[h] = 0.f;
   }
   for (int k0 = 0; k0 < N; k0 += KS) {
