@@ -12,6 +12,7 @@
 //     LayerNorm affine is folded into the packed forward weights, so the
 //     kernels hold x_hat, not the LayerNorm output).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "capi_util.hpp"
@@ -629,7 +630,7 @@ inline WgradPlan wgrad_plan(int M, int64_t pitch) {
   const int64_t maxs = pitch / 64 > 0 ? pitch / 64 : 1;
   if (ns > maxs) ns = maxs;
   if (ns < 1) ns = 1;
-  int64_t kc = round_up((pitch + ns - 1) / ns, 64);
+  const int64_t kc = std::max<int64_t>(round_up((pitch + ns - 1) / ns, 64), 64);  // (pitch 0: an empty batch)
   ns = (pitch + kc - 1) / kc;
   return WgradPlan{(int)(ns > 0 ? ns : 1), kc};
 }

@@ -1257,7 +1257,7 @@ constexpr int kDbQt = 2;  // query tiles per block
 // us more in the reduction; N = 384, 8 -> 10: 118 -> 101).  At most 16: 32 at N
 // = 128 took 11 + 12 us for the sums and the reduction against 26 + 5 with 8.
 inline int dbias_rh_chunks(int64_t B, int64_t N, int H) {
-  const int64_t blocks = B * H * (((N + 31) / 32 + kDbQt - 1) / kDbQt);
+  const int64_t blocks = std::max<int64_t>(B * H * (((N + 31) / 32 + kDbQt - 1) / kDbQt), 1);  // (0: an empty batch)
   const int64_t want = std::min<int64_t>(std::max<int64_t>(256 / blocks, 8), 16);
   return (int)std::min<int64_t>(want, std::max<int64_t>((N + 3) / 4, 8));
 }

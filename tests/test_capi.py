@@ -287,6 +287,23 @@ def test_empty_inputs_are_no_ops(lib):
                                      1e-5, GTK_F32, None, 0, None) == GTK_OK
 
 
+@pytest.mark.parametrize("dtype", [GTK_F32, GTK_BF16])
+def test_workspace_sizes_of_empty_inputs(lib, dtype):
+    """The size queries answer B = 0, N = 0 and rows = 0 (a caller asks for the
+    size before the call that then does nothing), and no more than for one pair
+    or row."""
+    one_mul = lib.gtk_tri_mul_backward_workspace_size(1, 1, 128, 128, dtype)
+    one_attn = lib.gtk_tri_attn_backward_workspace_size(1, 1, 128, 128, 4, dtype)
+    for B, N in ((0, 8), (2, 0), (0, 0)):
+        assert 0 < lib.gtk_tri_mul_backward_workspace_size(B, N, 128, 128, dtype) <= one_mul
+        assert 0 < lib.gtk_tri_attn_backward_workspace_size(B, N, 128, 128, 4, dtype) <= one_attn
+        for c_h in (32, 128):
+            assert lib.gtk_tri_attn_workspace_size(B, N, 128, c_h, 4, dtype) >= 0
+        assert lib.gtk_tri_mul_workspace_size(B, N, 128, 128, dtype) >= 0
+    assert (0 < lib.gtk_pair_transition_backward_workspace_size(0, 128, 4, dtype)
+            <= lib.gtk_pair_transition_backward_workspace_size(1, 128, 4, dtype))
+
+
 def test_timing_report_when_idle(lib):
     buf = ctypes.create_string_buffer(256)
     assert lib.gtk_timing_report(buf, 256) == GTK_OK
