@@ -210,7 +210,8 @@ const void* ptr_or_null(const at::Tensor& t) { return t.defined() ? t.data_ptr()
 
 // Parameter gradients as views of one fp32 buffer, each starting 16-byte
 // aligned (one allocation; the caller casts them with one conversion of the
-// buffer, which follows the views in out).
+// buffer, which follows the views in out).  Zero for an empty input, on which
+// the C functions do nothing.
 void flat_grads(std::vector<at::Tensor>& out, const at::Tensor& like,
                 const std::vector<std::vector<int64_t>>& shapes, float** const* gs) {
   auto numel = [](const std::vector<int64_t>& s) {
@@ -220,7 +221,8 @@ void flat_grads(std::vector<at::Tensor>& out, const at::Tensor& like,
   };
   int64_t total = 0;
   for (auto& s : shapes) total += (numel(s) + 3) / 4 * 4;
-  auto flat = at::empty({total}, like.options().dtype(at::kFloat));
+  const auto opts = like.options().dtype(at::kFloat);
+  auto flat = like.numel() == 0 ? at::zeros({total}, opts) : at::empty({total}, opts);
   int64_t o = 0;
   for (size_t i = 0; i < shapes.size(); ++i) {
     const int64_t n = numel(shapes[i]);

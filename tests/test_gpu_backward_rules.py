@@ -1,8 +1,9 @@
 """The backward kernels on both sides of the rules that choose between their
-forms: the same gradients either way."""
+forms: the same gradients either way.  An empty batch has zero gradients."""
 import pytest
 import torch
 
+from genie_tk.pair_transform import PairTransition
 from tests import helpers as H
 from tests.gpu_common import trimul_module, triattn_module
 
@@ -52,3 +53,22 @@ def test_attention_backward_split_tiles(starting):
     for k in range(8):
         err = (many[k] - one[0]).norm() / one[0].norm()
         assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,N", [(0, 8), (2, 0)])
+def test_empty_batch_has_zero_gradients(dt, B, N):
+    """As autograd of the PyTorch path gives them."""
+    mods = [trimul_module(H.draw_params(H.tri_mul_shapes(128, 128), seed=1), True, dt),
+            triattn_module(H.draw_params(H.tri_attn_shapes(128, 32, 4), seed=2), True, 4, dt),
+            triattn_module(H.draw_params(H.tri_attn_shapes(128, 128, 4), seed=3), False, 4, dt),
+            PairTransition(128, 4).to("cuda", dt)]
+    for mod in mods:
+        x = torch.zeros(B, N, N, 128, device="cuda", dtype=dt, requires_grad=True)
+        y = mod(x, torch.ones(B, N, N, device="cuda"))
+        assert y.shape == x.shape
+        junk = [torch.full((1 << 17,), float("nan"), device="cuda") for _ in range(8)]
+        del junk  # what a gradient buffer might hold
+        grads = torch.autograd.grad(y, [x, *mod.parameters()], torch.zeros_like(y))
+        for g, p in zip(grads, [x, *mod.parameters()]):
+            assert g.shape == p.shape and g.dtype == p.dtype and not g.any()
