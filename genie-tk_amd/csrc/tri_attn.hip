@@ -1464,9 +1464,9 @@ __global__ __launch_bounds__(256) void attn8_prologue_kernel(const float* __rest
 
 // Attention and output projection: a block is one row and up to blockDim/64
 // query tiles of it, one a wave; a wave attends its 32 queries in all four heads
-// and projects them, so heads never meet in LDS.  The keys of the row pass
-// through LDS in segments of KS positions (k and v of the four heads, 256 KS
-// bytes), read by every wave.
+// and projects them, so heads never meet in LDS.  The row's keys (nkeys: N
+// rounded up to 64, what the prologue wrote) pass through LDS in segments of KS
+// positions (k and v of the four heads, 256 KS bytes), read by every wave.
 //   S^T = bias + K Q^T: four 32x32x2 products a 32-key tile (lane = query, 16
 //   keys a half-wave).  Online softmax whose reference maximum moves only when a
 //   tile exceeds it by more than 8 (log2 units).  O^T += V^T P^T with the
@@ -1481,7 +1481,7 @@ template <int CIN, int KS>
 __global__ __launch_bounds__(512) void attn8_flash_kernel(const float* __restrict__ x, const float* __restrict__ mask,
                                                           float* __restrict__ out, TriAttnPacked<float> w, Attn8Ws ws,
                                                           int N, int Np, int starting, int residual, int r0, int nrows,
-                                                          float inf, int qgroups) {
+                                                          float inf, int nkeys, int qgroups) {
   constexpr int H = 4;
   constexpr float kRescale = 8.0f;
   __shared__ __attribute__((aligned(1024))) float ks[H][KS * 8];
@@ -1520,8 +1520,8 @@ __global__ __launch_bounds__(512) void attn8_flash_kernel(const float* __restric
     l_run[h] = 0.f;
   }
   for (int k0 = 0; k0 < N; k0 += KS) {
-    const int kn = min(KS, Np - k0);  // positions of the segment (a multiple of 64)
-    if (k0 > 0) __syncthreads();      // the segment before is read by every wave
+    const int kn = min(KS, nkeys - k0);  // positions of the segment (a multiple of 64)
+    if (k0 > 0) __syncthreads();         // the segment before is read by every wave
     // k: kn * 8 floats a head, contiguous; v: 8 rows of kn floats a head
     for (int c = threadIdx.x; c < H * 2 * kn; c += blockDim.x) {
       const int h = c / (2 * kn), i = c - h * 2 * kn;
@@ -1960,7 +1960,7 @@ static int fwd_attn8(const void* x, const float* mask, void* out, const void* pa
     StageTimer timer("triattn_flash", st);
     auto go = [&](auto kern) {
       kern<<<(unsigned)blocks, 64 * waves, 0, st>>>((const float*)x, mask, (float*)out, w, a, (int)N, Np, starting,
-                                                    residual, r0, nrows, inf, qgroups);
+                                                    residual, r0, nrows, inf, 32 * vtiles, qgroups);
     };
     if (Np <= 128) go(attn8_flash_kernel<CIN, 128>);
     else go(attn8_flash_kernel<CIN, 256>);
