@@ -1,9 +1,12 @@
-"""The kernels read no workspace value that the same call did not write: with
+"""No result depends on a workspace value that the same call did not write: with
 every uninitialised byte 0xff (NaN in bf16 and fp32) the results are those of
-any other call."""
+any other call.  The sizes cover each form of the kernels: resident and streamed
+forward, the (row, head) backward up to 512 and 1024 and the one beyond, narrow
+and full heads, ragged tiles of every operator."""
 import pytest
 import torch
 
+from genie_tk.pair_transform import PairTransition
 from tests import helpers as H
 from tests.gpu_common import trimul_module, triattn_module
 
@@ -12,11 +15,18 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dname", ["bf16", "fp32"])
 @pytest.mark.parametrize("op,N", [("tri_attn", 7), ("tri_attn", 33), ("tri_attn", 77), ("tri_attn", 264),
-                                  ("tri_mul", 33), ("tri_mul", 77)])
+                                  ("tri_attn", 520), ("tri_attn", 1030), ("tri_attn_wide", 77),
+                                  ("tri_attn_wide", 520), ("tri_mul", 33), ("tri_mul", 77), ("tri_mul", 301),
+                                  ("transition", 1), ("transition", 33)])
 def test_results_do_not_depend_on_workspace_contents(dname, op, N):
     dt = torch.bfloat16 if dname == "bf16" else torch.float32
-    if op == "tri_attn":
-        mod = triattn_module(H.draw_params(H.tri_attn_shapes(128, 32, 4), seed=3, bias_random=True), True, 4, dt)
+    if op in ("tri_attn", "tri_attn_wide"):
+        c_h = 32 if op == "tri_attn" else 128
+        mod = triattn_module(H.draw_params(H.tri_attn_shapes(128, c_h, 4), seed=3, bias_random=True), True, 4, dt)
+    elif op == "transition":
+        mod = PairTransition(128, 4)
+        mod.load_state_dict(H.to_state_dict(H.draw_params(H.pair_transition_shapes(128), seed=3, bias_random=True)))
+        mod = mod.to("cuda", dt)
     else:
         mod = trimul_module(H.draw_params(H.tri_mul_shapes(128, 128), seed=3, bias_random=True), True, dt)
     gen = torch.Generator(device="cuda").manual_seed(N)
