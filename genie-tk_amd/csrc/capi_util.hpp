@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <algorithm>
 #include <string>
 
 #include "../../include/genie_tk.h"
@@ -48,6 +49,14 @@ inline bool abs_at_most(float f, float lim) {
 // Compute units of the current device (cached per device; persistent kernels
 // launch one block per CU).
 int device_cus();
+
+// Waves that a tile's `units` independent pieces are dealt to, where one wave a
+// tile leaves the chip without waves: as many as keep the launch within
+// `per_cu` waves a CU, at most one a unit.  Each of them normalises the tile
+// again.
+inline int split_parts(int64_t tiles, int units, int per_cu) {
+  return (int)std::min<int64_t>(units, std::max<int64_t>(1, per_cu * (int64_t)device_cus() / std::max<int64_t>(tiles, 1)));
+}
 
 // Per-kernel timing (gtk_timing_enable / gtk_timing_report): when enabled, a
 // StageTimer records one HIP event before and one after the launch it

@@ -1892,7 +1892,7 @@ static int fwd_triattn(const void* x, const float* mask, void* out, const void* 
     auto prologue = [&](int r0, int nrows, int mode) {
       const int64_t ptiles = B * (int64_t)nrows * (Np / 32);
       StageTimer timer("triattn_prologue", st);
-      const int parts = (int)std::min<int64_t>(2 * H + 1, std::max<int64_t>(1, 8 * (int64_t)device_cus() / ptiles));
+      const int parts = split_parts(ptiles, 2 * H + 1, 8);
       auto go = [&](auto kern) {
         kern<<<dim3((unsigned)((ptiles + 3) / 4), parts), 256, 0, st>>>((const T*)x, w, a, (int)B, (int)N, Np,
                                                                         starting, eps, r0, nrows, mode);

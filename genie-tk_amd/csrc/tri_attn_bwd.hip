@@ -124,7 +124,7 @@ __host__ __device__ __forceinline__ int64_t bias_frag_elem(int h, int a, int k, 
 //
 // SPLIT: the 4 H + 1 projections of a tile (q, k, v and gate of each head, the
 // bias) are dealt over gridDim.y waves, each of which normalises the tile
-// again, where the tiles alone leave the chip without waves (attn_parts; N =
+// again, where the tiles alone leave the chip without waves (split_parts; N =
 // 128 in fp32: 103 -> 56 us).
 // ---------------------------------------------------------------------------
 template <typename T, int C, int H, bool SPLIT>
@@ -220,12 +220,6 @@ __global__ __launch_bounds__(256) void attn_bwd_proj_kernel(const T* __restrict_
     for (int h = 0; h < H; ++h) gate(h);
     bias();
   }
-}
-
-// Parts that a row tile's `units` independent pieces are dealt to: within
-// `per_cu` waves a CU, at most one part a unit.
-inline int attn_parts(int64_t tiles, int units, int per_cu) {
-  return (int)std::min<int64_t>(units, std::max<int64_t>(1, per_cu * (int64_t)device_cus() / std::max<int64_t>(tiles, 1)));
 }
 
 // ---------------------------------------------------------------------------
@@ -2008,7 +2002,7 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
       }
     }
     if (!std::is_same<T, bf16>::value || dmajor) {
-      const int parts = attn_parts(rowtiles, 4 * H + 1, 24);
+      const int parts = split_parts(rowtiles, 4 * H + 1, 24);
       auto go = [&](auto kern) {
         kern<<<dim3(g4(rowtiles), parts), 256, 0, st>>>((const T*)x, mask, a.w, a.b, (int)B, (int)N, np, starting,
                                                         eps, 1.0f / scale, dmajor);
@@ -2046,7 +2040,7 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
   }
   {
     StageTimer timer("triattn_bwd_epi", st);
-    const bool split = attn_parts(rowtiles, H, 8) == H;
+    const bool split = split_parts(rowtiles, H, 8) == H;
     auto go = [&](auto kern) {
       kern<<<dim3(g4(rowtiles), split ? H : 1), 256, 0, st>>>((const T*)dy, a.w, a.b, (int)B, (int)N, np, starting,
                                                              dmajor);

@@ -50,7 +50,7 @@ inline int64_t plane_stride(int64_t rows, int64_t Np) {
 // tile are dealt over gridDim.y waves, each of which normalises the tile again:
 // a tile's products are a serial chain of 64 matrix instructions a unit and
 // projection, 30 us for all units in fp32, so a small problem needs its waves
-// (SPLIT, units_split).
+// (SPLIT, split_parts).
 // ---------------------------------------------------------------------------
 template <typename T, int CZ, int CH, bool SPLIT>
 __global__ __launch_bounds__(256) void trimul_prologue_kernel(
@@ -828,7 +828,7 @@ __global__ __launch_bounds__(64 * (TI / 64) * (TJ / 64)) void trimul_contract_fp
 //
 // Generic form: one wave per 32-pair tile and NTB of its output channel tiles
 // (blockIdx.y), weights from L2.  NTB < CZ / 32 where the tiles alone would
-// leave the chip without waves (units_split; N = 64 fp32: 32 -> 18 us).
+// leave the chip without waves (split_parts; N = 64 fp32: 32 -> 18 us).
 // ---------------------------------------------------------------------------
 template <typename T, int CZ, int CH, int NTB>
 __global__ __launch_bounds__(256) void trimul_epilogue_kernel(
@@ -1342,16 +1342,6 @@ constexpr bool trimul_fast() {
 // Prologue over plane rows r0 .. r0 + nrows - 1 (default: all Np rows) for
 // sides side_lo .. side_hi - 1 (0: A, 1: Bm), into planes of stride ps
 // (default: the unpadded nrows * Np).
-// Parts that a row tile's `units` independent pieces are dealt to: as many as
-// keep the launch within `per_cu` waves a CU, at most one a unit.  Beyond that
-// the LayerNorm that each part repeats costs more than its waves give.  fp32,
-// times of the kernel unsplit / split: prologue (24 a CU) 63 / 17 us at N = 64,
-// 99 / 69 at 160, 101 / 103 at 256; epilogue (8 a CU, all or nothing) 32 / 18
-// at N = 64, 35 / 42 at 160, where it is not split any more.
-static int units_split(int64_t tiles, int units, int per_cu) {
-  return (int)std::min<int64_t>(units, std::max<int64_t>(1, per_cu * (int64_t)device_cus() / std::max<int64_t>(tiles, 1)));
-}
-
 template <typename T, int CZ, int CH>
 static int launch_trimul_prologue(const void* z, const float* mask, const TriMulPacked<T>& w, T* pa,
                                   T* pb, int64_t B, int64_t N, int Np, int outgoing, float eps_in,
@@ -1381,7 +1371,9 @@ static int launch_trimul_prologue(const void* z, const float* mask, const TriMul
     }
   } else {
     StageTimer timer("trimul_prologue", st);
-    const int parts = units_split(ptiles, (side_hi - side_lo) * (CH / 32), 24);
+    // fp32, c = 128, the kernel unsplit / split: 63 / 17 us at N = 64, 99 / 69 at
+    // 160, 101 / 103 at 256
+    const int parts = split_parts(ptiles, (side_hi - side_lo) * (CH / 32), 24);
     auto go = [&](auto kern) {
       kern<<<dim3((unsigned)((ptiles + 3) / 4), parts), 256, 0, st>>>((const T*)z, mask, pa, pb, w, (int)B, (int)N, Np,
                                                                       outgoing, eps_in, r0, nrows, side_lo, side_hi, ps);
@@ -1416,8 +1408,9 @@ static int launch_trimul_epilogue(const void* z, const T* px, void* out, const T
       kern<<<dim3((unsigned)((etiles + 3) / 4), parts), 256, 0, st>>>((const T*)z, px, (T*)out, w, (int)B, (int)N, Np,
                                                                       residual, eps_in, eps_out, r0, nrows, xrows, ps_x);
     };
+    // all or nothing: 32 / 18 us at N = 64, 35 / 42 at 160, which stays unsplit
     constexpr int NT = CZ / 32;
-    if (NT > 1 && units_split(etiles, NT, 8) == NT) go(trimul_epilogue_kernel<T, CZ, CH, 1>, NT);
+    if (NT > 1 && split_parts(etiles, NT, 8) == NT) go(trimul_epilogue_kernel<T, CZ, CH, 1>, NT);
     else go(trimul_epilogue_kernel<T, CZ, CH, NT>, 1);
   }
   GTK_LAUNCH_CHECK();
