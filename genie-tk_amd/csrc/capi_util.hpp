@@ -58,6 +58,14 @@ inline int split_parts(int64_t tiles, int units, int per_cu) {
   return (int)std::min<int64_t>(units, std::max<int64_t>(1, per_cu * (int64_t)device_cus() / std::max<int64_t>(tiles, 1)));
 }
 
+// Two or more whole rounds of one wave a SIMD (to 9/10): nothing idles with one
+// wave a tile, and splitting mostly costs the repeated LayerNorm.
+inline bool fills_rounds(int64_t tiles) {
+  const int64_t simds = 4 * (int64_t)device_cus();
+  const int64_t rounds = (tiles + simds - 1) / simds;
+  return rounds >= 2 && 10 * tiles >= 9 * rounds * simds;
+}
+
 // Per-kernel timing (gtk_timing_enable / gtk_timing_report): when enabled, a
 // StageTimer records one HIP event before and one after the launch it
 // scopes, on the launch stream.  Disabled, it costs one relaxed load.

@@ -1372,8 +1372,11 @@ static int launch_trimul_prologue(const void* z, const float* mask, const TriMul
   } else {
     StageTimer timer("trimul_prologue", st);
     // fp32, c = 128, the kernel unsplit / split: 63 / 17 us at N = 64, 99 / 69 at
-    // 160, 101 / 103 at 256
-    const int parts = split_parts(ptiles, (side_hi - side_lo) * (CH / 32), 24);
+    // 160.  At 2048 tiles (N = 256, three parts) the call takes 226 / 221 us at c =
+    // 128, but 78.4 / 81.1 at c = 64, whose four units three waves share unevenly,
+    // and 45.4 / 46.0 at c = 32; in bf16 38.6 / 39.0 at c = 64, 38.6 / 37.9 at N = 200.
+    const bool whole = sizeof(T) == 4 && CH <= 64 && fills_rounds(ptiles);
+    const int parts = whole ? 1 : split_parts(ptiles, (side_hi - side_lo) * (CH / 32), 24);
     auto go = [&](auto kern) {
       kern<<<dim3((unsigned)((ptiles + 3) / 4), parts), 256, 0, st>>>((const T*)z, mask, pa, pb, w, (int)B, (int)N, Np,
                                                                       outgoing, eps_in, r0, nrows, side_lo, side_hi, ps);

@@ -1,5 +1,5 @@
-"""The backward kernels on both sides of the rules that choose between their
-forms: the same gradients either way.  An empty batch has zero gradients."""
+"""The backward kernels (and the generic tri-mul prologue) on both sides of the
+rules that choose between their forms: the same results either way.  An empty batch has zero gradients."""
 import pytest
 import torch
 
@@ -40,19 +40,37 @@ def test_contraction_backward_on_64_tiles(monkeypatch, outgoing, B, N):
 @pytest.mark.parametrize("starting", [True, False])
 def test_attention_backward_split_tiles(starting):
     """fp32, N = 72: 216 row tiles take the prologue backward that four waves
-    share, 8 copies (1728 tiles) the one of a wave a tile.  Each copy's dx is
-    the single call's up to the order of four partial sums of 32-bit values."""
+    share, 8 copies (1728 tiles) the one of a wave a tile, 9 copies (1944, two
+    whole rounds of the chip) also the projections of a wave a tile.  Each copy's
+    dx is the single call's up to the order of four partial sums of 32-bit values."""
     mod = triattn_module(H.draw_params(H.tri_attn_shapes(128, 32, 4), seed=9, bias_random=True), starting, 4,
                          torch.float32)
     dx = []
-    for B in (1, 8):
+    for B in (1, 8, 9):
         x, dy, m = _inputs(B, 72, torch.float32, 72)
         x.requires_grad_()
         dx.append(torch.autograd.grad(mod(x, m), x, dy)[0])
-    one, many = dx
-    for k in range(8):
-        err = (many[k] - one[0]).norm() / one[0].norm()
-        assert err < 1e-6, err
+    one, *many = dx
+    for d in many:
+        for k in range(d.shape[0]):
+            err = (d[k] - one[0]).norm() / one[0].norm()
+            assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("c", [32, 64, 128])
+def test_trimul_prologue_parts(c):
+    """fp32, N = 30: 128 prologue tiles a copy, dealt to 2 c / 32 waves each; 12
+    copies (1536 tiles) to fewer, 15 (1920, two whole rounds of the chip) to one
+    at c <= 64.  The same products in every form: the same bits."""
+    mod = trimul_module(H.draw_params(H.tri_mul_shapes(c, c), seed=c, bias_random=True), True, torch.float32)
+    x, _, m = _inputs(1, 30, torch.float32, 30)
+    x = x[..., :c].contiguous()
+    with torch.no_grad():
+        one = mod(x, m)
+        for B in (12, 15):
+            many = mod(x.expand(B, -1, -1, -1).contiguous(), m.expand(B, -1, -1).contiguous())
+            for k in range(B):
+                assert torch.equal(many[k], one[0])
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
