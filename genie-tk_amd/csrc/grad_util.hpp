@@ -335,7 +335,12 @@ template <typename T> struct TailJobs {
   int64_t rows[kMax];
   int count = 0;
   int64_t most = 0;
+  bool overflow = false;
   void add(T* b, int64_t r) {
+    if (count == kMax) {
+      overflow = true;
+      return;
+    }
     base[count] = b;
     rows[count++] = r;
     most = r > most ? r : most;
@@ -351,6 +356,7 @@ __global__ void zero_tail_kernel(TailJobs<T> L, int64_t pitch, int64_t P) {
 
 template <typename T>
 inline int launch_zero_tails(const TailJobs<T>& L, int64_t pitch, int64_t P, hipStream_t st) {
+  GTK_REQUIRE(!L.overflow, GTK_EINVAL, "zeroed tails: too many operands");
   const int64_t n = L.most * (pitch - P);
   if (n <= 0) return GTK_OK;
   zero_tail_kernel<T><<<dim3((unsigned)((n + 255) / 256), L.count), 256, 0, st>>>(L, pitch, P);
@@ -826,6 +832,7 @@ struct RowJobs {  // rows of G, with or without X
   int nseg[kMax];
   int first[kMax + 1] = {0};  // first block of each job
   int count = 0;
+  bool overflow = false;
 };
 
 template <typename T, bool DOT>
@@ -914,6 +921,10 @@ inline int64_t rowred_floats(int rows) { return (int64_t)2 * rows * rowred_segs(
 template <typename T>
 inline void add_rowred(RowJobs& R, SumJobs& S, const T* G, const T* X, int rows, float* tmp, float* sums,
                        float* dots) {
+  if (R.count == RowJobs::kMax) {
+    R.overflow = true;
+    return;
+  }
   const int k = R.count++, nseg = rowred_segs(rows);
   R.G[k] = G;
   R.X[k] = X;
@@ -935,6 +946,7 @@ inline void add_rowred(RowJobs& R, SumJobs& S, const T* G, const T* X, int rows,
 
 template <typename T>
 inline int launch_rowred(const RowJobs& R, int64_t pitch, int64_t P, hipStream_t st) {
+  GTK_REQUIRE(!R.overflow, GTK_EINVAL, "row reductions: too many jobs");
   if (R.count == 0) return GTK_OK;
   rowred_kernel<T><<<(unsigned)R.first[R.count], 256, 0, st>>>(R, pitch, P);
   GTK_LAUNCH_CHECK();

@@ -1252,7 +1252,8 @@ constexpr int kDbQt = 2;  // query tiles per block
 // = 128 took 11 + 12 us for the sums and the reduction against 26 + 5 with 8.
 inline int dbias_rh_chunks(int64_t B, int64_t N, int H) {
   const int64_t blocks = std::max<int64_t>(B * H * (((N + 31) / 32 + kDbQt - 1) / kDbQt), 1);  // (0: an empty batch)
-  const int64_t want = std::min<int64_t>(std::max<int64_t>(256 / blocks, 8), 16);
+  // (kWgradBlocks: the 256 CUs that workspace plans count on, whatever device is current)
+  const int64_t want = std::min<int64_t>(std::max<int64_t>(kWgradBlocks / blocks, 8), 16);
   return (int)std::min<int64_t>(want, std::max<int64_t>((N + 3) / 4, 8));
 }
 
@@ -2002,15 +2003,16 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
       }
     }
     if (!std::is_same<T, bf16>::value || dmajor) {
-      // (forward + backward in fp32, unsplit / split: N = 256, 2048 tiles, 1508 / 1523
-      // us; N = 240 1451 / 1461; N = 208, 1456 tiles, 1151 / 1139)
-      const int parts = fills_rounds(rowtiles) ? 1 : split_parts(rowtiles, 4 * H + 1, 24);
-      auto go = [&](auto kern) {
+      auto go = [&](auto kern, int parts) {
         kern<<<dim3(g4(rowtiles), parts), 256, 0, st>>>((const T*)x, mask, a.w, a.b, (int)B, (int)N, np, starting,
                                                         eps, 1.0f / scale, dmajor);
       };
-      if (parts > 1) go(attn_bwd_proj_kernel<T, C, H, true>);
-      else go(attn_bwd_proj_kernel<T, C, H, false>);
+      // bf16 comes here beyond N = 1024 only, with tiles for every wave.  (fp32
+      // forward + backward, unsplit / split: N = 256, 2048 tiles, 1508 / 1523 us; N =
+      // 240 1451 / 1461; N = 208, 1456 tiles, 1151 / 1139)
+      const int parts = sizeof(T) != 4 || fills_rounds(rowtiles) ? 1 : split_parts(rowtiles, 4 * H + 1, 24);
+      if (parts > 1) go(attn_bwd_proj_kernel<T, C, H, sizeof(T) == 4>, parts);
+      else go(attn_bwd_proj_kernel<T, C, H, false>, 1);
     }
     GTK_LAUNCH_CHECK();
   }
@@ -2195,7 +2197,7 @@ static int bwd_triattn(const void* x, const float* mask, const void* dy,
 using namespace gtk;
 
 // Shapes of the backward kernels: c_in in {32, 64, 128}, four heads of 32
-// (modules with fewer or narrower heads pass their weights padded to this).
+// (pack_attn_bwd pads modules with fewer or narrower heads to this).
 static bool attn_bwd_shape_ok(int64_t c_in, int64_t c_h, int64_t H) {
   return (c_in == 32 || c_in == 64 || c_in == 128) && H == 4 && c_h == H * AD;
 }
