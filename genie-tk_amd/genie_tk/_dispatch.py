@@ -3,10 +3,8 @@ weight cache and the autograd rule.
 
 A call on a GPU tensor with ``use_fused_kernel=True`` runs the HIP kernels.
 When it must produce gradients (autograd enabled and the input or a
-parameter requires grad), the triangle modules run their kernel forward
-inside an autograd Function whose backward is the kernels' backward; the
-modules without backward kernels (PairTransition) run their PyTorch path
-then.
+parameter requires grad), the modules run their kernel forward inside an
+autograd Function whose backward is the kernels' backward.
 """
 from __future__ import annotations
 

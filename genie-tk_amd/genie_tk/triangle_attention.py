@@ -24,7 +24,6 @@ trains through autograd of its PyTorch path.
 """
 from __future__ import annotations
 
-import math
 from functools import partialmethod
 from typing import Optional
 
@@ -39,42 +38,6 @@ from genie_tk.utils import has_cuda_kernels, permute_final_dims
 _CUDA_AVAILABLE = has_cuda_kernels()
 
 
-# The backward kernels' head shape: four heads of HD_BWD channels.
-H_BWD, HD_BWD = 4, 32
-
-
-def _pad_heads(params, H: int, ch: int):
-    """The module's parameters for the backward kernels' four heads of 32:
-    head h's d = ch / H channels go to padded channels 32 h .. 32 h + d - 1,
-    every other row of W_q, W_k, W_v, W_g and b_g and column of W_o is zero,
-    and so are the triangle-bias rows of heads H .. 3.  W_q is scaled by
-    sqrt(32 / d), so that the kernels' score scale 1/sqrt(32) is the module's
-    1/sqrt(d).  The zero channels and heads add nothing to the output (their
-    v and their W_o columns are zero), so the padded module's gradients
-    restricted to the real parameters are the module's own.  Returns the
-    padded list and the channel index of the real ones.  (The kernels pad in
-    their packing, with the score scale of the real heads in place of the
-    scaled W_q; this is the same map in PyTorch.)"""
-    ln_w, ln_b, tri_w, q_w, k_w, v_w, g_w, g_b, o_w, o_b = params
-    d = ch // H
-    idx = (torch.arange(H, device=q_w.device)[:, None] * HD_BWD
-           + torch.arange(d, device=q_w.device)[None, :]).reshape(-1)
-    cp = H_BWD * HD_BWD
-    scale = math.sqrt(HD_BWD / d)
-
-    def rows(w, s=1.0):
-        out = w.new_zeros((cp,) + tuple(w.shape[1:]))
-        out[idx] = w * s if s != 1.0 else w
-        return out
-
-    o_p = o_w.new_zeros(o_w.shape[0], cp)
-    o_p[:, idx] = o_w
-    tri_p = tri_w.new_zeros(H_BWD, tri_w.shape[1])
-    tri_p[:H] = tri_w
-    return [ln_w, ln_b, tri_p, rows(q_w, scale), rows(k_w), rows(v_w), rows(g_w), rows(g_b), o_p,
-            o_b], idx, scale
-
-
 class _TriAttnFunction(torch.autograd.Function):
     """The update on the HIP kernels, forward and backward.
 
@@ -83,9 +46,9 @@ class _TriAttnFunction(torch.autograd.Function):
     same gradients on the kernels.  Activations are recomputed in the backward
     from x (only x, the mask and the parameters are saved).  Modules with
     fewer than four heads, or heads narrower than 32 channels, run the
-    backward on their weights padded to four heads of 32 as _pad_heads
-    describes; the kernels' packing and closing sums do that on the fly (in
-    PyTorch it took some 20 launches, 70 us a call)."""
+    backward padded to four heads of 32: the kernels' packing gives the
+    missing channels and heads zero weights, and the closing sums read the
+    real ones only (in PyTorch that took some 20 launches, 70 us a call)."""
 
     @staticmethod
     def forward(ctx, module, x, mask, chunk_size, *params):

@@ -385,15 +385,35 @@ def test_generic_class_direction_flag():
     assert TriangleAttention(16, 8, 2).starting
 
 
+def _pad_heads(params, h, ch, heads=4, width=32):
+    """The parameters of a module of h heads of d = ch / h channels as those of
+    four heads of 32: head i's channels go to 32 i .. 32 i + d - 1, every other
+    row of W_q, W_k, W_v, W_g and b_g, column of W_o and triangle-bias row is
+    zero.  W_q takes the factor sqrt(32 / d) that keeps the scores' 1/sqrt(d);
+    the kernels leave W_q alone and scale the scores by 1/sqrt(d) instead.
+    Returns also the padded indices of the real channels and that factor."""
+    ln_w, ln_b, tri_w, q_w, k_w, v_w, g_w, g_b, o_w, o_b = params
+    d = ch // h
+    idx = (torch.arange(h)[:, None] * width + torch.arange(d)[None, :]).reshape(-1)
+    scale = (width / d) ** 0.5
+
+    def rows(w):
+        out = w.new_zeros((heads * width,) + tuple(w.shape[1:]))
+        out[idx] = w
+        return out
+
+    tri_p = tri_w.new_zeros(heads, tri_w.shape[1])
+    tri_p[:h] = tri_w
+    return [ln_w, ln_b, tri_p, rows(q_w) * scale, rows(k_w), rows(v_w), rows(g_w), rows(g_b),
+            rows(o_w.t()).t(), o_b], idx, scale
+
+
 def test_head_padding_for_the_backward_kernels():
     """The attention backward kernels take four heads of 32 channels; a module
-    with fewer or narrower heads runs them on its weights padded with zero
-    channels and heads (triangle_attention._pad_heads), W_q scaled by
-    sqrt(32 / d).  The padded module computes the same function: checked
-    here in float64 on the PyTorch path, with the gradient of the real
-    parameters recovered as the backward does."""
-    from genie_tk import triangle_attention as ta
-
+    with fewer or narrower heads runs them padded with zero channels and heads.
+    The identity behind that, in float64 on the PyTorch path: the padded module
+    computes the same function, and its gradients at the real entries are the
+    module's own.  (test_gpu_grads checks the kernels themselves.)"""
     torch.manual_seed(0)
     for cin, ch, h in ((32, 16, 2), (64, 32, 4), (32, 8, 1)):
         mod = TriangleAttentionStartingNode(cin, ch, h, use_fused_kernel=False).double()
@@ -401,7 +421,7 @@ def test_head_padding_for_the_backward_kernels():
             with torch.no_grad():
                 p.copy_(torch.randn_like(p) * 0.3)
         params = mod._param_list()
-        padded, idx, scale = ta._pad_heads([p.detach() for p in params], h, ch)
+        padded, idx, scale = _pad_heads([p.detach() for p in params], h, ch)
         big = TriangleAttentionStartingNode(cin, 128, 4, use_fused_kernel=False).double()
         with torch.no_grad():
             for p, v in zip(big._param_list(), padded):
