@@ -399,7 +399,6 @@ KERNEL_KEYS = [
     ("trimul_epilogue_bf16_kernel", "trimul_epilogue"),
     ("triattn_prologue_bf16_kernel", "triattn_prologue"),
     ("triattn_flash_rh_kernel", "triattn_flash"),
-    ("triattn_flash_kernel", "triattn_flash"),
     ("triattn_out_kernel", "triattn_out"),
     ("ln_rows_kernel", "layernorm"),
     ("pair_transition_bf16_kernel", "pair_transition"),
