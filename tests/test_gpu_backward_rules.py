@@ -5,7 +5,7 @@ import torch
 
 from genie_tk.pair_transform import PairTransition
 from tests import helpers as H
-from tests.gpu_common import trimul_module, triattn_module
+from tests.gpu_common import ext, trimul_module, triattn_module
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +55,24 @@ def test_attention_backward_split_tiles(starting):
         for k in range(d.shape[0]):
             err = (d[k] - one[0]).norm() / one[0].norm()
             assert err < 1e-6, err
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_attention_backward_entries_agree(dt):
+    """_C.tri_attn_backward (gtk_tri_attn_backward: four heads of 32) and
+    _C.tri_attn_backward_heads (every head shape) are one pass: the same bits."""
+    mod = triattn_module(H.draw_params(H.tri_attn_shapes(64, 128, 4), seed=5, bias_random=True), True, 4, dt)
+    x, dy, m = _inputs(1, 45, dt, 45)
+    x, dy = x[..., :64].contiguous(), dy[..., :64].contiguous()
+    params = [p.detach() for p in mod._param_list()]
+    C = ext()
+    one = C.tri_attn_backward(x, m, dy, params, 64, 128, 4, True)
+    every = C.tri_attn_backward_heads(x, m, dy, params, 64, 128, 4, True)
+    for a, b in zip(one[:-1], every[:-1]):  # (the last is the buffer that holds them, with its gaps)
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+    narrow = triattn_module(H.draw_params(H.tri_attn_shapes(64, 32, 4), seed=5), True, 4, dt)
+    with pytest.raises(RuntimeError, match="unsupported"):
+        C.tri_attn_backward(x, m, dy, [p.detach() for p in narrow._param_list()], 64, 32, 4, True)
 
 
 @pytest.mark.parametrize("c", [32, 64, 128])
