@@ -1756,7 +1756,7 @@ static int raw_attn_entry(const void* q, const void* k, const void* v, const flo
   const char* name = starting ? "gtk_triangle_attention_starting" : "gtk_triangle_attention_ending";
   GTK_REQUIRE(dtype == GTK_F32 || dtype == GTK_BF16, GTK_EINVAL, "%s: bad dtype %d", name, dtype);
   GTK_REQUIRE(D == HD, GTK_EUNSUPPORTED, "%s: head dim %lld unsupported (32)", name, (long long)D);
-  GTK_REQUIRE(B >= 0 && H >= 1 && N >= 0 && N <= 8192, GTK_EINVAL, "%s: bad shape", name);
+  GTK_REQUIRE(B >= 0 && H >= 1 && N >= 0 && N <= MAXN, GTK_EINVAL, "%s: bad shape", name);
   if (B == 0 || N == 0) return GTK_OK;
   GTK_REQUIRE(q && k && v && bias && mask && out && ws, GTK_EINVAL, "%s: null pointer", name);
   const size_t need = gtk_triangle_attention_workspace_size(B, H, N, D, dtype);
@@ -2111,7 +2111,7 @@ extern "C" int gtk_tri_attn_forward_chunked(const void* x, const float* mask, vo
               "gtk_tri_attn_forward: c_in=%lld c_h=%lld H=%lld unsupported (c_in in {32,64,128}, "
               "H in {1,2,4}, c_h / H <= 32)",
               (long long)c_in, (long long)c_h, (long long)H);
-  GTK_REQUIRE(B >= 0 && N >= 0 && N <= 8192 && chunk_rows >= 0, GTK_EINVAL,
+  GTK_REQUIRE(B >= 0 && N >= 0 && N <= MAXN && chunk_rows >= 0, GTK_EINVAL,
               "gtk_tri_attn_forward: bad shape");
   GTK_REQUIRE(abs_at_most(inf, 1e37f), GTK_EINVAL,
               "gtk_tri_attn_forward: |inf| must be at most 1e37, got %g", (double)inf);

@@ -52,6 +52,7 @@ def lib():
     L.gtk_tri_attn_backward_workspace_size.argtypes = [i64, i64, i64, i64, i64, ci]
     L.gtk_tri_attn_backward.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, ci, fp,
                                         ci, vp, sz, vp]
+    L.gtk_tri_attn_backward_heads.argtypes = L.gtk_tri_attn_backward.argtypes
     L.gtk_tri_attn_workspace_size_chunked.argtypes = [i64, i64, i64, i64, i64, i64, ci]
     L.gtk_tri_mul_workspace_size_chunked.argtypes = [i64, i64, i64, i64, ci, i64]
     L.gtk_pair_transition_packed_size.argtypes = [i64, i64, ci]
@@ -285,6 +286,20 @@ def test_empty_inputs_are_no_ops(lib):
                                     1e-5, GTK_BF16, None, 0, None) == GTK_OK
     assert lib.gtk_tri_attn_backward(None, None, None, None, None, None, 3, 0, 128, 128, 4, 0,
                                      1e-5, GTK_F32, None, 0, None) == GTK_OK
+    assert lib.gtk_tri_attn_backward_heads(None, None, None, None, None, None, 0, 8, 128, 32, 4, 0,
+                                           1e-5, GTK_BF16, None, 0, None) == GTK_OK
+
+
+def test_backward_heads_accepts_the_forward_head_shapes(lib):
+    """gtk_tri_attn_backward_heads: H in {1, 2, 4}, d = c_h / H <= 32 pass the shape
+    check (the null pointers are what fails); everything else does not."""
+    def call(c_in, c_h, H):
+        return lib.gtk_tri_attn_backward_heads(None, None, None, None, None, None, 1, 8, c_in, c_h, H, 1,
+                                               1e-5, GTK_BF16, None, 0, None)
+    for c_in, c_h, H in ((128, 128, 4), (128, 32, 4), (64, 32, 2), (32, 5, 1), (128, 4, 4)):
+        assert call(c_in, c_h, H) == GTK_EINVAL and "null" in _err(lib)
+    for c_in, c_h, H in ((96, 32, 4), (128, 96, 3), (128, 132, 4), (128, 30, 4), (128, 0, 4), (128, 64, 1)):
+        assert call(c_in, c_h, H) == GTK_EUNSUPPORTED and "unsupported" in _err(lib)
 
 
 @pytest.mark.parametrize("dtype", [GTK_F32, GTK_BF16])
