@@ -451,10 +451,12 @@ struct TileWalk {
   int b, r, c;     // the current tile
   int db, dr, dc;  // the stride, decomposed the same way
   int rows, cols;
-  __device__ __forceinline__ void init(int64_t t, int64_t stride, int rows_, int cols_) {
+  // I: the type of the divisions (uint32_t where every tile index fits)
+  template <typename I>
+  __device__ __forceinline__ void init(I t, I stride, int rows_, int cols_) {
     rows = rows_;
     cols = cols_;
-    const int64_t plane = (int64_t)rows * cols;
+    const I plane = (I)rows * (I)cols;
     c = (int)(t % cols);
     r = (int)((t / cols) % rows);
     b = (int)(t / plane);
