@@ -770,7 +770,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   constexpr int ST = NTM / 2;         // STREAM: key tiles per stage (two stages)
   constexpr int CPW = 4 * ST / NW;    // STREAM: copies of 1 KiB per wave and stage
   constexpr float kRescale = 8.0f;    // lazy-rescale threshold (log2 units)
-  static_assert(NTM <= 64 && 64 % ST == 0, "excluded-key bits: one word per lane");
+  static_assert(NTM <= 64 && 64 % ST == 0 && (NTM & (NTM - 1)) == 0, "excluded-key bits: one word per lane");
   static_assert(!STREAM || ((4 * ST) % NW == 0 && CPW <= ST && ST % 2 == 0), "whole copies, at most one a tile");
   __shared__ __attribute__((aligned(1024))) char kv[2 * NTM * 2048];
   __shared__ __attribute__((aligned(1024))) char stg[NW][2048];
@@ -799,15 +799,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
 
   // K^T / V^T of (row, head) in copies of 1 KiB (kind, key tile, row half);
   // tiled layout: key tile t is [32 d][32 keys], 2 KiB contiguous.  Tile t
-  // lands in slot t % NTM.
+  // lands in slot t, or (STREAM) t % NTM.
   const bf16* kbase = ws.k + (rowbase * H + h) * (int64_t)HD * Np;
   const bf16* vbase = ws.vt + (rowbase * H + h) * (int64_t)HD * Np;
   const uint32_t kv_lds = lds_addr(kv);
+  auto slot = [](int t) { return STREAM ? t & (NTM - 1) : t; };
   auto copy_piece = [&](int kind, int t, int rh) {
-    const uint32_t ln = (uint32_t)(lane + opaque_zero());
+    // (STREAM issues its copies inside the key loop: offsets kept across it would spill)
+    const uint32_t ln = (uint32_t)(STREAM ? lane + opaque_zero() : lane);
     const uint32_t p = kind ? (ln & 3) ^ ((ln >> 4) & 3) : ln & 3;
     const bf16* src = (kind ? vbase : kbase) + t * 1024 + rh * 512;
-    const uint32_t dst = kv_lds + ((kind * NTM + t % NTM) * 2 + rh) * 1024;
+    const uint32_t dst = kv_lds + ((kind * NTM + slot(t)) * 2 + rh) * 1024;
     // read once by this row's block, or (STREAM) by its few query groups
     if constexpr (STREAM) g2lds16_sv(src, (ln >> 2) * 64 + p * 16, dst);
     else g2lds16_sv_nt(src, (ln >> 2) * 64 + p * 16, dst);
@@ -911,7 +913,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   };
   // K fragments of key tile t (transposing reads of K^T)
   auto k_read = [&](int t, Frag<bf16>* kf) {
-    const char* kt_base = kv + (t % NTM) * 2048 + kt_lane;
+    const char* kt_base = kv + slot(t) * 2048 + kt_lane;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       const s16x4 p0 = lds_read_tr16(kt_base + (m * 16) * 64);
@@ -961,7 +963,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const bool fast_ok = row_valid && !row_frac;
   // P = 2^sc (bf16), l += row sums of P, O^T += V^T P^T
   auto pv_tile = [&](int t, const f32x16& sc, f32x16& o, float& l_run) {
-    const char* vt_base = kv + (NTM + t % NTM) * 2048;
+    const char* vt_base = kv + (NTM + slot(t)) * 2048;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       Frag<bf16> pf, vf;
