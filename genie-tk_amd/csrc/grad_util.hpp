@@ -51,6 +51,7 @@ inline int launch_pack_acc(Tout* dst, const void* src, int wdtype, int out_dim, 
                     pk, 1});
     return GTK_OK;
   }
+  GTK_REQUIRE(pk.gp == kNoPad, GTK_EINVAL, "padded accumulator-order packing needs a batch");
   const int64_t total = packed_elems(out_dim, k_dim);
   const int blocks = (int)((total + 255) / 256);
   if (wdtype == GTK_F32)
